@@ -61,6 +61,32 @@ __device__ inline int xcd_remap(int b, int nb) {
   return xcd * q + (xcd < r ? xcd : r) + idx;
 }
 
+// A value's x neighbours within a 64-wide row held one cell per lane: lane n
+// takes lane n-1's (row_prev) or lane n+1's (row_next) by a wavefront DPP
+// shift of the two register halves, without LDS; lane 0, and lane `last` (the
+// row's last cell), take `edge`.
+__device__ __forceinline__ double dpp_shift(double v, double edge, bool up) {
+  const unsigned long long a = (unsigned long long)__double_as_longlong(v);
+  const unsigned long long e = (unsigned long long)__double_as_longlong(edge);
+  int lo, hi;
+  if (up) {  // wave_shr:1
+    lo = __builtin_amdgcn_update_dpp((int)e, (int)a, 0x138, 0xf, 0xf, false);
+    hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(a >> 32), 0x138, 0xf, 0xf, false);
+  } else {   // wave_shl:1
+    lo = __builtin_amdgcn_update_dpp((int)e, (int)a, 0x130, 0xf, 0xf, false);
+    hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(a >> 32), 0x130, 0xf, 0xf, false);
+  }
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) |
+                                          (unsigned long long)(unsigned)lo));
+}
+__device__ __forceinline__ double row_prev(double v, double edge) {
+  return dpp_shift(v, edge, true);
+}
+__device__ __forceinline__ double row_next(double v, double edge, int lane, int last) {
+  const double r = dpp_shift(v, edge, false);
+  return lane == last ? edge : r;
+}
+
 // Reproducible sums.  Each double term is truncated to a multiple of 2^-80
 // and split into four signed 32-bit limbs accumulated in int64: integer
 // addition is associative, so the total is independent of the order and of
@@ -460,6 +486,16 @@ struct BatchWork {
 // mixed solve's FP32 tables must exist)
 int ppe_batch_ws(c3d_ctx* c, int nb, const void* prsrc, void* phi, int sweeps,
                  const BatchWork& ws);
+// z planes per workgroup of the residual kernels, which march z over `tiles`
+// x-y tiles of nb fields: long runs amortise the lead-in plane, short ones
+// keep every CU supplied on small grids (a target of 8 workgroups per CU)
+inline int resid_kchunk(const Geom& g, int tiles, int nb) {
+  const long long per_plane = (long long)tiles * nb;
+  long long nch = (2048 + per_plane - 1) / per_plane;
+  int kc = (int)((g.nz + nch - 1) / nch);
+  if (kc < 4) kc = 4;
+  return kc > g.nz ? g.nz : kc;
+}
 // (1 - b Dxx)(1 - b Dzz)(1 - b Dyy) du = rhs for nb fields (k_adi.hip)
 int run_helmholtz_batch(c3d_ctx* c, int comp, int ns, int nb, const void* rhs, void* du,
                         int sweeps);

@@ -755,13 +755,27 @@ int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], cons
 // r = rhs - (1 - b Dxx)(1 - b Dzz) M du, in FP64, stored as TR.  M is the y
 // matrix the sweeps invert: rows 1..ny, diagonal bm(j), lower am(j) (j > 1),
 // upper cm(j) (j < ny).  WALL: row 1 is the wall condition du = 0, its
-// residual is 0.  A thread owns an (i, j) column and marches a chunk of
-// kchunk z planes: each plane's x-y part zs(k) = sum_x wx (M du)(x, k) is
-// formed once and rolls through registers, so every du value is loaded for
-// three planes' outputs once (9 loads per cell instead of 27), and the sum
-// over z keeps the order wzo zs(k-1) + wzc zs(k) + wzo zs(k+1).
-// blockIdx.z = q nch + chunk for field q (bf reals apart).
-template <typename TR, bool WALL>
+// residual is 0.
+//
+// A wavefront owns 64 x cells of HR rows and marches a chunk of kchunk z
+// planes.  Per plane it loads its HR rows and the row on either side once,
+// plus the two x cells beside them (every lane but the last reads the left
+// one, the last the right one), so M du needs no other load: the y neighbours
+// are the lane's own registers, and the x neighbours of M du come from the
+// lanes beside it by DPP.  The x-y part zs(k) = sum_x wx (M du)(x, k) is formed
+// once and rolls through registers, and the sum over z keeps the order
+// wzo zs(k-1) + wzc zs(k) + wzo zs(k+1).  The next plane's words are requested
+// before the current plane is computed.  Bound: HBM, 20 B per cell (du, rhs
+// read, r written).  The form it replaced (a thread per cell column, nine du
+// loads per plane, workgroups of a plane spread over the XCDs) was bound by
+// its loads: 1.461 ms for two 512x256x512 fields, this one 0.560 ms (4.8 TB/s;
+// a plain copy reaches 4.8-6.0 TB/s).  HR = 8 rows keep the reloaded
+// neighbour rows at 2 in 8 within the register budget of two planes in flight.
+// blockIdx.x = the tile (x fastest, then y, z chunk, field; bf reals apart),
+// XCD-remapped so that tiles sharing rows share an L2.
+constexpr int HR = 8;
+
+template <typename TR, bool WALL, bool NTS>
 __global__ __launch_bounds__(256) void k_helm_resid(Geom g, const double* __restrict__ am,
                                                     const double* __restrict__ bm,
                                                     const double* __restrict__ cm, double wxc,
@@ -770,47 +784,108 @@ __global__ __launch_bounds__(256) void k_helm_resid(Geom g, const double* __rest
                                                     const double* __restrict__ du,
                                                     TR* __restrict__ r, long long bf,
                                                     int kchunk) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  const int jc = blockIdx.y * 4 + threadIdx.y + 1;
+  const int gxb = (g.nx + 63) / 64, gyb = (g.ny + 4 * HR - 1) / (4 * HR);
   const int nch = (g.nz + kchunk - 1) / kchunk;
-  const int q = blockIdx.z / nch;
-  const int k0 = (blockIdx.z - q * nch) * kchunk;
-  if (i >= g.nx || jc > g.ny) return;
+  int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int i0 = (lb % gxb) * 64;
+  lb /= gxb;
+  const int j0 = ((lb % gyb) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.y)) * HR + 1;
+  lb /= gyb;
+  const int k0 = (lb % nch) * kchunk, q = lb / nch;
+  if (j0 > g.ny) return;
+  const int k1 = min(g.nz, k0 + kchunk);
   rhs += bf * q;
   du += bf * q;
   r += bf * q;
-  const int k1 = min(g.nz, k0 + kchunk);
-  if (WALL && jc == 1) {
-    for (int k = k0; k < k1; ++k) r[fidx(g, i, jc, k)] = TR(0);
-    return;
-  }
-  const int im = i == 0 ? g.nx - 1 : i - 1, ip = i == g.nx - 1 ? 0 : i + 1;
-  const double a = jc > 1 ? am[jc] : 0.0, b = bm[jc], cc = jc < g.ny ? cm[jc] : 0.0;
-  auto plane = [&](int k) {
-    const int ii[3] = {im, i, ip};
-    double zs = 0.0;
-#pragma unroll
-    for (int di = 0; di < 3; ++di) {
-      const long long p = fidx(g, ii[di], jc, k);
-      double my = b * du[p];
-      if (jc > 1) my += a * du[p - g.nx];
-      if (jc < g.ny) my += cc * du[p + g.nx];
-      zs += (di == 1 ? wxc : wxo) * my;
-    }
-    return zs;
+  const int lane = threadIdx.x, last = min(63, g.nx - 1 - i0);
+  const int i = min(i0 + lane, g.nx - 1);
+  const bool live = lane <= last;
+  const int ie = lane == last ? (i0 + last == g.nx - 1 ? 0 : i0 + last + 1)
+                              : (i0 == 0 ? g.nx - 1 : i0 - 1);
+  const int nx = g.nx, ny = g.ny;
+  // rows j0-1 .. j0+HR of a plane; rows past the top ghost read the ghost
+  struct Plane {
+    double c[HR + 2], e[HR + 2], f[HR];
   };
-  double zm = plane(k0 == 0 ? g.nz - 1 : k0 - 1);
-  double zc = plane(k0);
-  for (int k = k0; k < k1; ++k) {
-    const double zp = plane(k == g.nz - 1 ? 0 : k + 1);
-    double acc = 0.0;
-    acc += wzo * zm;
-    acc += wzc * zc;
-    acc += wzo * zp;
-    const long long c0 = fidx(g, i, jc, k);
-    r[c0] = (TR)(rhs[c0] - acc);
-    zm = zc;
-    zc = zp;
+  auto fetch = [&](int k, Plane& a, bool want_rhs) {
+    const double* p = du + g.plane * k;
+#pragma unroll
+    for (int t = 0; t < HR + 2; ++t) {
+      const long long row = (long long)nx * min(j0 - 1 + t, ny + 1);
+      a.c[t] = p[row + i];
+      a.e[t] = p[row + ie];
+    }
+    if (want_rhs) {
+      const double* pf = rhs + g.plane * k;
+#pragma unroll
+      for (int t = 0; t < HR; ++t)
+        a.f[t] = C3D_LD_ONCE(&pf[(long long)nx * min(j0 + t, ny) + i]);  // read once
+    }
+  };
+  // zs of the plane's HR rows
+  auto zsum = [&](const Plane& a, double* zs) {
+#pragma unroll
+    for (int t = 0; t < HR; ++t) {
+      const int j = min(j0 + t, ny);
+      const double bj = bm[j];
+      double mc = bj * a.c[t + 1], me = bj * a.e[t + 1];
+      if (j > 1) {
+        const double aj = am[j];
+        mc += aj * a.c[t];
+        me += aj * a.e[t];
+      }
+      if (j < ny) {
+        const double cj = cm[j];
+        mc += cj * a.c[t + 2];
+        me += cj * a.e[t + 2];
+      }
+      zs[t] = wxo * row_prev(mc, me) + wxc * mc + wxo * row_next(mc, me, lane, last);
+    }
+  };
+  double zm[HR], zc[HR];
+  {
+    Plane a;
+    fetch(k0 == 0 ? g.nz - 1 : k0 - 1, a, false);
+    zsum(a, zm);
+  }
+  // cur holds plane k+1's du and, in f, plane k's right-hand side
+  auto step = [&](int k, const Plane& cur, const double* f) {
+    double zp[HR];
+    zsum(cur, zp);
+#pragma unroll
+    for (int t = 0; t < HR; ++t) {
+      const int j = j0 + t;
+      double acc = 0.0;
+      acc += wzo * zm[t];
+      acc += wzc * zc[t];
+      acc += wzo * zp[t];
+      if (live && j <= ny) {
+        const TR v = WALL && j == 1 ? TR(0) : (TR)(f[t] - acc);
+        r[(long long)nx * j + g.plane * k + i] = v;
+      }
+      zm[t] = zc[t];
+      zc[t] = zp[t];
+    }
+  };
+  Plane a, b;
+  fetch(k0, a, true);
+  zsum(a, zc);
+  // a.f: the right-hand side of plane k; b: plane k+1 with its own right-hand side
+  // past the chunk's last plane (k1) the prefetch repeats it
+  auto wrapk = [&](int k) { return min(k, k1) == g.nz ? 0 : min(k, k1); };
+  fetch(wrapk(k0 + 1), b, true);
+  for (int k = k0; k < k1; k += 2) {
+    double f[HR];
+#pragma unroll
+    for (int t = 0; t < HR; ++t) f[t] = a.f[t];
+    fetch(wrapk(k + 2), a, true);
+    step(k, b, f);
+    if (k + 1 < k1) {
+#pragma unroll
+      for (int t = 0; t < HR; ++t) f[t] = b.f[t];
+      fetch(wrapk(k + 3), b, true);
+      step(k + 1, a, f);
+    }
   }
 }
 
@@ -918,17 +993,21 @@ int run_helmholtz_batch(c3d_ctx* c, int comp, int ns, int nb, const void* rhs, v
   double* const* yt = comp == 1 ? tb.d_yp : tb.d_yc;
   for (int s = 0; s < sweeps; ++s) {
     prof_begin(c, ST_RESID, &ev);
-    constexpr int KCH = 8;
-    const int nch = (g.nz + KCH - 1) / KCH;
-    const dim3 grid((g.nx + 63) / 64, (g.ny + 3) / 4, nch * nb), blk(64, 4);
-    if (comp == 1)
-      hipLaunchKernelGGL((k_helm_resid<float, true>), grid, blk, 0, c->stream, g, yt[0], yt[3],
-                         yt[4], wxc, wxo, wzc, wzo, (const double*)rhs, (const double*)du,
-                         (float*)c->bres, bf, KCH);
-    else
-      hipLaunchKernelGGL((k_helm_resid<float, false>), grid, blk, 0, c->stream, g, yt[0], yt[3],
-                         yt[4], wxc, wxo, wzc, wzo, (const double*)rhs, (const double*)du,
-                         (float*)c->bres, bf, KCH);
+    const int tiles = ((g.nx + 63) / 64) * ((g.ny + 4 * HR - 1) / (4 * HR));
+    const int kch = resid_kchunk(g, tiles, nb);
+    const dim3 grid(tiles * ((g.nz + kch - 1) / kch) * nb), blk(64, 4);
+    auto launch = [&](auto wallc, auto ntc) {
+      hipLaunchKernelGGL((k_helm_resid<float, decltype(wallc)::value, decltype(ntc)::value>), grid,
+                         blk, 0, c->stream, g, yt[0], yt[3], yt[4], wxc, wxo, wzc, wzo,
+                         (const double*)rhs, (const double*)du, (float*)c->bres, bf, kch);
+    };
+    if (comp == 1) {
+      if (g.nt) launch(std::true_type{}, std::true_type{});
+      else launch(std::true_type{}, std::false_type{});
+    } else {
+      if (g.nt) launch(std::false_type{}, std::true_type{});
+      else launch(std::false_type{}, std::false_type{});
+    }
     C3D_HIP(hipGetLastError());
     prof_end(c, ST_RESID, ev, N * (8 + 8 + 4));
     prof_begin(c, ST_ADI_XZ, &ev);

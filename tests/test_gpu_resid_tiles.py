@@ -1,0 +1,64 @@
+"""The FP64 residual passes of the refined solves at the edges of their tiles:
+64 x cells per wavefront (a last tile of 2 cells, one exact tile, less than a
+tile), blocks of 4 and 8 rows in workgroups of 16 and 32, z chunks with
+remainders.  A cell whose residual is wrong keeps the FP32 solve's error, so
+the refined solution must agree with the FP64 solve of the same source (which
+the oracle tests cover) everywhere: each sweep multiplies the error by the FP32
+solve's relative error, at most 1e-5 here for the pressure and 1e-6 for the
+velocity operator."""
+import math
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GRIDS = [(450, 33, 12), (128, 31, 50), (64, 32, 18), (72, 17, 25), (64, 16, 64)]
+
+
+def _channel(nx, ny, nz):
+    from channel3d_amd import Channel
+    return Channel(dict(nxc=nx, nyc=ny, nzc=nz, xlx=2 * math.pi, yly=2.0, zlz=math.pi,
+                        xnu=1.0e-4, dt=0.001, gamma=1.2, ubulk=1.0))
+
+
+def _fields(g, nb, compatible):
+    rng = np.random.default_rng(3)
+    out = []
+    for _ in range(nb):
+        f = rng.standard_normal((g.nxc, g.nyc, g.nzc))
+        if compatible:
+            d = np.diff(np.asarray(g.yp[1:g.nyc + 2]))
+            f -= (f.mean(axis=(0, 2)) * d).sum() / d.sum()
+        out.append(np.asfortranarray(f))
+    return out
+
+
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
+def test_pressure_refinement(grid):
+    from channel3d_amd import lib as L
+    with _channel(*grid) as g:
+        src, a, b = (g.alloc_batch(lay, 2) for lay in (L.INTERIOR, L.HALO, L.HALO))
+        for q, f in enumerate(_fields(g, 2, True)):
+            g.upload(src[q], f, L.INTERIOR)
+        g.ppe_batch(src, a, -1)
+        g.ppe_batch(src, b, 2)
+        n = slice(1, g.nyc + 1)
+        for q in range(2):
+            x, y = (g.download(h[q], L.HALO)[1:-2, n, 1:-2] for h in (a, b))
+            assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max()
+
+
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("comp", [0, 1])
+def test_velocity_refinement(grid, comp):
+    from channel3d_amd import lib as L
+    with _channel(*grid) as g:
+        rhs, a, b = (g.alloc_batch(L.INTERIOR, 2) for _ in range(3))
+        for q, f in enumerate(_fields(g, 2, False)):
+            g.upload(rhs[q], f, L.INTERIOR)
+        g.helmholtz_batch(comp, 1, rhs, a, -1)
+        g.helmholtz_batch(comp, 1, rhs, b, 1)
+        for q in range(2):
+            x, y = g.download(a[q], L.INTERIOR), g.download(b[q], L.INTERIOR)
+            assert np.abs(x - y).max() <= 1e-11 * np.abs(x).max()
