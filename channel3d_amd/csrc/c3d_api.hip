@@ -497,6 +497,21 @@ int ensure_mixed_tables(c3d_ctx* c) {
   if ((rc = dalloc(c, &w, nw * sizeof(double)))) return rc;
   C3D_HIP(hipMemset(w, 0, nw * sizeof(double)));
   c->d_mean64 = (double*)w;
+  // pivots and factors of the (0,0) line, by the elimination's operations
+  std::vector<double> fac(2 * (size_t)g.ny, 0.0);
+  const auto &am = c->met[C3D_M_AM2PR], &ac = c->met[C3D_M_AC2PR], &ap = c->met[C3D_M_AP2PR];
+  fac[0] = 1.0;
+  double cprev = 0.0;
+  for (int j = 1; j < g.ny; ++j) {
+    const double arr = cprev / fac[j - 1];
+    fac[j] = ((ac[j + 1] + c->met[C3D_M_WAVEX][0]) + c->met[C3D_M_WAVEZ][0]) - am[j + 1] * arr;
+    fac[g.ny + j] = arr;
+    cprev = ap[j + 1];
+  }
+  void* mf = nullptr;
+  if ((rc = dalloc(c, &mf, fac.size() * sizeof(double)))) return rc;
+  c->d_meanfac = (double*)mf;
+  C3D_HIP(hipMemcpy(mf, fac.data(), fac.size() * sizeof(double), hipMemcpyHostToDevice));
   c->d_tw32 = tw;
   return C3D_OK;
 }
@@ -580,7 +595,7 @@ extern "C" int c3d_destroy(c3d_ctx* c) {
     if (c->state[i]) hipFree(c->state[i]);
   for (void* p : c->user_fields) hipFree(p);
   void* bufs[] = {c->tmpA, c->spec, c->sarr, c->d_partials, c->d_sc, c->d_tw, c->d_met, c->d_tabs,
-                  c->d_dyp, c->d_stat, c->d_tw32, c->d_met32, c->resid32, c->d_mean64,
+                  c->d_dyp, c->d_stat, c->d_tw32, c->d_met32, c->resid32, c->d_mean64, c->d_meanfac,
                   c->d_lesmet, c->d_spec1d, c->spec2, c->d_spec2d, c->cln_d, c->cln_f,
                   c->cln_fb, c->bspec, c->bsarr, c->bmean, c->bres, c->btmp,
                   c->les_arr[0], c->les_arr[1]};

@@ -352,6 +352,10 @@ struct c3d_ctx {
   long prof_calls[c3d::ST_COUNT] = {};
   double prof_ms[c3d::ST_COUNT] = {};
   double prof_bytes[c3d::ST_COUNT] = {};
+
+  // mixed-precision pressure solve: the (0,0) line's pivots vecm[ny] and
+  // factors arr[ny]
+  double* d_meanfac = nullptr;
 };
 
 namespace c3d {

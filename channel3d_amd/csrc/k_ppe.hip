@@ -22,14 +22,30 @@ struct CT2<double> { using t = double2; };
 template <>
 struct CT2<float> { using t = float2; };
 
+// Lines (kx, kz) are numbered kx + (nk+1) kz and dealt to consecutive
+// threads, so only the last workgroup has idle threads.  nk+1 is one more
+// than a power of two or a multiple of 64 on most grids: with 64 threads per
+// kz row, a row's last wavefront held one live thread (512x256x512: 320
+// threads for 257 lines).  The two-lane sweep of 192x128x160 (97 lines a row)
+// takes 0.051 ms instead of 0.064; the memory-bound one-lane sweeps of large
+// grids are unchanged (512x256x512 x 4: 1.64 ms either way).
+struct Line {
+  int kx, kz;
+};
+__device__ __forceinline__ Line line_of(const Geom& g, long long l) {
+  Line r;
+  r.kz = (int)(l / (g.nk + 1));
+  r.kx = (int)(l - (long long)(g.nk + 1) * r.kz);
+  return r;
+}
+
 template <typename T>
 __device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& m,
                                                typename CT2<T>::t* __restrict__ spec,
-                                               T* __restrict__ sarr) {
+                                               T* __restrict__ sarr, Line ln) {
   using T2 = typename CT2<T>::t;
-  const int kx = blockIdx.x * 64 + threadIdx.x;
-  const int kz = blockIdx.y * 4 + threadIdx.y;
-  if (kx > g.nk || kz >= g.nz) return;
+  const int kx = ln.kx, kz = ln.kz;
+  if (kz >= g.nz) return;
   const int ny = g.ny;
   const long long P = g.P;
   const long long base = kx + P * (long long)ny * kz;
@@ -140,11 +156,10 @@ __device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& 
 template <typename T, int C, bool NTS = false>
 __device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, const Metrics<T>& m,
                                                   typename CT2<T>::t* __restrict__ spec,
-                                                  T* __restrict__ ckp) {
+                                                  T* __restrict__ ckp, Line ln) {
   using T2 = typename CT2<T>::t;
-  const int kx = blockIdx.x * 64 + threadIdx.x;
-  const int kz = blockIdx.y * 4 + threadIdx.y;
-  if (kx > g.nk || kz >= g.nz) return;
+  const int kx = ln.kx, kz = ln.kz;
+  if (kz >= g.nz) return;
   const int ny = g.ny;
   const int nseg = (ny + C - 1) / C;
   const long long P = g.P;
@@ -251,9 +266,9 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
                                                    typename CT2<T>::t* __restrict__ spec,
                                                    T* __restrict__ ckp) {
   const int part = threadIdx.x & 1;  // 0: real, 1: imaginary part
-  const int kx = blockIdx.x * 32 + (threadIdx.x >> 1);
-  const int kz = blockIdx.y * blockDim.y + threadIdx.y;
-  if (kx > g.nk || kz >= g.nz) return;
+  const Line ln = line_of(g, ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 1);
+  const int kx = ln.kx, kz = ln.kz;
+  if (kz >= g.nz) return;
   const int ny = g.ny;
   const int nseg = (ny + C - 1) / C, top = nseg - 1;
   const long long P = g.P;
@@ -380,20 +395,21 @@ __global__ __launch_bounds__(256) void k_tridiag_ck2(Geom g, Metrics<T> m,
                                                      typename CT2<T>::t* __restrict__ spec,
                                                      T* __restrict__ ckp, long long bsp,
                                                      long long bck) {
-  k_tridiag_ck2_body<T, C, NTS>(g, m, spec + bsp * blockIdx.z, ckp + bck * blockIdx.z);
+  k_tridiag_ck2_body<T, C, NTS>(g, m, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y);
 }
 
 // At least 4 waves per SIMD: the FP64 body fits 128 VGPRs without spilling
 // (136 unconstrained, 3 waves), and at 768x384x576 the 1008 workgroups then
 // run in one round instead of 1.3 -- 0.99 ms per solve instead of 1.21 ms.
-// Batches: blockIdx.z selects the field; its spectrum starts bsp complex
+// Batches: blockIdx.y selects the field; its spectrum starts bsp complex
 // elements, its checkpoints bck reals after the first field's.
 template <typename T, int C, bool NTS = false>
 __global__ __launch_bounds__(256, 4) void k_tridiag_ck(Geom g, Metrics<T> m,
                                                     typename CT2<T>::t* __restrict__ spec,
                                                     T* __restrict__ ckp, long long bsp,
                                                     long long bck) {
-  k_tridiag_ck_body<T, C, NTS>(g, m, spec + bsp * blockIdx.z, ckp + bck * blockIdx.z);
+  k_tridiag_ck_body<T, C, NTS>(g, m, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y,
+                               line_of(g, (long long)blockIdx.x * 256 + threadIdx.x));
 }
 
 template <typename T>
@@ -401,13 +417,15 @@ __global__ __launch_bounds__(256) void k_tridiag_b(Geom g, Metrics<T> m,
                                                    typename CT2<T>::t* __restrict__ spec,
                                                    T* __restrict__ sarr, long long bsp,
                                                    long long bck) {
-  k_tridiag_body<T>(g, m, spec + bsp * blockIdx.z, sarr + bck * blockIdx.z);
+  k_tridiag_body<T>(g, m, spec + bsp * blockIdx.y, sarr + bck * blockIdx.y,
+                    line_of(g, (long long)blockIdx.x * 256 + threadIdx.x));
 }
 
 template <typename T>
 static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
   const Geom& g = c->g;
-  dim3 grid((g.nk + 1 + 63) / 64, (g.nz + 3) / 4, b.n), blk(64, 4);
+  const long long nl = (long long)(g.nk + 1) * g.nz;  // lines of one field
+  const dim3 grid((unsigned)((nl + 255) / 256), b.n), blk(256);
   const Metrics<T>& m = *(const Metrics<T>*)(c->prec == C3D_FP64 ? (const void*)&c->md
                                                                   : (const void*)&c->mf);
   constexpr int CSEG = 16;
@@ -415,13 +433,12 @@ static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
   const long long need = 3LL * ((g.ny + CSEG - 1) / CSEG) * g.P * g.nz;
   // two lanes per wavenumber pair where a lane per pair leaves the SIMDs
   // short of wavefronts (fewer than two per SIMD of the 256-CU device)
-  const long long lines = (long long)(g.nk + 1) * g.nz * b.n;
-  const bool two = c->tri_lanes ? c->tri_lanes == 2 : lines * 2 <= 2048LL * 64;
+  const bool two = c->tri_lanes ? c->tri_lanes == 2 : nl * b.n * 2 <= 2048LL * 64;
   if (c->ymode != YS_STORE && need <= (long long)g.P * g.ny * g.nz && two) {
-    // one wavefront (32 wavenumber pairs of one kz) per workgroup: the
-    // grids that take this form have few lines, and single-wave workgroups
-    // spread them over more CUs
-    const dim3 grid2((g.nk + 1 + 31) / 32, g.nz, b.n), blk2(64, 1);
+    // one wavefront (32 wavenumber pairs) per workgroup: the grids that take
+    // this form have few lines, and single-wave workgroups spread them over
+    // more CUs
+    const dim3 grid2((unsigned)((nl + 31) / 32), b.n), blk2(64);
     if (g.nt)
       hipLaunchKernelGGL((k_tridiag_ck2<T, CSEG, true>), grid2, blk2, 0, c->stream, g, m,
                          (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
@@ -461,61 +478,105 @@ int launch_tridiag(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
 
 // The (0,0) mode in FP64: the Neumann y operator with the gauge row is the
 // ill-conditioned system of the solve (its FP32 error would bound what the
-// refinement can reach).  One thread; w holds 3 ny doubles, then the gauge
-// value at w[3 ny]: the first row is phi(0,0,1) = w[3 ny] (0 in the first
-// solve, as the reference pins it; in a correction solve, minus the current
-// solution's value, so the refined solution keeps the reference's gauge --
-// without it the FP32 rounding of the first solve's plane mean at j = 1
-// would survive every sweep as a constant offset).
+// refinement can reach).  w holds 3 ny doubles, then the gauge value at
+// w[3 ny]: the first row is phi(0,0,1) = w[3 ny] (0 in the first solve, as the
+// reference pins it; in a correction solve, minus the current solution's
+// value, so the refined solution keeps the reference's gauge -- without it
+// the FP32 rounding of the first solve's plane mean at j = 1 would survive
+// every sweep as a constant offset).
+//
+// One workgroup: its threads move the line through LDS, MCH rows at a time,
+// and lanes 0 and 1 run the recurrence of the real and the imaginary part from
+// there; the pivots and factors of the line (fac: vecm[ny], arr[ny]) do not
+// depend on the data and come from the host, formed with the same operations.
+// As one thread's loop over global memory (two dependent loads and three
+// divisions per row) this line bounded the
+// kernel: 0.60 ms for two 512x256x512 fields, now 0.48 ms, which the
+// other lines take.
+constexpr int MCH = 256;
+
 template <typename T2>
-__device__ void mean_mode_fp64(const Geom& g, const Metrics<double>& m, T2* spec, double* w) {
-  const int ny = g.ny;
+__device__ void mean_mode_fp64(const Geom& g, const Metrics<double>& m,
+                               const double* __restrict__ fac, T2* spec, double* w) {
+  __shared__ double sv[2][MCH], sa[MCH], sd[MCH];
+  const int ny = g.ny, t = threadIdx.x;
   const long long P = g.P;
-  double vecm = 1.0, cprev = 0.0, fx = w[3 * ny], fy = 0.0;  // row 0: the gauge row
-  w[0] = fx;
-  w[ny] = 0.0;
-  w[2 * ny] = 0.0;
-  for (int j0 = 1; j0 < ny; ++j0) {
-    const int jr = j0 + 1;
-    const double arr = cprev / vecm;
-    const double a = m.am2Pr[jr];
-    vecm = ((m.ac2Pr[jr] + m.wavex[0]) + m.wavez[0]) - a * arr;
-    const T2 fj = spec[P * j0];
-    fx = ((double)fj.x - a * fx) / vecm;
-    fy = ((double)fj.y - a * fy) / vecm;
-    w[j0] = fx;
-    w[ny + j0] = fy;
-    w[2 * ny + j0] = arr;
-    cprev = m.ap2Pr[jr];
+  double f = 0.0;
+  for (int c0 = 0; c0 < ny; c0 += MCH) {
+    const int n = min(MCH, ny - c0);
+    __syncthreads();
+    if (t < n) {
+      const T2 v = spec[P * (c0 + t)];
+      sv[0][t] = c0 + t == 0 ? w[3 * ny] : (double)v.x;  // row 0: the gauge row
+      sv[1][t] = c0 + t == 0 ? 0.0 : (double)v.y;
+      sa[t] = c0 + t == 0 ? 0.0 : m.am2Pr[c0 + t + 1];
+      sd[t] = fac[c0 + t];
+    }
+    __syncthreads();
+    if (t < 2) {
+      int r = 0;
+      if (c0 == 0) {
+        f = sv[t][0];
+        r = 1;
+      }
+#pragma unroll 8
+      for (; r < n; ++r) {
+        f = (sv[t][r] - sa[r] * f) / sd[r];
+        sv[t][r] = f;
+      }
+    }
+    __syncthreads();
+    if (t < n) {
+      w[c0 + t] = sv[0][t];
+      w[ny + c0 + t] = sv[1][t];
+    }
   }
-  T2 o;
-  o.x = fx;
-  o.y = fy;
-  spec[P * (ny - 1)] = o;
-  for (int j0 = ny - 2; j0 >= 0; --j0) {
-    fx = w[j0] - w[2 * ny + j0 + 1] * fx;
-    fy = w[ny + j0] - w[2 * ny + j0 + 1] * fy;
-    o.x = fx;
-    o.y = fy;
-    spec[P * j0] = o;
+  // backward: x_j = w_j - arr_{j+1} x_{j+1}, the last row's f is x
+  for (int c0 = (ny - 1) / MCH * MCH; c0 >= 0; c0 -= MCH) {
+    const int n = min(MCH, ny - c0);
+    __syncthreads();
+    if (t < n) {
+      sv[0][t] = w[c0 + t];
+      sv[1][t] = w[ny + c0 + t];
+      sa[t] = c0 + t + 1 < ny ? fac[ny + c0 + t + 1] : 0.0;
+    }
+    __syncthreads();
+    if (t < 2) {
+      int r = n - 1;
+      if (c0 + r == ny - 1) --r;  // already f
+#pragma unroll 8
+      for (; r >= 0; --r) {
+        f = sv[t][r] - sa[r] * f;
+        sv[t][r] = f;
+      }
+    }
+    __syncthreads();
+    if (t < n) {
+      T2 o;
+      o.x = sv[0][t];
+      o.y = sv[1][t];
+      spec[P * (c0 + t)] = o;
+    }
   }
 }
 
-template <typename T, int C>
+// Workgroup 0 of a field solves the (0,0) mode, the others every other line
+// by the checkpointed elimination.
+template <typename T, int C, bool NTS>
 __global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, Metrics<T> m, Metrics<double> md,
+                                                       const double* __restrict__ fac,
                                                        typename CT2<T>::t* __restrict__ spec,
                                                        T* __restrict__ ckp, double* w,
                                                        long long bsp, long long bck,
                                                        long long bw) {
-  spec += bsp * blockIdx.z;
-  ckp += bck * blockIdx.z;
-  w += bw * blockIdx.z;
-  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && threadIdx.y == 0) {
-    mean_mode_fp64(g, md, spec, w);
+  spec += bsp * blockIdx.y;
+  if (blockIdx.x == 0) {
+    mean_mode_fp64(g, md, fac, spec, w + bw * blockIdx.y);
     return;
   }
-  // every other mode: the checkpointed elimination (the (0,0) thread left)
-  k_tridiag_ck_body<T, C>(g, m, spec, ckp);
+  const long long l = (long long)(blockIdx.x - 1) * 256 + threadIdx.x;
+  if (l == 0) return;
+  k_tridiag_ck_body<T, C, NTS>(g, m, spec, ckp + bck * blockIdx.y, line_of(g, l));
 }
 
 // r = f - L phi in FP64, L the discrete operator the spectral solve inverts:
@@ -666,9 +727,10 @@ static int ppe_mixed(c3d_ctx* c, const void* prsrc, void* phi, int sweeps, void*
     hipEvent_t ev;
     prof_begin(c, ST_TRIDIAG, &ev);
     constexpr int CSEG = 16;
-    dim3 grid((g.nk + 1 + 63) / 64, (g.nz + 3) / 4, b.n), blk(64, 4);
-    hipLaunchKernelGGL((k_tridiag_mixed<float, CSEG>), grid, blk, 0, c->stream, g, c->mf, c->md,
-                       (float2*)spec, (float*)ck, w, b.spec32, b.ck, b.mean);
+    const long long nl = (long long)(g.nk + 1) * g.nz;
+    const dim3 grid((unsigned)(1 + (nl + 255) / 256), b.n), blk(256);
+    hipLaunchKernelGGL((k_tridiag_mixed<float, CSEG, false>), grid, blk, 0, c->stream, g, c->mf,
+                       c->md, c->d_meanfac, (float2*)spec, (float*)ck, w, b.spec32, b.ck, b.mean);
     C3D_HIP(hipGetLastError());
     prof_end(c, ST_TRIDIAG, ev, 2.0 * (double)g.nx * g.ny * g.nz * b.n * 4);
     return launch_fft32(c, FFT32_Z_INV, nullptr, spec, nullptr, 0, b);

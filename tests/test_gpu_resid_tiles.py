@@ -34,7 +34,12 @@ def _fields(g, nb, compatible):
     return out
 
 
-@pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
+# the (0, 0) mode's line moves through LDS 256 rows at a time: one row more, two chunks
+# and a remainder
+LONG = [(16, 257, 8), (16, 530, 8), (16, 256, 8)]
+
+
+@pytest.mark.parametrize("grid", GRIDS + LONG, ids=lambda v: "x".join(map(str, v)))
 def test_pressure_refinement(grid):
     from channel3d_amd import lib as L
     with _channel(*grid) as g:
