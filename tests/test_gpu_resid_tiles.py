@@ -2,10 +2,11 @@
 64 x cells per wavefront (a last tile of 2 cells, one exact tile, less than a
 tile), blocks of 4 and 8 rows in workgroups of 16 and 32, z chunks with
 remainders.  A cell whose residual is wrong keeps the FP32 solve's error, so
-the refined solution must agree with the FP64 solve of the same source (which
-the oracle tests cover) everywhere: each sweep multiplies the error by the FP32
-solve's relative error, at most 1e-5 here for the pressure and 1e-6 for the
-velocity operator."""
+the refined solution must approach the FP64 solve of the same source (which
+the oracle tests cover) everywhere.  Bounds: a sweep multiplies the error by at
+most the FP32 solve's relative error, FP32's eps times the condition number of
+the operator: about ny^2 for the Neumann line of the pressure's mean mode, below
+20 for the velocity operator; what remains is FP64 rounding (1e-12)."""
 import math
 
 import numpy as np
@@ -43,15 +44,18 @@ LONG = [(16, 257, 8), (16, 530, 8), (16, 256, 8)]
 def test_pressure_refinement(grid):
     from channel3d_amd import lib as L
     with _channel(*grid) as g:
-        src, a, b = (g.alloc_batch(lay, 2) for lay in (L.INTERIOR, L.HALO, L.HALO))
+        src, a, b0, b2 = (g.alloc_batch(lay, 2) for lay in (L.INTERIOR,) + (L.HALO,) * 3)
         for q, f in enumerate(_fields(g, 2, True)):
             g.upload(src[q], f, L.INTERIOR)
-        g.ppe_batch(src, a, -1)
-        g.ppe_batch(src, b, 2)
+        for out, sweeps in ((a, -1), (b0, 0), (b2, 2)):
+            g.ppe_batch(src, out, sweeps)
         n = slice(1, g.nyc + 1)
+        rate = min(0.1, np.finfo(np.float32).eps * g.nyc ** 2)
         for q in range(2):
-            x, y = (g.download(h[q], L.HALO)[1:-2, n, 1:-2] for h in (a, b))
-            assert np.abs(x - y).max() <= 1e-10 * np.abs(x).max()
+            x, y0, y2 = (g.download(h[q], L.HALO)[1:-2, n, 1:-2] for h in (a, b0, b2))
+            e0, e2 = (np.abs(x - y).max() / np.abs(x).max() for y in (y0, y2))
+            assert e0 <= rate
+            assert e2 <= rate ** 2 * e0 + 1e-12
 
 
 @pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
@@ -66,4 +70,4 @@ def test_velocity_refinement(grid, comp):
         g.helmholtz_batch(comp, 1, rhs, b, 1)
         for q in range(2):
             x, y = g.download(a[q], L.INTERIOR), g.download(b[q], L.INTERIOR)
-            assert np.abs(x - y).max() <= 1e-11 * np.abs(x).max()
+            assert np.abs(x - y).max() <= 1e-11 * np.abs(x).max()  # (20 eps)^2, rounding
