@@ -35,35 +35,6 @@ struct View {
   }
 };
 
-// 4-point interpolations of the helper fields: "A" uses offsets -1..+2
-// (uxhx in x, uzhz in z), "B" offsets -2..+1 (uyhx, uzhx in x; uxhz, uyhz in z)
-template <typename T>
-__device__ __forceinline__ T ix_a(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.ic1 * f(i - 1, j, k) + c.ic2 * f(i, j, k) + c.ic3 * f(i + 1, j, k) + c.ic4 * f(i + 2, j, k);
-}
-template <typename T>
-__device__ __forceinline__ T ix_b(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.ic1 * f(i - 2, j, k) + c.ic2 * f(i - 1, j, k) + c.ic3 * f(i, j, k) + c.ic4 * f(i + 1, j, k);
-}
-template <typename T>
-__device__ __forceinline__ T iz_a(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.ic1 * f(i, j, k - 1) + c.ic2 * f(i, j, k) + c.ic3 * f(i, j, k + 1) + c.ic4 * f(i, j, k + 2);
-}
-template <typename T>
-__device__ __forceinline__ T iz_b(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.ic1 * f(i, j, k - 2) + c.ic2 * f(i, j, k - 1) + c.ic3 * f(i, j, k) + c.ic4 * f(i, j, k + 1);
-}
-// 5-point second differences
-template <typename T>
-__device__ __forceinline__ T dxx5(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.dxx1 * f(i - 2, j, k) + c.dxx2 * f(i - 1, j, k) + c.dxx3 * f(i, j, k) +
-         c.dxx4 * f(i + 1, j, k) + c.dxx5 * f(i + 2, j, k);
-}
-template <typename T>
-__device__ __forceinline__ T dzz5(const View<T>& f, const Coef4<T>& c, int i, int j, int k) {
-  return c.dzz1 * f(i, j, k - 2) + c.dzz2 * f(i, j, k - 1) + c.dzz3 * f(i, j, k) +
-         c.dzz4 * f(i, j, k + 1) + c.dzz5 * f(i, j, k + 2);
-}
 
 // 1-D grid of 64 x 4 (i, j) tiles times z runs, XCD-remapped, x fastest
 #define CELL4_BLOCK(KCH)                                                      \
@@ -112,22 +83,61 @@ __device__ __forceinline__ double block_max4(double v, double* sh) {
 // coupling).  RhsX (:243-290), RhsY (:293-330), RhsZ (:333-370); with
 // want_flow the block partial of s3tot = sum (d11+d33+d22) dyp (:271) is
 // accumulated as reproducible fixed-point limbs.
+//
+// A wavefront owns 64 x cells of one row and marches a run of z planes.
+//  - z: every value along the own column (u, v, w, p, uy one row up, and the
+//    z- and x-interpolated factors of the z fluxes) enters once, when its
+//    plane arrives, and rolls through registers.
+//  - x: each plane's rows go through LDS with three cells on either side; lane
+//    n < 6 also carries one of those six edge columns.  A row belongs to its
+//    wavefront alone and a wavefront's LDS accesses complete in order, so
+//    nothing waits at a workgroup barrier.
+//  - y: the neighbour rows are read directly; the wavefront one row over has
+//    just read them, so they come from L1.
+// The next plane's words are requested before this plane is computed, and this
+// plane's results are stored after that, so waiting for the one never waits
+// for the other.  26 memory operations per wavefront and plane where every
+// operand fetched on its own took about 110, each with its own periodic index:
+// bound by the FP64 pipeline (about 450 operations per cell, uncontracted)
+// and HBM (13 words).  192x128x160 FP64: 0.288 ms so, 0.125 ms now (3.3 TB/s
+// of its 13 words).
 // ---------------------------------------------------------------------------
+constexpr int R4E = 3;                 // edge columns on either side
+constexpr int R4L = 64 + 2 * R4E + 2;  // an LDS row, with a slot for idle lanes
+
 template <typename T>
 __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef4<T> cf,
                                                    const double* __restrict__ dyp,
-                                                   const T* __restrict__ ux_, const T* __restrict__ uy_,
-                                                   const T* __restrict__ uz_, const T* __restrict__ pr_,
+                                                   const T* __restrict__ ux, const T* __restrict__ uy,
+                                                   const T* __restrict__ uz, const T* __restrict__ pr,
                                                    T* __restrict__ rx, T* __restrict__ ry,
                                                    T* __restrict__ rz, T* __restrict__ hx,
                                                    T* __restrict__ hy, T* __restrict__ hz,
-                                                   double* __restrict__ partials, int want_flow) {
+                                                   double* __restrict__ partials, int want_flow,
+                                                   int kchunk) {
   __shared__ long long shf[8][4];
-  CELL4_BLOCK(K4CH);
+  enum { RU, RV, RW, RP, RVP, RUM, RIZ, RW2, NROW };
+  __shared__ T rows[B4Y][NROW][R4L];
+  const int gxb = (g.nx + B4X - 1) / B4X, gyb = (g.ny + B4Y - 1) / B4Y;
+  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int i0 = (lb % gxb) * B4X;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int jc = ((lb / gxb) % gyb) * B4Y + wv + 1;
+  const int k0 = (lb / (gxb * gyb)) * kchunk, k1 = min(g.nz, k0 + kchunk);
+  const int lane = threadIdx.x;
+  const int nx = g.nx, nz = g.nz;
   long long s3[4] = {0, 0, 0, 0};
-  if (i < g.nx && jc <= g.ny) {
-    const View<T> ux{ux_, g.nx, g.nz, g.plane}, uy{uy_, g.nx, g.nz, g.plane};
-    const View<T> uz{uz_, g.nx, g.nz, g.plane}, pr{pr_, g.nx, g.nz, g.plane};
+  if (jc <= g.ny) {
+    const int last = min(B4X, nx - i0) - 1;
+    const bool live = lane <= last;
+    const int i = min(i0 + lane, nx - 1);
+    // edge column of lanes 0..5 and its place in a row; idle lanes repeat
+    // lane 0's column into the spare slot
+    const int ie = lane < 3 || lane >= 6 ? wr(i0 - 3 + (lane < 3 ? lane : 0), nx)
+                                         : wr(i0 + last + 1 + lane - 3, nx);
+    const int pe = lane < 3 ? lane : lane < 6 ? last + 1 + lane : R4L - 1;
+    const int e = R4E + lane;
+    T(*const row)[R4L] = rows[wv];
     const int jm = jc - 1, jp = jc + 1, nyp = g.ny + 1;
     const T sucaj = m.rdyp[jc], sucac = m.rdyc[jc];
     const T qsucac = T(0.25) * sucac;
@@ -137,89 +147,246 @@ __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef
     const T am2p = m.am2p[jc], ac2p = m.ac2p[jc], ap2p = m.ap2p[jc];
     const double dy = dyp[jc];
     const T ucrf = cf.ucrf;
+    // word at byte `at` of row j, plane k (periodic): a scalar row address
+    // plus a 32-bit lane offset
+    auto ld = [&](const T* f, int j, int k, unsigned at) {
+      return *(const T*)((const char*)(f + ((long long)nx * j + g.plane * wr(k, nz))) + at);
+    };
+    const unsigned oi = i * (unsigned)sizeof(T), oe = ie * (unsigned)sizeof(T);
+    // 4-point interpolation (-1, 9, 9, -1)/16, difference (1, -27, 27, -1)/24
+    // and second difference (-1, 16, -30, 16, -1)/12 of neighbouring values.
+    // The weights are symmetric to the bit, so one of each pair is kept: a
+    // product with the negated weight, subtracted, rounds the same.
+    auto i4 = [](T a, T b, T c, T d) {
+      return T(-0.0625) * a + T(0.5625) * b + T(0.5625) * c + T(-0.0625) * d;
+    };
+    const T dx1 = cf.dx1, dx3 = cf.dx3, dz1 = cf.dz1, dz3 = cf.dz3;
+    auto d5x = [&](T a, T b, T c, T d, T f) {
+      return cf.dxx1 * a + cf.dxx2 * b + cf.dxx3 * c + cf.dxx2 * d + cf.dxx1 * f;
+    };
+    auto d5z = [&](const T* c) {
+      return cf.dzz1 * c[0] + cf.dzz2 * c[1] + cf.dzz3 * c[2] + cf.dzz2 * c[3] + cf.dzz1 * c[4];
+    };
+    auto put = [&](int r, T own, T edge) {
+      row[r][e] = own;
+      row[r][pe] = edge;  // after the own cells: a partial tile's right edge wins
+    };
+    auto fence = [&]() {
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      __builtin_amdgcn_wave_barrier();
+    };
+    // x interpolation ("B") of the row in r at the own cell
+    auto ixb_of = [&](int r) { return i4(row[r][e - 2], row[r][e - 1], row[r][e], row[r][e + 1]); };
+
+    // the words of one plane's step: u, v, w at k+3; uz one row down at k+2;
+    // p, uy one row up and the edge of ux at k+1; the rest at k
+    struct Next {
+      T u3, v3, w3, wm2, ew2, p1, vp1, eu1;
+      T um, up, vm, wp, pm, ev, ep, evp, eum, hx, hy, hz;
+    };
+    auto fetch = [&](int k, Next& n) {
+      const int kc = wr(k, nz);
+      n.hx = ld(hx, jc, kc, oi);
+      n.hy = ld(hy, jc, kc, oi);
+      n.hz = ld(hz, jc, kc, oi);
+      n.u3 = ld(ux, jc, k + 3, oi);
+      n.v3 = ld(uy, jc, k + 3, oi);
+      n.w3 = ld(uz, jc, k + 3, oi);
+      n.wm2 = ld(uz, jm, k + 2, oi);
+      n.ew2 = ld(uz, jc, k + 2, oe);
+      n.p1 = ld(pr, jc, k + 1, oi);
+      n.vp1 = ld(uy, jp, k + 1, oi);
+      n.eu1 = ld(ux, jc, k + 1, oe);
+      n.um = ld(ux, jm, kc, oi);
+      n.up = ld(ux, jp, kc, oi);
+      n.vm = ld(uy, jm, kc, oi);
+      n.wp = ld(uz, jp, kc, oi);
+      n.pm = ld(pr, jm, kc, oi);
+      n.ev = ld(uy, jc, kc, oe);
+      n.ep = ld(pr, jc, kc, oe);
+      n.evp = ld(uy, jp, kc, oe);
+      n.eum = ld(ux, jm, kc, oe);
+    };
+
+    // rolled columns; index 0 is the oldest plane named beside each
+    T u[6], v[6], w[6];             // k-2 .. k+3
+    T zu[4], zv[4], xw[4], yw[4];   // izb(ux), izb(uy), ixb(uz), uz at the xz edge: k-1 .. k+2
+    T za[4];                        // iza(uz): k-2 .. k+1
+    T p[4], vp[4], eu[4];           // k-2 .. k+1
+    T wm[3], ew[3];                 // k .. k+2
+    {
+      T a[6], b[6], c[6];           // planes k0-3 .. k0+2
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        a[q] = ld(ux, jc, k0 - 3 + q, oi);
+        b[q] = ld(uy, jc, k0 - 3 + q, oi);
+        c[q] = ld(uz, jc, k0 - 3 + q, oi);
+      }
+      T wl[3], el[3];               // planes k0-1 .. k0+1
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        wl[q] = ld(uz, jm, k0 - 1 + q, oi);
+        el[q] = ld(uz, jc, k0 - 1 + q, oe);
+        p[q + 1] = ld(pr, jc, k0 - 2 + q, oi);
+        vp[q + 1] = ld(uy, jp, k0 - 2 + q, oi);
+        eu[q + 1] = ld(ux, jc, k0 - 2 + q, oe);
+      }
+      // every column holds its values one slot up: the first step shifts
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        u[q + 1] = a[q + 1];
+        v[q + 1] = b[q + 1];
+        w[q + 1] = c[q + 1];
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        zu[q + 1] = i4(a[q], a[q + 1], a[q + 2], a[q + 3]);
+        zv[q + 1] = i4(b[q], b[q + 1], b[q + 2], b[q + 3]);
+        za[q + 1] = i4(c[q], c[q + 1], c[q + 2], c[q + 3]);
+        yw[q + 1] = IY1 * wl[q] + IY2 * c[q + 2];
+        put(RW2, c[q + 2], el[q]);
+        fence();
+        xw[q + 1] = ixb_of(RW2);
+        fence();
+      }
+      wm[1] = wl[1];
+      wm[2] = wl[2];
+      ew[1] = el[1];
+      ew[2] = el[2];
+    }
+
+    Next n;
+    fetch(k0, n);
     for (int k = k0; k < k1; ++k) {
-      const long long c = fidx(g, i, jc, k);
+      // the arriving planes
+#pragma unroll
+      for (int q = 0; q < 5; ++q) {
+        u[q] = u[q + 1];
+        v[q] = v[q + 1];
+        w[q] = w[q + 1];
+      }
+      u[5] = n.u3;
+      v[5] = n.v3;
+      w[5] = n.w3;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        zu[q] = zu[q + 1];
+        zv[q] = zv[q + 1];
+        xw[q] = xw[q + 1];
+        yw[q] = yw[q + 1];
+        za[q] = za[q + 1];
+        p[q] = p[q + 1];
+        vp[q] = vp[q + 1];
+        eu[q] = eu[q + 1];
+      }
+      p[3] = n.p1;
+      vp[3] = n.vp1;
+      eu[3] = n.eu1;
+      wm[0] = wm[1]; wm[1] = wm[2]; wm[2] = n.wm2;
+      ew[0] = ew[1]; ew[1] = ew[2]; ew[2] = n.ew2;
+      zu[3] = i4(u[2], u[3], u[4], u[5]);
+      zv[3] = i4(v[2], v[3], v[4], v[5]);
+      za[3] = i4(w[2], w[3], w[4], w[5]);
+      yw[3] = IY1 * wm[2] + IY2 * w[4];
+      const T uc = u[2], vc = v[2], wc = w[2], pc = p[2];
+      put(RU, uc, eu[2]);
+      put(RV, vc, n.ev);
+      put(RW, wc, ew[0]);
+      put(RP, pc, n.ep);
+      put(RVP, vp[2], n.evp);
+      put(RUM, n.um, n.eum);
+      put(RIZ, zu[1], i4(eu[0], eu[1], eu[2], eu[3]));
+      put(RW2, w[4], ew[2]);
+      const T um = n.um, up = n.up, vm = n.vm, wp = n.wp, pm = n.pm;
+      const T hxo = n.hx, hyo = n.hy, hzo = n.hz;
+      fence();
+      // past the run's last plane this reads (periodic) planes it drops
+      fetch(k + 1, n);
+      fence();
+      const T* U = row[RU] + e;
+      const T* V = row[RV] + e;
+      const T* W = row[RW] + e;
+      const T* P = row[RP] + e;
+      const T* UM = row[RUM] + e;
+      const T* IZ = row[RIZ] + e;
+      xw[3] = ixb_of(RW2);
+      auto sto = [&](T* f, T val) {
+        if (live) *(T*)((char*)(f + ((long long)nx * jc + g.plane * k)) + oi) = val;
+      };
+      // The three components one after the other: moved together, their LDS
+      // operands do not fit the registers.
       // ---- RhsX ----
       {
-        const T uxhyc = IY1 * ux(i, jm, k) + IY2 * ux(i, jc, k);
-        const T uxhyp = IY3 * ux(i, jc, k) + IY4 * ux(i, jp, k);
-        const T as = ix_a(ux, cf, i - 2, jc, k), am = ix_a(ux, cf, i - 1, jc, k);
-        const T ac = ix_a(ux, cf, i, jc, k), ap = ix_a(ux, cf, i + 1, jc, k);
-        const T h11 = cf.dx1 * as * (as + ucrf) + cf.dx2 * am * (am + ucrf) +
-                      cf.dx3 * ac * (ac + ucrf) + cf.dx4 * ap * (ap + ucrf);
-        const T uyhx_p = (jp == nyp) ? T(0) : ix_b(uy, cf, i, jp, k);
-        const T uyhx_c = ix_b(uy, cf, i, jc, k);
-        const T h12 = (uyhx_p * uxhyp - uyhx_c * uxhyc) * sucaj;
-        const T h13 = cf.dz1 * iz_b(ux, cf, i, jc, k - 1) * ix_b(uz, cf, i, jc, k - 1) +
-                      cf.dz2 * iz_b(ux, cf, i, jc, k) * ix_b(uz, cf, i, jc, k) +
-                      cf.dz3 * iz_b(ux, cf, i, jc, k + 1) * ix_b(uz, cf, i, jc, k + 1) +
-                      cf.dz4 * iz_b(ux, cf, i, jc, k + 2) * ix_b(uz, cf, i, jc, k + 2);
-        const T d11 = dxx5(ux, cf, i, jc, k);
-        const T d22 = ap2c * ux(i, jp, k) + ac2c * ux(i, jc, k) + am2c * ux(i, jm, k);
-        const T d33 = dzz5(ux, cf, i, jc, k);
+        const T u3m = U[-3], u2m = U[-2], u1m = U[-1], u1p = U[1], u2p = U[2], u3p = U[3];
+        const T vxc = ixb_of(RV);
+        const T uxhyc = IY1 * um + IY2 * uc;
+        const T uxhyp = IY3 * uc + IY4 * up;
+        const T as = i4(u3m, u2m, u1m, uc), am = i4(u2m, u1m, uc, u1p);
+        const T ac = i4(u1m, uc, u1p, u2p), ap = i4(uc, u1p, u2p, u3p);
+        const T h11 = dx1 * as * (as + ucrf) - dx3 * am * (am + ucrf) + dx3 * ac * (ac + ucrf) -
+                      dx1 * ap * (ap + ucrf);
+        const T uyhx_p = (jp == nyp) ? T(0) : ixb_of(RVP);
+        const T h12 = (uyhx_p * uxhyp - vxc * uxhyc) * sucaj;
+        const T h13 = dz1 * zu[0] * xw[0] - dz3 * zu[1] * xw[1] + dz3 * zu[2] * xw[2] -
+                      dz1 * zu[3] * xw[3];
+        const T d11 = d5x(u2m, u1m, uc, u1p, u2p);
+        const T d22 = ap2c * up + ac2c * uc + am2c * um;
+        const T d33 = d5z(u);
         const T dcq13 = d11 + d33;
-        if (want_flow) fix_add(s3, (double)(dcq13 + d22) * dy);
+        if (want_flow && live) fix_add(s3, (double)(dcq13 + d22) * dy);
         const T conv = -h11 - h12 - h13 + cf.xnu * dcq13 + cf.gx;
-        const T gradp = cf.dx1 * pr(i - 2, jc, k) + cf.dx2 * pr(i - 1, jc, k) +
-                        cf.dx3 * pr(i, jc, k) + cf.dx4 * pr(i + 1, jc, k);
-        // read and written once: non-temporal
-        const T hold_ = C3D_LD_ONCE(&hx[c]);
-        C3D_ST_ONCE(cf.pmGamma * conv + cf.pmTheta * hold_ - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22, &rx[c]);
-        C3D_ST_ONCE(conv, &hx[c]);
+        const T gradp = dx1 * P[-2] - dx3 * P[-1] + dx3 * pc - dx1 * P[1];
+        sto(rx, cf.pmGamma * conv + cf.pmTheta * hxo - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22);
+        sto(hx, conv);
       }
+      __builtin_amdgcn_sched_barrier(0);
       // ---- RhsY ----
       {
-        const T uxhym = IY1 * ux(i - 1, jm, k) + IY2 * ux(i - 1, jc, k) + ucrf;
-        const T uzhym = IY1 * uz(i, jm, k - 1) + IY2 * uz(i, jc, k - 1);
-        const T uxhyc = IY1 * ux(i, jm, k) + IY2 * ux(i, jc, k) + ucrf;
-        const T uzhyc = IY1 * uz(i, jm, k) + IY2 * uz(i, jc, k);
-        const T uxhyp = IY1 * ux(i + 1, jm, k) + IY2 * ux(i + 1, jc, k) + ucrf;
-        const T uzhyp = IY1 * uz(i, jm, k + 1) + IY2 * uz(i, jc, k + 1);
-        const T uxhyu = IY1 * ux(i + 2, jm, k) + IY2 * ux(i + 2, jc, k) + ucrf;
-        const T uzhyu = IY1 * uz(i, jm, k + 2) + IY2 * uz(i, jc, k + 2);
-        const T h21 = cf.dx1 * ix_b(uy, cf, i - 1, jc, k) * uxhym + cf.dx2 * ix_b(uy, cf, i, jc, k) * uxhyc +
-                      cf.dx3 * ix_b(uy, cf, i + 1, jc, k) * uxhyp + cf.dx4 * ix_b(uy, cf, i + 2, jc, k) * uxhyu;
-        const T vp = uy(i, jp, k), vc = uy(i, jc, k), vm = uy(i, jm, k);
-        const T h22 = ((vp + vc) * (vp + vc) - (vc + vm) * (vc + vm)) * qsucac;
-        const T h23 = cf.dz1 * iz_b(uy, cf, i, jc, k - 1) * uzhym + cf.dz2 * iz_b(uy, cf, i, jc, k) * uzhyc +
-                      cf.dz3 * iz_b(uy, cf, i, jc, k + 1) * uzhyp + cf.dz4 * iz_b(uy, cf, i, jc, k + 2) * uzhyu;
-        const T d11 = dxx5(uy, cf, i, jc, k);
-        const T d22 = ap2p * vp + ac2p * vc + am2p * vm;
-        const T d33 = dzz5(uy, cf, i, jc, k);
+        const T v3m = V[-3], v2m = V[-2], v1m = V[-1], v1p = V[1], v2p = V[2], v3p = V[3];
+        const T vxc = i4(v2m, v1m, vc, v1p);
+        const T uxhym = IY1 * UM[-1] + IY2 * U[-1] + ucrf;
+        const T uxhyc = IY1 * um + IY2 * uc + ucrf;
+        const T uxhyp = IY1 * UM[1] + IY2 * U[1] + ucrf;
+        const T uxhyu = IY1 * UM[2] + IY2 * U[2] + ucrf;
+        const T h21 = dx1 * i4(v3m, v2m, v1m, vc) * uxhym - dx3 * vxc * uxhyc +
+                      dx3 * i4(v1m, vc, v1p, v2p) * uxhyp - dx1 * i4(vc, v1p, v2p, v3p) * uxhyu;
+        const T vpc = vp[2];
+        const T h22 = ((vpc + vc) * (vpc + vc) - (vc + vm) * (vc + vm)) * qsucac;
+        const T h23 = dz1 * zv[0] * yw[0] - dz3 * zv[1] * yw[1] + dz3 * zv[2] * yw[2] -
+                      dz1 * zv[3] * yw[3];
+        const T d11 = d5x(v2m, v1m, vc, v1p, v2p);
+        const T d22 = ap2p * vpc + ac2p * vc + am2p * vm;
+        const T d33 = d5z(v);
         const T dcq13 = d11 + d33;
         const T conv = -h21 - h22 - h23 + cf.xnu * dcq13 + cf.gy;
-        const T gradp = (pr(i, jc, k) - pr(i, jm, k)) * sucac;
-        // read and written once: non-temporal
-        const T hold_ = C3D_LD_ONCE(&hy[c]);
-        C3D_ST_ONCE(cf.pmGamma * conv + cf.pmTheta * hold_ - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22, &ry[c]);
-        C3D_ST_ONCE(conv, &hy[c]);
+        const T gradp = (pc - pm) * sucac;
+        sto(ry, cf.pmGamma * conv + cf.pmTheta * hyo - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22);
+        sto(hy, conv);
       }
+      __builtin_amdgcn_sched_barrier(0);
       // ---- RhsZ ----
       {
-        const T uzhyc = IY1 * uz(i, jm, k) + IY2 * uz(i, jc, k);
-        const T uzhyp = IY3 * uz(i, jc, k) + IY4 * uz(i, jp, k);
-        const T h31 = cf.dx1 * ix_b(uz, cf, i - 1, jc, k) * (iz_b(ux, cf, i - 1, jc, k) + ucrf) +
-                      cf.dx2 * ix_b(uz, cf, i, jc, k) * (iz_b(ux, cf, i, jc, k) + ucrf) +
-                      cf.dx3 * ix_b(uz, cf, i + 1, jc, k) * (iz_b(ux, cf, i + 1, jc, k) + ucrf) +
-                      cf.dx4 * ix_b(uz, cf, i + 2, jc, k) * (iz_b(ux, cf, i + 2, jc, k) + ucrf);
-        const T uyhz_p = (jp == nyp) ? T(0) : iz_b(uy, cf, i, jp, k);
-        const T uyhz_c = iz_b(uy, cf, i, jc, k);
-        const T h32 = (uyhz_p * uzhyp - uyhz_c * uzhyc) * sucaj;
-        const T zs = iz_a(uz, cf, i, jc, k - 2), zm = iz_a(uz, cf, i, jc, k - 1);
-        const T zc = iz_a(uz, cf, i, jc, k), zp = iz_a(uz, cf, i, jc, k + 1);
-        const T h33 = cf.dz1 * zs * zs + cf.dz2 * zm * zm + cf.dz3 * zc * zc + cf.dz4 * zp * zp;
-        const T d11 = dxx5(uz, cf, i, jc, k);
-        const T d22 = ap2c * uz(i, jp, k) + ac2c * uz(i, jc, k) + am2c * uz(i, jm, k);
-        const T d33 = dzz5(uz, cf, i, jc, k);
+        const T zvp = (jp == nyp) ? T(0) : i4(vp[0], vp[1], vp[2], vp[3]);
+        const T w3m = W[-3], w2m = W[-2], w1m = W[-1], w1p = W[1], w2p = W[2], w3p = W[3];
+        const T uzhyc = IY1 * wm[0] + IY2 * wc;
+        const T uzhyp = IY3 * wc + IY4 * wp;
+        const T h31 = dx1 * i4(w3m, w2m, w1m, wc) * (IZ[-1] + ucrf) -
+                      dx3 * xw[1] * (zu[1] + ucrf) +
+                      dx3 * i4(w1m, wc, w1p, w2p) * (IZ[1] + ucrf) -
+                      dx1 * i4(wc, w1p, w2p, w3p) * (IZ[2] + ucrf);
+        const T h32 = (zvp * uzhyp - zv[1] * uzhyc) * sucaj;
+        const T h33 = dz1 * za[0] * za[0] - dz3 * za[1] * za[1] + dz3 * za[2] * za[2] -
+                      dz1 * za[3] * za[3];
+        const T d11 = d5x(w2m, w1m, wc, w1p, w2p);
+        const T d22 = ap2c * wp + ac2c * wc + am2c * wm[0];
+        const T d33 = d5z(w);
         const T dcq13 = d11 + d33;
         const T conv = -h31 - h32 - h33 + cf.xnu * dcq13 + cf.gz;
-        const T gradp = cf.dz1 * pr(i, jc, k - 2) + cf.dz2 * pr(i, jc, k - 1) +
-                        cf.dz3 * pr(i, jc, k) + cf.dz4 * pr(i, jc, k + 1);
-        // read and written once: non-temporal
-        const T hold_ = C3D_LD_ONCE(&hz[c]);
-        C3D_ST_ONCE(cf.pmGamma * conv + cf.pmTheta * hold_ - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22, &rz[c]);
-        C3D_ST_ONCE(conv, &hz[c]);
+        const T gradp = dz1 * p[0] - dz3 * p[1] + dz3 * pc - dz1 * p[3];
+        sto(rz, cf.pmGamma * conv + cf.pmTheta * hzo - cf.pmAlpha * gradp + T(2) * cf.pmBeta * d22);
+        sto(hz, conv);
       }
+      fence();
     }
   }
   if (want_flow) {
@@ -229,6 +396,24 @@ __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef
       for (int q = 0; q < 4; ++q) pf[q] = s3[q];
     }
   }
+}
+
+// z planes per wavefront: the run that finishes first, counting the rounds of
+// wavefronts the device holds at two per SIMD and four planes' worth of
+// lead-in per run
+static int rhs4_kchunk(const Geom& g) {
+  const long long wv = (long long)((g.nx + B4X - 1) / B4X) * ((g.ny + B4Y - 1) / B4Y * B4Y);
+  long long best = 0;
+  int kc = g.nz;
+  for (int n = 1; n <= (g.nz + 3) / 4; ++n) {
+    const int c = (g.nz + n - 1) / n;
+    const long long cost = (wv * ((g.nz + c - 1) / c) + 2047) / 2048 * (c + 4);
+    if (best == 0 || cost < best) {
+      best = cost;
+      kc = c;
+    }
+  }
+  return kc;
 }
 
 // constant flow rate of the 4th-order code (m_TScheme.f90:392-407):
@@ -433,7 +618,8 @@ template <typename T>
 static int rhs4_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, const void* pr,
                   void* rx, void* ry, void* rz, void* hx, void* hy, void* hz, int want_flow) {
   const Geom& g = c->g;
-  const int nb = nblocks4(g, K4CH);
+  const int kc = rhs4_kchunk(g);
+  const int nb = nblocks4(g, kc);
   if (want_flow && 4 * nb > c->max_partials) {
     set_error("rhs4: partial buffer too small");
     return C3D_ERR_ARG;
@@ -441,7 +627,7 @@ static int rhs4_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, co
   hipLaunchKernelGGL((k_rhs4<T>), dim3(nb), dim3(B4X, B4Y), 0, c->stream, g, mets4<T>(c),
                      make_coef4<T>(c), (const double*)c->d_dyp, (const T*)ux, (const T*)uy,
                      (const T*)uz, (const T*)pr, (T*)rx, (T*)ry, (T*)rz, (T*)hx, (T*)hy, (T*)hz,
-                     c->d_partials, want_flow);
+                     c->d_partials, want_flow, kc);
   C3D_HIP(hipGetLastError());
   if (want_flow) {
     hipLaunchKernelGGL(k_flow4_finalize, dim3(1), dim3(1024), 0, c->stream, c->d_partials, nb,
