@@ -490,6 +490,23 @@ struct BatchWork {
 // mixed solve's FP32 tables must exist)
 int ppe_batch_ws(c3d_ctx* c, int nb, const void* prsrc, void* phi, int sweeps,
                  const BatchWork& ws);
+// z planes per run of a kernel whose wavefronts march z, `per_plane` of them
+// side by side: the split that finishes first, counting the rounds of
+// wavefronts the device holds at two per SIMD and `lead` planes' worth of work
+// before each run's first result.
+inline int march_kchunk(long long per_plane, int nz, int lead) {
+  long long best = 0;
+  int kc = nz;
+  for (int n = 1; n <= (nz + 3) / 4; ++n) {
+    const int c = (nz + n - 1) / n;
+    const long long cost = (per_plane * ((nz + c - 1) / c) + 2047) / 2048 * (c + lead);
+    if (best == 0 || cost < best) {
+      best = cost;
+      kc = c;
+    }
+  }
+  return kc;
+}
 // z planes per workgroup of the residual kernels, which march z over `tiles`
 // x-y tiles of nb fields: long runs amortise the lead-in plane, short ones
 // keep every CU supplied on small grids (a target of 8 workgroups per CU)

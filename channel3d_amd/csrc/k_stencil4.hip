@@ -398,24 +398,6 @@ __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef
   }
 }
 
-// z planes per wavefront: the run that finishes first, counting the rounds of
-// wavefronts the device holds at two per SIMD and four planes' worth of
-// lead-in per run
-static int rhs4_kchunk(const Geom& g) {
-  const long long wv = (long long)((g.nx + B4X - 1) / B4X) * ((g.ny + B4Y - 1) / B4Y * B4Y);
-  long long best = 0;
-  int kc = g.nz;
-  for (int n = 1; n <= (g.nz + 3) / 4; ++n) {
-    const int c = (g.nz + n - 1) / n;
-    const long long cost = (wv * ((g.nz + c - 1) / c) + 2047) / 2048 * (c + 4);
-    if (best == 0 || cost < best) {
-      best = cost;
-      kc = c;
-    }
-  }
-  return kc;
-}
-
 // constant flow rate of the 4th-order code (m_TScheme.f90:392-407):
 // dpmdxns = xnu * s3tot1 / (nxc*nzc) / yly, dp1ns = pmAlpha * dpmdxns,
 // PrGradAver += dpmdxns * pmAlphaC (reset by PMcoeUpdate at ns=1).
@@ -618,7 +600,8 @@ template <typename T>
 static int rhs4_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, const void* pr,
                   void* rx, void* ry, void* rz, void* hx, void* hy, void* hz, int want_flow) {
   const Geom& g = c->g;
-  const int kc = rhs4_kchunk(g);
+  const int kc = march_kchunk((long long)((g.nx + B4X - 1) / B4X) * ((g.ny + B4Y - 1) / B4Y * B4Y),
+                              g.nz, 4);
   const int nb = nblocks4(g, kc);
   if (want_flow && 4 * nb > c->max_partials) {
     set_error("rhs4: partial buffer too small");

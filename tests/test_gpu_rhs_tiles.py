@@ -1,8 +1,7 @@
-"""The 4th-order right-hand sides at the edges of their tiles, bit for bit
-against the oracle: 64 x cells per wavefront with three cells taken from beside
-them (a last tile of 2 cells, of 8, an exact tile, less than one tile), four
-rows per workgroup (one, two or three of them past the top), runs of z planes
-with remainders and with every plane a periodic neighbour of the others."""
+"""The 4th-order and LES right-hand sides at the edges of their tiles, bit for bit
+against the oracle: 64 x cells per wavefront with the cells beside them (a
+last tile of 2 cells, of 8, an exact tile, less than one tile), four rows
+per workgroup (one, two or three of them past the top), runs of z planes with remainders and with every plane a periodic neighbour of the others."""
 import numpy as np
 import pytest
 
@@ -39,5 +38,37 @@ def test_rhs4_tiles_bitwise(O, grid, half):
         assert np.abs(g.download(gid) - o.field(fid)).max() == 0.0, fid
     assert np.abs(interior4(g.download(L.HALOARR)) - interior4(rz)).max() == 0.0
     assert g.diagnostics()["PrGradNow"] == o.scalar(O.S_PRGRADNOW)
+    g.close()
+    o.close()
+
+
+@pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
+def test_rhs_les_tiles_bitwise(O, grid):
+    from channel3d_amd import lib as L
+    from tests import test_gpu_parity as P2
+    nx, ny, nz = grid
+    o, g = P2.make_pair(O, dict(cases.SMALL, nxc=nx, nyc=ny, nzc=nz, les_type=3, filter_type=1),
+                        laminar=False)
+    P2.random_state(O, o, g, seed=ny)
+    u = (o.field(O.UX), o.field(O.UY), o.field(O.UZ))
+    nut = o.field(O.NUT)
+    o.call("Clc_SGS_Vis", *u, nut)
+    g.upload(L.NUT, nut)
+    o.call("PMcoeUpdate", 2)
+    g.PMcoeUpdate(2)
+    rx, ry = (np.zeros((nx, ny, nz), order="F") for _ in range(2))
+    rz = np.zeros((nx + 3, ny + 3, nz + 3), order="F")
+    o.call("clcRhsX_les", *u, rx, o.field(O.HISTX), o.field(O.PR), nut)
+    o.call("clcRhsY_les", *u, ry, o.field(O.HISTY), o.field(O.PR), nut)
+    o.call("clcRhsZ_les", *u, rz, o.field(O.HISTZ), o.field(O.PR), nut)
+    g.clcRhsX(L.UX, L.UY, L.UZ, L.ARR1, L.HISTX, L.PR)
+    g.clcRhsY(L.UX, L.UY, L.UZ, L.ARR2, L.HISTY, L.PR)
+    g.clcRhsZ(L.UX, L.UY, L.UZ, L.HALOARR, L.HISTZ, L.PR)
+    for gid, ref in ((L.ARR1, rx), (L.ARR2, ry), (L.HALOARR, rz), (L.HISTX, o.field(O.HISTX)),
+                     (L.HISTY, o.field(O.HISTY)), (L.HISTZ, o.field(O.HISTZ))):
+        got = g.download(gid)
+        if gid == L.HALOARR:
+            got, ref = P2.interior(got), P2.interior(ref)
+        assert np.abs(got - ref).max() == 0.0, gid
     g.close()
     o.close()
