@@ -480,124 +480,245 @@ __global__ __launch_bounds__(LBX* LBY, 2) void k_rhs_les(Geom g, Metrics<T> m, L
 // ---------------------------------------------------------------------------
 // clcU1Hat_PIMP_LES (:466-499), clcU2Hat_PIMP_LES (:626-662),
 // clcU3Hat_PIMP_LES (:776-809): per (i, k) line, InverseTridiagonal
-// (m_Tools.f90:218-245) with the coefficients of each row built from nut as
-// the sweep reaches it.  The forward pass keeps the modified right-hand side
-// in place and the elimination factors in `arr` (a field-shaped scratch);
-// the backward pass adds the solution to u.  ADDD adds dpmdxns to RhsX as it
-// is loaded (the constant-flow-rate shift of clcRhsX, :146-151).
+// (m_Tools.f90:218-245) with the coefficients of each row built from nut.
+// ADDD adds dpmdxns to RhsX as it is loaded (the constant-flow-rate shift of
+// clcRhsX, :146-151).
+//
+// The line is cut into segments of LC rows, as in the full-implicit sweep:
+// the forward pass keeps only each segment's last value and pivot (two words
+// per segment and line, in the scratch field), the backward pass forms a
+// segment's rows again from there (the same operations on the same operands,
+// so the same values), substitutes and updates u.  A segment's right-hand
+// side and nut rows are requested one segment ahead of the recurrence, in
+// unconditional loads (rows past the last are read from it and not used).
+// Traffic: the right-hand side and nut twice, u once, u written (7 words per
+// component before: the forward values and factors of every row went to memory
+// and back).  The metric rows are restrict arguments, so they come through
+// scalar loads: as vector loads among the prefetches, waiting for one would
+// wait for the prefetch before it.  The two quotients by a row's pivot share its reciprocal.
+// Storing sweeps that loaded row by row were bound by HBM on large grids and
+// by the loads' latency on small ones: the three took 0.896 ms at 384x192x288 and
+// 0.072 ms at 96x96x72 (FP64), these take 0.490 and 0.030 ms.
+// Lines are dealt flat over (i, k); the three components of a line's tile are
+// neighbouring workgroups on one XCD and share its nut rows in L2.
 // ---------------------------------------------------------------------------
-template <typename T, int COMP>
-__device__ __forceinline__ void les_row(const Geom& g, const LesMet<T>& lm, const Metrics<T>& m,
-                                        T bt, const T* __restrict__ nut, int i, int im, int j,
-                                        int k, int km, T& rt1, T& rt2) {
-  const int nx = g.nx, nyh = g.nyh;
-  if (COMP == 0) {
-    const T visc = T(0.25) * (A(nut, i, j, k) + A(nut, im, j, k) + A(nut, i, j - 1, k) + A(nut, im, j - 1, k));
-    const T visd = T(0.25) * (A(nut, i, j, k) + A(nut, im, j, k) + A(nut, i, j + 1, k) + A(nut, im, j + 1, k));
-    rt1 = bt * visc * lm.am2ccn[j];
-    rt2 = bt * visd * lm.ap2ccn[j];
-  } else if (COMP == 1) {
-    rt1 = bt * A(nut, i, j - 1, k) * m.am2p[j];
-    rt2 = bt * A(nut, i, j, k) * m.ap2p[j];
-  } else {
-    const T visc = T(0.25) * (A(nut, i, j, km) + A(nut, i, j - 1, km) + A(nut, i, j, k) + A(nut, i, j - 1, k));
-    const T visd = T(0.25) * (A(nut, i, j, km) + A(nut, i, j + 1, km) + A(nut, i, j, k) + A(nut, i, j + 1, k));
-    rt1 = bt * visc * lm.am2ccn[j];
-    rt2 = bt * visd * lm.ap2ccn[j];
-  }
-}
+constexpr int LC = 8;
 
-template <typename T, int COMP, bool ADDD>
-__device__ __forceinline__ void les_y_line(const Geom& g, const Metrics<T>& m, const LesMet<T>& lm,
-                                           T bt, const T* __restrict__ nut,
-                                           T* __restrict__ rhs, T* __restrict__ arr,
+template <typename T, int COMP, bool ADDD, bool NTS>
+__device__ __forceinline__ void les_y_line(const Geom& g, const T* __restrict__ am,
+                                           const T* __restrict__ ap, T bt,
+                                           const T* __restrict__ nut,
+                                           const T* __restrict__ rhs, T* __restrict__ ck,
                                            T* __restrict__ u, const T* __restrict__ duy,
-                                           const DevScalars* __restrict__ sc, int i, int k) {
-  const int ny = g.ny;
-  const int im = wm(i, g.nx), km = wm(k, g.nz);
+                                           const DevScalars* __restrict__ sc, long long line) {
+  const int nx = g.nx, ny = g.ny;
+  const int i = (int)(line % nx), k = (int)(line / nx);
+  const long long base = i + g.plane * k, nl = (long long)nx * g.nz;
+  const T* pr = rhs + base;
+  const T* pa = nut + base;
+  // the face neighbour of nut: one cell down in x (ux) or z (uz)
+  const T* pb = nut + (COMP == 0 ? wm(i, nx) + g.plane * k : i + g.plane * wm(k, g.nz));
+  T* pu = u + base;
+  T* pc = ck + line;
   const T dd = ADDD ? (T)sc->dpmdxns : T(0);
-  // row 1
-  T a, b, cprev, f;
-  if (COMP == 1) {
-    a = T(0); b = T(1); cprev = T(0);
-    f = duy[i + (long long)g.nx * k];
-  } else {
-    T rt1, rt2;
-    les_row<T, COMP>(g, lm, m, bt, nut, i, im, 1, k, km, rt1, rt2);
-    a = -rt1; b = rt1 + rt2 + T(1); cprev = -rt2;
-    f = rhs[fidx(g, i, 1, k)];
-    if (ADDD) f = f + dd;
+  const T wallv = COMP == 1 ? duy[line] : T(0);
+  const int nseg = (ny + LC - 1) / LC, top = nseg - 1;
+  struct Seg {
+    T r[LC], a[LC + 2], b[LC + 2];  // right-hand side; nut rows one below to one above
+  };
+  // Only the top segment has rows past the last (read from it, not used); the
+  // others run without the row clamp and guard, which is a branch of its own
+  // around every row.
+  using Gd = std::true_type;
+  using Un = std::false_type;
+  auto load = [&](Seg& y, int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+    const int lo = s * LC + 1;
+#pragma unroll
+    for (int q = 0; q < LC; ++q) y.r[q] = pr[(long long)nx * (G ? min(lo + q, ny) : lo + q)];
+#pragma unroll
+    for (int q = 0; q < LC + 2; ++q) {
+      const long long o = (long long)nx * (G ? min(lo - 1 + q, ny + 1) : lo - 1 + q);
+      y.a[q] = pa[o];
+      if (COMP != 1) y.b[q] = pb[o];
+    }
+  };
+  // the matrix row's coefficients: rt1 below, rt2 above
+  auto coef = [&](const Seg& y, int q, int j, T& rt1, T& rt2) {
+    if (COMP == 0) {
+      const T c = y.a[q + 1] + y.b[q + 1];
+      rt1 = bt * (T(0.25) * (c + y.a[q] + y.b[q])) * am[j];
+      rt2 = bt * (T(0.25) * (c + y.a[q + 2] + y.b[q + 2])) * ap[j];
+    } else if (COMP == 1) {
+      rt1 = bt * y.a[q] * am[j];
+      rt2 = bt * y.a[q + 1] * ap[j];
+    } else {
+      rt1 = bt * (T(0.25) * (y.b[q + 1] + y.b[q] + y.a[q + 1] + y.a[q])) * am[j];
+      rt2 = bt * (T(0.25) * (y.b[q + 1] + y.b[q + 2] + y.a[q + 1] + y.a[q + 2])) * ap[j];
+    }
+  };
+  T f = T(0), vecm = T(1), rv = T(1), cprev = T(0);  // rv: 1/vecm
+  T ar[LC];
+  // forward through segment s from (f, vecm, rv, cprev): values into y.r,
+  // factors into ar.  Row 1 has nothing below: f = 0, vecm = 1 and cprev = 0
+  // give its pivot b and value r/b.
+  auto fwd = [&](Seg& y, int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+    const int lo = s * LC + 1;
+#pragma unroll
+    for (int q = 0; q < LC; ++q) {
+      const int j = lo + q;
+      if (!G || j <= ny) {
+        T rt1, rt2, fj = ADDD ? y.r[q] + dd : y.r[q];
+        coef(y, q, j, rt1, rt2);
+        if (COMP == 1 && q == 0 && s == 0) {  // the wall row
+          rt1 = rt2 = T(0);
+          fj = wallv;
+        }
+        const T a = -rt1, b = rt1 + rt2 + T(1);
+        ar[q] = quot(cprev, vecm, rv);
+        vecm = b - a * ar[q];
+        rv = quot_recip(vecm);
+        f = quot(fj - a * f, vecm, rv);
+        cprev = -rt2;
+        y.r[q] = f;
+      }
+    }
+  };
+  auto save = [&](int s) {
+    pc[nl * (2 * s)] = f;
+    pc[nl * (2 * s + 1)] = vecm;
+  };
+  T x = T(0), arn = T(0);  // the solution and factor of the row above
+  // through segment s: u's words are requested before the next segment's, so
+  // waiting for them leaves that prefetch in flight
+  T uv[LC];
+  auto loadu = [&](int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+    const int lo = s * LC + 1;
+#pragma unroll
+    for (int q = 0; q < LC; ++q)
+      uv[q] = C3D_LD_ONCE(&pu[(long long)nx * (G ? min(lo + q, ny) : lo + q)]);
+  };
+  auto back = [&](const Seg& y, int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+    const int lo = s * LC + 1;
+#pragma unroll
+    for (int q = LC - 1; q >= 0; --q) {
+      const int j = lo + q;
+      if (!G || j <= ny) {
+        if (!G || j < ny) x = y.r[q] - (q + 1 < LC ? ar[q + 1] : arn) * x;
+        C3D_ST_ONCE(uv[q] + x, &pu[(long long)nx * j]);
+      }
+    }
+    arn = ar[0];
+  };
+  Seg ya, yb;
+  int s = 0;
+  if (top == 0) load(ya, 0, Gd{});
+  else load(ya, 0, Un{});
+  for (; s + 2 < top; s += 2) {
+    load(yb, s + 1, Un{});
+    __builtin_amdgcn_sched_barrier(0);
+    fwd(ya, s, Un{});
+    save(s);
+    load(ya, s + 2, Un{});
+    __builtin_amdgcn_sched_barrier(0);
+    fwd(yb, s + 1, Un{});
+    save(s + 1);
   }
-  T vecm = b;
-  f = f / vecm;
-  rhs[fidx(g, i, 1, k)] = f;
-  T fprev = f;
-  for (int j = 2; j <= ny; ++j) {
-    T rt1, rt2;
-    les_row<T, COMP>(g, lm, m, bt, nut, i, im, j, k, km, rt1, rt2);
-    a = -rt1; b = rt1 + rt2 + T(1);
-    const long long q = fidx(g, i, j, k);
-    T fj = rhs[q];
-    if (ADDD) fj = fj + dd;
-    const T r = cprev / vecm;
-    arr[q] = r;
-    vecm = b - a * r;
-    fj = (fj - a * fprev) / vecm;
-    rhs[q] = fj;
-    fprev = fj;
-    cprev = -rt2;
+  if (s + 2 == top) {
+    load(yb, s + 1, Un{});
+    __builtin_amdgcn_sched_barrier(0);
+    fwd(ya, s, Un{});
+    save(s);
+    load(ya, top, Gd{});
+    __builtin_amdgcn_sched_barrier(0);
+    fwd(yb, s + 1, Un{});
+    save(s + 1);
+  } else if (s + 1 == top) {
+    load(yb, top, Gd{});
+    __builtin_amdgcn_sched_barrier(0);
+    fwd(ya, s, Un{});
+    save(s);
+    ya = yb;
   }
-  // back substitution, u += f
-  T fnext = fprev;
-  {
-    const long long q = fidx(g, i, ny, k);
-    u[q] = u[q] + fnext;
-  }
-  for (int j = ny - 1; j >= 1; --j) {
-    const long long q = fidx(g, i, j, k);
-    const T fj = rhs[q] - arr[q + g.nx] * fnext;
-    u[q] = u[q] + fj;
-    fnext = fj;
+  fwd(ya, top, Gd{});
+  x = f;
+  loadu(top, Gd{});
+  if (top > 0) load(yb, top - 1, Un{});
+  __builtin_amdgcn_sched_barrier(0);
+  back(ya, top, Gd{});
+  for (s = top - 1; s >= 0; --s) {
+    ya = yb;
+    loadu(s, Un{});
+    f = T(0);
+    vecm = rv = T(1);
+    cprev = T(0);
+    if (s > 0) {
+      f = pc[nl * (2 * s - 2)];
+      vecm = pc[nl * (2 * s - 1)];
+      load(yb, s - 1, Un{});
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (s > 0) {
+      rv = quot_recip(vecm);
+      // the row below the segment's first: its upper coefficient
+      const int j = s * LC;
+      T rt2;
+      if (COMP == 0)
+        rt2 = bt * (T(0.25) * (ya.a[0] + ya.b[0] + ya.a[1] + ya.b[1])) * ap[j];
+      else if (COMP == 1)
+        rt2 = bt * ya.a[0] * ap[j];
+      else
+        rt2 = bt * (T(0.25) * (ya.b[0] + ya.b[1] + ya.a[0] + ya.a[1])) * ap[j];
+      cprev = -rt2;
+    }
+    fwd(ya, s, Un{});
+    back(ya, s, Un{});
   }
 }
 
-template <typename T, int COMP, bool ADDD>
-__global__ __launch_bounds__(64) void k_les_y(Geom g, Metrics<T> m, LesMet<T> lm, T bt,
-                                              const T* __restrict__ nut, T* __restrict__ rhs,
-                                              T* __restrict__ arr, T* __restrict__ u,
-                                              const T* __restrict__ duy,
+template <typename T, int COMP, bool ADDD, bool NTS>
+__global__ __launch_bounds__(64) void k_les_y(Geom g, const T* __restrict__ am,
+                                              const T* __restrict__ ap, T bt,
+                                              const T* __restrict__ nut,
+                                              const T* __restrict__ rhs, T* __restrict__ ck,
+                                              T* __restrict__ u, const T* __restrict__ duy,
                                               const DevScalars* __restrict__ sc) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  if (i >= g.nx) return;
-  les_y_line<T, COMP, ADDD>(g, m, lm, bt, nut, rhs, arr, u, duy, sc, i, blockIdx.y);
+  const long long line = (long long)blockIdx.x * 64 + threadIdx.x;
+  if (line >= (long long)g.nx * g.nz) return;
+  les_y_line<T, COMP, ADDD, NTS>(g, am, ap, bt, nut, rhs, ck, u, duy, sc, line);
 }
 
-// The three component solves of one LES substep in one launch: blockIdx.z is
-// the component, each with its own velocity, right-hand side and elimination
-// scratch. The solves are independent (each reads only nut and its own
-// arrays), and a single component's launch fills few CUs on small grids, so
-// three sequential launches would each wait out one line's serial sweep.
+// The three component solves of one LES substep in one launch, component
+// fastest, each with its own velocity, right-hand side and checkpoint scratch.
+// The solves are independent (each reads only nut and its own arrays).
 template <typename T>
 struct LesY3 {
   T* u[3];
-  T* rhs[3];
-  T* arr[3];
+  const T* rhs[3];
+  T* ck[3];
   const T* duy;
 };
 
-template <typename T, bool ADDD>
-__global__ __launch_bounds__(64) void k_les_y3(Geom g, Metrics<T> m, LesMet<T> lm, T bt,
+template <typename T, bool ADDD, bool NTS>
+__global__ __launch_bounds__(64) void k_les_y3(Geom g, const T* __restrict__ amc,
+                                               const T* __restrict__ apc,
+                                               const T* __restrict__ amp,
+                                               const T* __restrict__ app, T bt,
                                                const T* __restrict__ nut, LesY3<T> a,
                                                const DevScalars* __restrict__ sc) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  if (i >= g.nx) return;
-  const int k = blockIdx.y;
-  if (blockIdx.z == 0)
-    les_y_line<T, 0, ADDD>(g, m, lm, bt, nut, a.rhs[0], a.arr[0], a.u[0], nullptr, sc, i, k);
-  else if (blockIdx.z == 1)
-    les_y_line<T, 1, false>(g, m, lm, bt, nut, a.rhs[1], a.arr[1], a.u[1], a.duy, sc, i, k);
+  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int comp = lb % 3;
+  const long long line = (long long)(lb / 3) * 64 + threadIdx.x;
+  if (line >= (long long)g.nx * g.nz) return;
+  if (comp == 0)
+    les_y_line<T, 0, ADDD, NTS>(g, amc, apc, bt, nut, a.rhs[0], a.ck[0], a.u[0], nullptr, sc, line);
+  else if (comp == 1)
+    les_y_line<T, 1, false, NTS>(g, amp, app, bt, nut, a.rhs[1], a.ck[1], a.u[1], a.duy, sc, line);
   else
-    les_y_line<T, 2, false>(g, m, lm, bt, nut, a.rhs[2], a.arr[2], a.u[2], nullptr, sc, i, k);
+    les_y_line<T, 2, false, NTS>(g, amc, apc, bt, nut, a.rhs[2], a.ck[2], a.u[2], nullptr, sc, line);
 }
 
 // ---------------------------------------------------------------------------
@@ -717,19 +838,28 @@ int launch_rhs_les(c3d_ctx* c, int mask, const void* ux, const void* uy, const v
 }
 
 template <typename T>
-static int les_y_t(c3d_ctx* c, int comp, void* u, void* rhs, const void* duy, int addd) {
+static int les_y_t(c3d_ctx* c, int comp, void* u, const void* rhs, const void* duy, int addd) {
   const Geom& g = c->g;
-  dim3 grid((g.nx + 63) / 64, g.nz), blk(64);
+  const dim3 grid((unsigned)(((long long)g.nx * g.nz + 63) / 64)), blk(64);
   const T bt = (T)c->pmBetaT;
   const T* nut = (const T*)c->state[C3D_NUT];
-#define LY(C, D)                                                                                 \
-  hipLaunchKernelGGL((k_les_y<T, C, D>), grid, blk, 0, c->stream, g, met<T>(c), lesmet<T>(c), bt, \
-                     nut, (T*)rhs, (T*)c->tmpA, (T*)u, (const T*)duy, (const DevScalars*)c->d_sc)
-  if (comp == 0 && addd) LY(0, true);
-  else if (comp == 0) LY(0, false);
-  else if (comp == 1) LY(1, false);
-  else LY(2, false);
-#undef LY
+  auto launch = [&](auto cc, auto dc, auto ntc) {
+    hipLaunchKernelGGL(
+        (k_les_y<T, decltype(cc)::value, decltype(dc)::value, decltype(ntc)::value>), grid, blk, 0,
+        c->stream, g, comp == 1 ? met<T>(c).am2p : lesmet<T>(c).am2ccn,
+        comp == 1 ? met<T>(c).ap2p : lesmet<T>(c).ap2ccn, bt, nut, (const T*)rhs, (T*)c->tmpA,
+        (T*)u, (const T*)duy, (const DevScalars*)c->d_sc);
+  };
+  using Yes = std::true_type;
+  using No = std::false_type;
+  auto by_nt = [&](auto cc, auto dc) {
+    if (g.nt) launch(cc, dc, Yes{});
+    else launch(cc, dc, No{});
+  };
+  if (comp == 0 && addd) by_nt(std::integral_constant<int, 0>{}, Yes{});
+  else if (comp == 0) by_nt(std::integral_constant<int, 0>{}, No{});
+  else if (comp == 1) by_nt(std::integral_constant<int, 1>{}, No{});
+  else by_nt(std::integral_constant<int, 2>{}, No{});
   C3D_HIP(hipGetLastError());
   return C3D_OK;
 }
@@ -753,22 +883,28 @@ template <typename T>
 static int les_y3_t(c3d_ctx* c, void* const u[3], void* const rhs[3], const void* duy, int addd) {
   const Geom& g = c->g;
   LesY3<T> a;
-  void* const arr[3] = {c->tmpA, c->les_arr[0], c->les_arr[1]};
+  void* const ck[3] = {c->tmpA, c->les_arr[0], c->les_arr[1]};
   for (int d = 0; d < 3; ++d) {
     a.u[d] = (T*)u[d];
-    a.rhs[d] = (T*)rhs[d];
-    a.arr[d] = (T*)arr[d];
+    a.rhs[d] = (const T*)rhs[d];
+    a.ck[d] = (T*)ck[d];
   }
   a.duy = (const T*)duy;
-  dim3 grid((g.nx + 63) / 64, g.nz, 3), blk(64);
+  const dim3 grid((unsigned)(3 * (((long long)g.nx * g.nz + 63) / 64))), blk(64);
   const T bt = (T)c->pmBetaT;
   const T* nut = (const T*)c->state[C3D_NUT];
-  if (addd)
-    hipLaunchKernelGGL((k_les_y3<T, true>), grid, blk, 0, c->stream, g, met<T>(c), lesmet<T>(c),
-                       bt, nut, a, (const DevScalars*)c->d_sc);
-  else
-    hipLaunchKernelGGL((k_les_y3<T, false>), grid, blk, 0, c->stream, g, met<T>(c), lesmet<T>(c),
-                       bt, nut, a, (const DevScalars*)c->d_sc);
+  auto launch = [&](auto dc, auto ntc) {
+    hipLaunchKernelGGL((k_les_y3<T, decltype(dc)::value, decltype(ntc)::value>), grid, blk, 0,
+                       c->stream, g, lesmet<T>(c).am2ccn, lesmet<T>(c).ap2ccn, met<T>(c).am2p,
+                       met<T>(c).ap2p, bt, nut, a, (const DevScalars*)c->d_sc);
+  };
+  if (addd) {
+    if (g.nt) launch(std::true_type{}, std::true_type{});
+    else launch(std::true_type{}, std::false_type{});
+  } else {
+    if (g.nt) launch(std::false_type{}, std::true_type{});
+    else launch(std::false_type{}, std::false_type{});
+  }
   C3D_HIP(hipGetLastError());
   return C3D_OK;
 }
