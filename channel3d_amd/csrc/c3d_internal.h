@@ -102,8 +102,14 @@ __device__ __forceinline__ double quot(double a, double v, double r) {
   const double q = a * r;
   return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-v, q, a), r, q), v, a);
 }
-__device__ __forceinline__ float quot_recip(float) { return 0.f; }
-__device__ __forceinline__ float quot(float a, float v, float) { return a / v; }
+__device__ __forceinline__ float quot_recip(float v) {
+  const float r = __builtin_amdgcn_rcpf(v);  // within an ulp: one step suffices
+  return __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
+}
+__device__ __forceinline__ float quot(float a, float v, float r) {
+  const float q = a * r;
+  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-v, q, a), r, q), v, a);
+}
 
 // Reproducible sums.  Each double term is truncated to a multiple of 2^-80
 // and split into four signed 32-bit limbs accumulated in int64: integer
@@ -264,8 +270,8 @@ struct c3d_ctx {
   void* d_tabs = nullptr;
   // y solver (YS_*): checkpointed sweeps, or the sweeps storing the forward pass
   int ymode = 0;
-  // lanes per wavenumber pair of the checkpointed PPE sweep: 0 by the line
-  // count, 1 or 2 forced (tests of both forms)
+  // lanes per wavenumber pair of the checkpointed PPE sweep: 2 (or 0), 1 forced
+  // for tests of both forms
   int tri_lanes = 0;
   int y_threads = 0;  // lines per workgroup of the checkpointed y sweep (0: by grid size)
   int z_tile = 0;     // kx lines per workgroup of the z transform (0: 8)

@@ -27,8 +27,7 @@ struct CT2<float> { using t = float2; };
 // than a power of two or a multiple of 64 on most grids: with 64 threads per
 // kz row, a row's last wavefront held one live thread (512x256x512: 320
 // threads for 257 lines).  The two-lane sweep of 192x128x160 (97 lines a row)
-// takes 0.051 ms instead of 0.064; the memory-bound one-lane sweeps of large
-// grids are unchanged (512x256x512 x 4: 1.64 ms either way).
+// took 0.051 ms instead of 0.064 for it.
 struct Line {
   int kx, kz;
 };
@@ -39,8 +38,18 @@ __device__ __forceinline__ Line line_of(const Geom& g, long long l) {
   return r;
 }
 
+// The rows of the wall-normal operator and the wavenumber terms, as restrict
+// arguments of their own: a sweep's row coefficients are the same for every
+// lane, and the compiler loads them through the scalar unit only where no
+// store can alias them.  As vector loads (from a struct of pointers) they
+// queue behind the prefetched segment, and waiting for one drains it.
+#define PprRows(T)                                                                      \
+  const T *__restrict__ am, const T *__restrict__ ac, const T *__restrict__ ap,         \
+      const T *__restrict__ wx, const T *__restrict__ wz
+#define PPR_OF(m) (m).am2Pr, (m).ac2Pr, (m).ap2Pr, (m).wavex, (m).wavez
+
 template <typename T>
-__device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& m,
+__device__ __forceinline__ void k_tridiag_body(const Geom& g, PprRows(T),
                                                typename CT2<T>::t* __restrict__ spec,
                                                T* __restrict__ sarr, Line ln) {
   using T2 = typename CT2<T>::t;
@@ -49,11 +58,12 @@ __device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& 
   const int ny = g.ny;
   const long long P = g.P;
   const long long base = kx + P * (long long)ny * kz;
-  const T lx = m.wavex[kx], lz = m.wavez[kz];
+  const T lx = wx[kx], lz = wz[kz];
   const bool pin = (kx == 0 && kz == 0);
   // row j = 1
-  T vecm = pin ? T(1) : (m.ac2Pr[1] + lx) + lz;
-  T cprev = pin ? T(0) : m.ap2Pr[1];
+  T vecm = pin ? T(1) : (ac[1] + lx) + lz;
+  T rv = quot_recip(vecm);
+  T cprev = pin ? T(0) : ap[1];
   // register rings keep the next PD rows of each sweep in flight; the main
   // loops carry no conditionals so the loads stay outstanding across steps
   constexpr int PD = 8;
@@ -65,18 +75,19 @@ __device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& 
     f.x = 0;
     f.y = 0;
   }
-  f.x = f.x / vecm;
-  f.y = f.y / vecm;
+  f.x = quot(f.x, vecm, rv);
+  f.y = quot(f.y, vecm, rv);
   spec[base] = f;
   auto fwd = [&](int j0, T2 fj) {
     const int jr = j0 + 1;
-    const T arr = cprev / vecm;
-    const T a = m.am2Pr[jr];
-    vecm = ((m.ac2Pr[jr] + lx) + lz) - a * arr;
-    f.x = (fj.x - a * f.x) / vecm;
-    f.y = (fj.y - a * f.y) / vecm;
+    const T arr = quot(cprev, vecm, rv);
+    const T a = am[jr];
+    vecm = ((ac[jr] + lx) + lz) - a * arr;
+    rv = quot_recip(vecm);
+    f.x = quot(fj.x - a * f.x, vecm, rv);
+    f.y = quot(fj.y - a * f.y, vecm, rv);
     sarr[base + P * j0] = arr;
-    cprev = m.ap2Pr[jr];
+    cprev = ap[jr];
   };
   int jb = 1;
   for (; jb + 2 * PD <= ny - 1; jb += PD) {
@@ -154,7 +165,7 @@ __device__ __forceinline__ void k_tridiag_body(const Geom& g, const Metrics<T>& 
 // results equal k_tridiag's bit for bit.
 // ---------------------------------------------------------------------------
 template <typename T, int C, bool NTS = false>
-__device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, const Metrics<T>& m,
+__device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, PprRows(T),
                                                   typename CT2<T>::t* __restrict__ spec,
                                                   T* __restrict__ ckp, Line ln) {
   using T2 = typename CT2<T>::t;
@@ -166,79 +177,59 @@ __device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, const Metrics<T
   const long long base = kx + P * (long long)ny * kz;
   const long long cs = P * (long long)g.nz;             // checkpoint plane stride
   T* ck = ckp + kx + P * (long long)kz;
-  const T lx = m.wavex[kx], lz = m.wavez[kz];
+  const T lx = wx[kx], lz = wz[kz];
   const bool pin = (kx == 0 && kz == 0);
+  using Gd = std::true_type;   // the top segment: rows past the last one
+  using Un = std::false_type;  // the others, without the row guard
   T2 y[C];
   T ar[C];
-  T vecm = T(1), cprev = T(0);
+  T vecm = T(1), rv = T(1), cprev = T(0);  // rv: 1/vecm
   T2 f;
   f.x = 0;
   f.y = 0;
-  // one segment's forward recurrence from (f, vecm, cprev); rows lo..lo+C-1
-  auto run = [&](int lo) {
+  auto load = [&](int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+#pragma unroll
+    for (int q = 0; q < C; ++q)
+      if (!G || s * C + q < ny) y[q] = spec[base + P * (s * C + q)];
+  };
+  // one segment's forward recurrence from (f, vecm, rv, cprev).  Row 1 has
+  // nothing below: f = 0, vecm = 1 and cprev = 0 give its pivot and value.
+  auto run = [&](int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
-      const int j0 = lo + q;
-      if (j0 < ny) {
-        if (j0 == 0) {
-          vecm = pin ? T(1) : (m.ac2Pr[1] + lx) + lz;
-          cprev = pin ? T(0) : m.ap2Pr[1];
-          T2 fj = y[q];
-          if (pin) {
-            fj.x = 0;
-            fj.y = 0;
-          }
-          f.x = fj.x / vecm;
-          f.y = fj.y / vecm;
-          ar[q] = T(0);
-        } else {
-          const int jr = j0 + 1;
-          const T arr = cprev / vecm;
-          const T a = m.am2Pr[jr];
-          vecm = ((m.ac2Pr[jr] + lx) + lz) - a * arr;
-          f.x = (y[q].x - a * f.x) / vecm;
-          f.y = (y[q].y - a * f.y) / vecm;
-          cprev = m.ap2Pr[jr];
-          ar[q] = arr;
+      const int j0 = s * C + q;
+      if (!G || j0 < ny) {
+        const int jr = j0 + 1;
+        const T arr = quot(cprev, vecm, rv);
+        const T a = am[jr];
+        T2 fj = y[q];
+        T cj = ap[jr];
+        vecm = ((ac[jr] + lx) + lz) - a * arr;
+        if (q == 0 && s == 0 && pin) {  // the gauge row
+          vecm = T(1);
+          fj.x = fj.y = cj = T(0);
         }
+        rv = quot_recip(vecm);
+        f.x = quot(fj.x - a * f.x, vecm, rv);
+        f.y = quot(fj.y - a * f.y, vecm, rv);
+        cprev = cj;
+        ar[q] = arr;
         y[q] = f;
       }
     }
   };
-  for (int s = 0; s < nseg; ++s) {
-    const int lo = s * C;
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-      if (lo + q < ny) y[q] = spec[base + P * (lo + q)];
-    }
-    run(lo);
-    if (s + 1 < nseg) {
-      ck[cs * (3 * s + 0)] = f.x;
-      ck[cs * (3 * s + 1)] = f.y;
-      ck[cs * (3 * s + 2)] = vecm;
-    }
-  }
-  // backward; y and ar hold the top segment
-  T2 x = f;
+  // backward through segment s (forward values in y)
+  T2 x;
   T arnext = T(0);
-  for (int s = nseg - 1; s >= 0; --s) {
-    const int lo = s * C;
-    if (s < nseg - 1) {
-#pragma unroll
-      for (int q = 0; q < C; ++q) y[q] = spec[base + P * (lo + q)];  // full segment
-      if (s > 0) {
-        f.x = ck[cs * (3 * (s - 1) + 0)];
-        f.y = ck[cs * (3 * (s - 1) + 1)];
-        vecm = ck[cs * (3 * (s - 1) + 2)];
-        cprev = m.ap2Pr[lo];
-      }
-      run(lo);
-    }
+  auto back = [&](int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
 #pragma unroll
     for (int q = C - 1; q >= 0; --q) {
-      const int j0 = lo + q;
-      if (j0 < ny) {
-        if (j0 < ny - 1) {
+      const int j0 = s * C + q;
+      if (!G || j0 < ny) {
+        if (!G || j0 < ny - 1) {
           const T a1 = q + 1 < C ? ar[q + 1] : arnext;
           x.x = y[q].x - a1 * x.x;
           x.y = y[q].y - a1 * x.y;
@@ -248,6 +239,34 @@ __device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, const Metrics<T
       }
     }
     arnext = ar[0];
+  };
+  const int top = nseg - 1;
+  for (int s = 0; s < top; ++s) {
+    load(s, Un{});
+    run(s, Un{});
+    ck[cs * (3 * s + 0)] = f.x;
+    ck[cs * (3 * s + 1)] = f.y;
+    ck[cs * (3 * s + 2)] = vecm;
+  }
+  load(top, Gd{});
+  run(top, Gd{});
+  x = f;
+  back(top, Gd{});
+  for (int s = top - 1; s >= 0; --s) {
+    f.x = f.y = T(0);
+    vecm = rv = T(1);
+    cprev = T(0);
+    if (s > 0) {
+      f.x = ck[cs * (3 * (s - 1) + 0)];
+      f.y = ck[cs * (3 * (s - 1) + 1)];
+      vecm = ck[cs * (3 * (s - 1) + 2)];
+      cprev = ap[s * C];
+    }
+    load(s, Un{});
+    __builtin_amdgcn_sched_barrier(0);
+    if (s > 0) rv = quot_recip(vecm);
+    run(s, Un{});
+    back(s, Un{});
   }
 }
 
@@ -255,18 +274,22 @@ __device__ __forceinline__ void k_tridiag_ck_body(const Geom& g, const Metrics<T
 // pair on two neighbouring lanes (lane 2n the real part, 2n+1 the
 // imaginary part), both computing the shared pivots -- the same operations,
 // so the same values -- and with each segment's right-hand side loaded one
-// segment ahead.  Twice the lanes of k_tridiag_ck_body for the same lines:
-// for grids whose line count fills only a fraction of the device (at
-// 192x160 or 96x72 a lane per pair leaves most SIMDs without a wavefront).
+// segment ahead.  Half the registers per lane of k_tridiag_ck_body: twice the
+// wavefronts on grids with few lines, room for the prefetch and for longer
+// segments on large ones.  The three quotients by a pivot share its
+// reciprocal.  Before (vector loads of the row coefficients, a guard around
+// every row, divisions; one lane on large grids) and now, FP64: four
+// 512x256x512 fields 1.640 -> 1.241 ms, 768x384x576 0.986 -> 0.903 ms,
+// 192x128x160 0.051 -> 0.040 ms, 96x96x72 0.031 -> 0.025 ms, 64^3 0.023 ->
+// 0.017 ms.
 // Only the top segment has rows past ny, so only its loads and stores carry
 // the row guard (a guarded access is a branch of its own, and the compiler
 // then waits for every outstanding load, the prefetched segment included).
 template <typename T, int C, bool NTS = false>
-__device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<T>& m,
+__device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, PprRows(T),
                                                    typename CT2<T>::t* __restrict__ spec,
-                                                   T* __restrict__ ckp) {
+                                                   T* __restrict__ ckp, Line ln) {
   const int part = threadIdx.x & 1;  // 0: real, 1: imaginary part
-  const Line ln = line_of(g, ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 1);
   const int kx = ln.kx, kz = ln.kz;
   if (kz >= g.nz) return;
   const int ny = g.ny;
@@ -277,7 +300,7 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
   const long long P2 = 2 * P;
   const long long cs = P * (long long)g.nz;  // checkpoint plane stride
   T* ck = ckp + kx + P * (long long)kz;
-  const T lx = m.wavex[kx], lz = m.wavez[kz];
+  const T lx = wx[kx], lz = wz[kz];
   const bool pin = (kx == 0 && kz == 0);
   using Gd = std::true_type;
   using Un = std::false_type;
@@ -289,29 +312,29 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
       if (!G || lo + q < ny) y[q] = sp[P2 * (lo + q)];
   };
   T ar[C];
-  T vecm = T(1), cprev = T(0), f = T(0);
-  // one segment's forward recurrence from (f, vecm, cprev); rows lo..lo+C-1
-  auto run = [&](T* y, int lo, auto gv) {
+  T vecm = T(1), rv = T(1), cprev = T(0), f = T(0);  // rv: 1/vecm
+  // one segment's forward recurrence from (f, vecm, rv, cprev).  Row 1 has
+  // nothing below: f = 0, vecm = 1 and cprev = 0 give its pivot and value.
+  auto run = [&](T* y, int s, auto gv) {
     constexpr bool G = decltype(gv)::value;
+    const int lo = s * C;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       const int j0 = lo + q;
       if (!G || j0 < ny) {
-        if (j0 == 0) {
-          vecm = pin ? T(1) : (m.ac2Pr[1] + lx) + lz;
-          cprev = pin ? T(0) : m.ap2Pr[1];
-          const T fj = pin ? T(0) : y[q];
-          f = fj / vecm;
-          ar[q] = T(0);
-        } else {
-          const int jr = j0 + 1;
-          const T arr = cprev / vecm;
-          const T a = m.am2Pr[jr];
-          vecm = ((m.ac2Pr[jr] + lx) + lz) - a * arr;
-          f = (y[q] - a * f) / vecm;
-          cprev = m.ap2Pr[jr];
-          ar[q] = arr;
+        const int jr = j0 + 1;
+        const T arr = quot(cprev, vecm, rv);
+        const T a = am[jr];
+        T fj = y[q], cj = ap[jr];
+        vecm = ((ac[jr] + lx) + lz) - a * arr;
+        if (q == 0 && s == 0 && pin) {  // the gauge row
+          vecm = T(1);
+          fj = cj = T(0);
         }
+        rv = quot_recip(vecm);
+        f = quot(fj - a * f, vecm, rv);
+        cprev = cj;
+        ar[q] = arr;
         y[q] = f;
       }
     }
@@ -329,7 +352,7 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
     for (int q = C - 1; q >= 0; --q) {
       const int j0 = lo + q;
       if (!G || j0 < ny) {
-        if (j0 < ny - 1) {
+        if (!G || j0 < ny - 1) {
           const T a1 = q + 1 < C ? ar[q + 1] : arnext;
           x = y[q] - a1 * x;
         }
@@ -348,25 +371,30 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
     int s = 0;
     for (; s + 2 < top; s += 2) {
       load(yb, s + 1, Un{});
-      run(ya, s * C, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
       save(s);
       load(ya, s + 2, Un{});
-      run(yb, (s + 1) * C, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(yb, s + 1, Un{});
       save(s + 1);
     }
     if (s + 1 < top) {
       load(yb, s + 1, Un{});
-      run(ya, s * C, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
       save(s);
       load(ya, top, Gd{});
-      run(yb, (s + 1) * C, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(yb, s + 1, Un{});
       save(s + 1);
-      run(ya, top * C, Gd{});
+      run(ya, top, Gd{});
     } else {
       load(yb, top, Gd{});
-      run(ya, s * C, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
       save(s);
-      run(yb, top * C, Gd{});
+      run(yb, top, Gd{});
 #pragma unroll
       for (int q = 0; q < C; ++q) ya[q] = yb[q];
     }
@@ -374,16 +402,23 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
   // backward; ya and ar hold the top segment
   x = f;
   if (top > 0) load(yb, top - 1, Un{});
+  __builtin_amdgcn_sched_barrier(0);
   back(ya, top, Gd{});
   for (int s = top - 1; s >= 0; --s) {
-    // yb holds segment s as stored; the segment below goes into ya
-    if (s > 0) load(ya, s - 1, Un{});
+    // yb holds segment s as stored; its checkpoint is requested before the
+    // segment below, which goes into ya
+    f = T(0);
+    vecm = rv = T(1);
+    cprev = T(0);
     if (s > 0) {
       f = ck[cs * (3 * (s - 1) + part)];
       vecm = ck[cs * (3 * (s - 1) + 2)];
-      cprev = m.ap2Pr[s * C];
+      load(ya, s - 1, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      rv = quot_recip(vecm);
+      cprev = ap[s * C];
     }
-    run(yb, s * C, Un{});
+    run(yb, s, Un{});
     back(yb, s, Un{});
 #pragma unroll
     for (int q = 0; q < C; ++q) yb[q] = ya[q];
@@ -391,70 +426,78 @@ __device__ __forceinline__ void k_tridiag_ck2_body(const Geom& g, const Metrics<
 }
 
 template <typename T, int C, bool NTS = false>
-__global__ __launch_bounds__(256) void k_tridiag_ck2(Geom g, Metrics<T> m,
+__global__ __launch_bounds__(256) void k_tridiag_ck2(Geom g, PprRows(T),
                                                      typename CT2<T>::t* __restrict__ spec,
                                                      T* __restrict__ ckp, long long bsp,
                                                      long long bck) {
-  k_tridiag_ck2_body<T, C, NTS>(g, m, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y);
+  k_tridiag_ck2_body<T, C, NTS>(g, am, ac, ap, wx, wz, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y,
+                                line_of(g, ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 1));
 }
 
-// At least 4 waves per SIMD: the FP64 body fits 128 VGPRs without spilling
-// (136 unconstrained, 3 waves), and at 768x384x576 the 1008 workgroups then
-// run in one round instead of 1.3 -- 0.99 ms per solve instead of 1.21 ms.
+// The one-lane form, which C3D_TRIDIAG_LANES=1 selects to compare with.  At
+// least 4 waves per SIMD: the FP64 body fits 128 VGPRs without spilling.
 // Batches: blockIdx.y selects the field; its spectrum starts bsp complex
 // elements, its checkpoints bck reals after the first field's.
 template <typename T, int C, bool NTS = false>
-__global__ __launch_bounds__(256, 4) void k_tridiag_ck(Geom g, Metrics<T> m,
+__global__ __launch_bounds__(256, 4) void k_tridiag_ck(Geom g, PprRows(T),
                                                     typename CT2<T>::t* __restrict__ spec,
                                                     T* __restrict__ ckp, long long bsp,
                                                     long long bck) {
-  k_tridiag_ck_body<T, C, NTS>(g, m, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y,
+  k_tridiag_ck_body<T, C, NTS>(g, am, ac, ap, wx, wz, spec + bsp * blockIdx.y, ckp + bck * blockIdx.y,
                                line_of(g, (long long)blockIdx.x * 256 + threadIdx.x));
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void k_tridiag_b(Geom g, Metrics<T> m,
+__global__ __launch_bounds__(256) void k_tridiag_b(Geom g, PprRows(T),
                                                    typename CT2<T>::t* __restrict__ spec,
                                                    T* __restrict__ sarr, long long bsp,
                                                    long long bck) {
-  k_tridiag_body<T>(g, m, spec + bsp * blockIdx.y, sarr + bck * blockIdx.y,
+  k_tridiag_body<T>(g, am, ac, ap, wx, wz, spec + bsp * blockIdx.y, sarr + bck * blockIdx.y,
                     line_of(g, (long long)blockIdx.x * 256 + threadIdx.x));
+}
+
+// Rows per segment of the two-lane sweep on large grids.  A segment costs three
+// checkpoint words per line, written and read (9 % of the traffic at 16 FP64
+// rows), its rows the registers.  FP64 (256-thread workgroups) 16 / 20 / 24 / 32
+// rows: 1.361 / 1.295 / 1.241 / 1.487 ms for four 512x256x512 fields and 1.004
+// / 0.904 / 0.903 / 0.946 ms at 768x384x576; the one-lane form takes 1.58 and
+// 1.08 ms on the same box.  FP32 16 / 24 / 32 / 48 rows: 0.402 / 0.387 / 0.368 /
+// 0.398 ms for two 512x256x512 fields.
+template <typename T>
+constexpr int tri_rows() {
+  return sizeof(T) == 8 ? 24 : 32;
 }
 
 template <typename T>
 static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
   const Geom& g = c->g;
   const long long nl = (long long)(g.nk + 1) * g.nz;  // lines of one field
-  const dim3 grid((unsigned)((nl + 255) / 256), b.n), blk(256);
   const Metrics<T>& m = *(const Metrics<T>*)(c->prec == C3D_FP64 ? (const void*)&c->md
                                                                   : (const void*)&c->mf);
   constexpr int CSEG = 16;
+  auto launch = [&](auto kern, int threads, int lanes) {
+    const dim3 grid((unsigned)((nl * lanes + threads - 1) / threads), b.n), blk(threads);
+    hipLaunchKernelGGL(kern, grid, blk, 0, c->stream, g, PPR_OF(m), (typename CT2<T>::t*)spec,
+                       (T*)ck, b.spec, b.ck);
+  };
   // checkpoints: 3 reals per line and segment, in the spectral scratch
   const long long need = 3LL * ((g.ny + CSEG - 1) / CSEG) * g.P * g.nz;
-  // two lanes per wavenumber pair where a lane per pair leaves the SIMDs
-  // short of wavefronts (fewer than two per SIMD of the 256-CU device)
-  const bool two = c->tri_lanes ? c->tri_lanes == 2 : nl * b.n * 2 <= 2048LL * 64;
-  if (c->ymode != YS_STORE && need <= (long long)g.P * g.ny * g.nz && two) {
-    // one wavefront (32 wavenumber pairs) per workgroup: the grids that take
-    // this form have few lines, and single-wave workgroups spread them over
-    // more CUs
-    const dim3 grid2((unsigned)((nl + 31) / 32), b.n), blk2(64);
-    if (g.nt)
-      hipLaunchKernelGGL((k_tridiag_ck2<T, CSEG, true>), grid2, blk2, 0, c->stream, g, m,
-                         (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
-    else
-      hipLaunchKernelGGL((k_tridiag_ck2<T, CSEG, false>), grid2, blk2, 0, c->stream, g, m,
-                         (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
-  } else if (c->ymode != YS_STORE && need <= (long long)g.P * g.ny * g.nz) {
-    if (g.nt)
-      hipLaunchKernelGGL((k_tridiag_ck<T, CSEG, true>), grid, blk, 0, c->stream, g, m,
-                         (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
-    else
-      hipLaunchKernelGGL((k_tridiag_ck<T, CSEG, false>), grid, blk, 0, c->stream, g, m,
-                         (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
+  if (c->ymode == YS_STORE || need > (long long)g.P * g.ny * g.nz) {
+    launch(k_tridiag_b<T>, 256, 1);
+  } else if (c->tri_lanes == 1) {
+    if (g.nt) launch(k_tridiag_ck<T, CSEG, true>, 256, 1);
+    else launch(k_tridiag_ck<T, CSEG, false>, 256, 1);
+  } else if (nl * b.n * 2 <= 1024LL * 64) {
+    // at most a wavefront per SIMD: the lines' serial chains bound the sweep,
+    // and single-wave workgroups of 16-row segments spread them over the most
+    // CUs (192x128x160: 0.040 ms against 0.043, 64^3: 0.017 against 0.022)
+    if (g.nt) launch(k_tridiag_ck2<T, CSEG, true>, 64, 2);
+    else launch(k_tridiag_ck2<T, CSEG, false>, 64, 2);
   } else {
-    hipLaunchKernelGGL(k_tridiag_b<T>, grid, blk, 0, c->stream, g, m,
-                       (typename CT2<T>::t*)spec, (T*)ck, b.spec, b.ck);
+    // memory bound (384x192x288: 0.103 ms against 0.114 in FP64, 0.065 against
+    // 0.073 in FP32)
+    if (g.nt) launch(k_tridiag_ck2<T, tri_rows<T>(), true>, 256, 2);
+    else launch(k_tridiag_ck2<T, tri_rows<T>(), false>, 256, 2);
   }
   C3D_HIP(hipGetLastError());
   return C3D_OK;
@@ -491,8 +534,8 @@ int launch_tridiag(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
 // depend on the data and come from the host, formed with the same operations.
 // As one thread's loop over global memory (two dependent loads and three
 // divisions per row) this line bounded the
-// kernel: 0.60 ms for two 512x256x512 fields, now 0.48 ms, which the
-// other lines take.
+// kernel: 0.60 ms for two 512x256x512 fields, 0.48 ms from LDS, where the
+// other lines' one-lane sweep bounds it (0.37 ms with the two-lane sweep).
 constexpr int MCH = 256;
 
 template <typename T2>
@@ -563,7 +606,7 @@ __device__ void mean_mode_fp64(const Geom& g, const Metrics<double>& m,
 // Workgroup 0 of a field solves the (0,0) mode, the others every other line
 // by the checkpointed elimination.
 template <typename T, int C, bool NTS>
-__global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, Metrics<T> m, Metrics<double> md,
+__global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, PprRows(T), Metrics<double> md,
                                                        const double* __restrict__ fac,
                                                        typename CT2<T>::t* __restrict__ spec,
                                                        T* __restrict__ ckp, double* w,
@@ -574,9 +617,10 @@ __global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, Metrics<T> m, Met
     mean_mode_fp64(g, md, fac, spec, w + bw * blockIdx.y);
     return;
   }
-  const long long l = (long long)(blockIdx.x - 1) * 256 + threadIdx.x;
+  const long long l = ((long long)(blockIdx.x - 1) * 256 + threadIdx.x) >> 1;
   if (l == 0) return;
-  k_tridiag_ck_body<T, C, NTS>(g, m, spec, ckp + bck * blockIdx.y, line_of(g, l));
+  k_tridiag_ck2_body<T, C, NTS>(g, am, ac, ap, wx, wz, spec, ckp + bck * blockIdx.y,
+                                line_of(g, l));
 }
 
 // r = f - L phi in FP64, L the discrete operator the spectral solve inverts:
@@ -726,11 +770,11 @@ static int ppe_mixed(c3d_ctx* c, const void* prsrc, void* phi, int sweeps, void*
     if ((r = launch_fft32(c, FFT32_Z_FWD, nullptr, spec, nullptr, 0, b))) return r;
     hipEvent_t ev;
     prof_begin(c, ST_TRIDIAG, &ev);
-    constexpr int CSEG = 16;
     const long long nl = (long long)(g.nk + 1) * g.nz;
-    const dim3 grid((unsigned)(1 + (nl + 255) / 256), b.n), blk(256);
-    hipLaunchKernelGGL((k_tridiag_mixed<float, CSEG, false>), grid, blk, 0, c->stream, g, c->mf,
-                       c->md, c->d_meanfac, (float2*)spec, (float*)ck, w, b.spec32, b.ck, b.mean);
+    const dim3 grid((unsigned)(1 + (2 * nl + 255) / 256), b.n), blk(256);
+    hipLaunchKernelGGL((k_tridiag_mixed<float, tri_rows<float>(), false>), grid, blk, 0, c->stream,
+                       g, PPR_OF(c->mf), c->md, c->d_meanfac, (float2*)spec, (float*)ck, w,
+                       b.spec32, b.ck, b.mean);
     C3D_HIP(hipGetLastError());
     prof_end(c, ST_TRIDIAG, ev, 2.0 * (double)g.nx * g.ny * g.nz * b.n * 4);
     return launch_fft32(c, FFT32_Z_INV, nullptr, spec, nullptr, 0, b);
