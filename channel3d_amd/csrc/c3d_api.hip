@@ -358,7 +358,7 @@ static void thomas_factors(const std::vector<double>& a, const std::vector<doubl
 // cell operator's a, vecm, arr, the node operator's a, vecm, arr, the cell
 // operator's b and c, the node operator's b and c
 static size_t adi_table_len(const Geom& g) {
-  return (size_t)g.nx + (size_t)g.nz + 10 * ((size_t)g.ny + 2);
+  return (size_t)g.nx + (size_t)g.nz + 12 * ((size_t)g.ny + 2);
 }
 
 static int build_adi_tables(c3d_ctx* c) {
@@ -392,6 +392,7 @@ static int build_adi_tables(c3d_ctx* c) {
     std::memcpy(yb + 0 * L, a.data(), sizeof(double) * L);
     std::memcpy(yb + 1 * L, vecm.data(), sizeof(double) * L);
     std::memcpy(yb + 2 * L, arr.data(), sizeof(double) * L);
+    for (size_t j = 0; j < L; ++j) yb[10 * L + j] = vecm[j] != 0.0 ? 1.0 / vecm[j] : 0.0;
     std::memcpy(yb + 6 * L, b.data(), sizeof(double) * L);
     std::memcpy(yb + 7 * L, cc.data(), sizeof(double) * L);
     for (int q = 0; q < 3; ++q) tb.d_yc[q] = db + nx + nz + q * L;
@@ -407,6 +408,7 @@ static int build_adi_tables(c3d_ctx* c) {
     std::memcpy(yb + 3 * L, a.data(), sizeof(double) * L);
     std::memcpy(yb + 4 * L, vecm.data(), sizeof(double) * L);
     std::memcpy(yb + 5 * L, arr.data(), sizeof(double) * L);
+    for (size_t j = 0; j < L; ++j) yb[11 * L + j] = vecm[j] != 0.0 ? 1.0 / vecm[j] : 0.0;
     std::memcpy(yb + 8 * L, b.data(), sizeof(double) * L);
     std::memcpy(yb + 9 * L, cc.data(), sizeof(double) * L);
     for (int q = 0; q < 3; ++q) tb.d_yp[q] = db + nx + nz + (3 + q) * L;
@@ -837,6 +839,11 @@ extern "C" int c3d_create(const c3d_params* p, const double* yp, c3d_ctx** out) 
     if (e != hipSuccess) return fail(hip_fail(e, "hipMemset"));
   }
   if ((rc = dalloc(c, &c->tmpA, fbytes))) return fail(rc);
+  // convolved right-hand sides of uy and uz where a substep convolves the three
+  // components in one launch (small fields; an LES context uses them as well)
+  if (c->order == 2 && adi3_fields(g, c->esize))
+    for (int d = 0; d < 2; ++d)
+      if ((rc = dalloc(c, &c->les_arr[d], fbytes))) return fail(rc);
   if ((rc = dalloc(c, &c->spec, (size_t)g.nspec * 2 * c->esize))) return fail(rc);
   if ((rc = dalloc(c, &c->sarr, (size_t)g.nspec * c->esize))) return fail(rc);
   {
@@ -1527,9 +1534,16 @@ extern "C" int c3d_substep(c3d_ctx* c, int ns) {
     return rc;
   // clcU1Hat..U3Hat (:104-106); the constant-flow-rate shift of RhsX is
   // applied while the x sweep loads it
-  if ((rc = launch_adi(c, 0, ns, s[C3D_UX], s[C3D_ARR1], nullptr, c->p.is_ux_const))) return rc;
-  if ((rc = launch_adi(c, 1, ns, s[C3D_UY], s[C3D_ARR2], s[C3D_DUY_YM], 0))) return rc;
-  if ((rc = launch_adi(c, 2, ns, s[C3D_UZ], s[C3D_HALOARR], nullptr, 0))) return rc;
+  {
+    void* const u[3] = {s[C3D_UX], s[C3D_UY], s[C3D_UZ]};
+    void* const r[3] = {s[C3D_ARR1], s[C3D_ARR2], s[C3D_HALOARR]};
+    bool done = false;
+    if ((rc = launch_adi3(c, ns, u, r, s[C3D_DUY_YM], c->p.is_ux_const, &done))) return rc;
+    for (int d = 0; d < 3 && !done; ++d)
+      if ((rc = launch_adi(c, d, ns, u[d], r[d], d == 1 ? s[C3D_DUY_YM] : nullptr,
+                           d == 0 ? c->p.is_ux_const : 0)))
+        return rc;
+  }
   // :110-114
   if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
   if (c->ppe_sweeps < 0 && fft_size_compiled(c->g.nk) && !c->g.fftrt) {

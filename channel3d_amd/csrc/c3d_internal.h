@@ -111,6 +111,14 @@ __device__ __forceinline__ float quot(float a, float v, float r) {
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-v, q, a), r, q), v, a);
 }
 
+// quot by a divisor whose reciprocal is tabulated: r is 1/v rounded (FP64), or
+// that rounded to FP32 and refined for the FP32 divisor.
+__device__ __forceinline__ double tab_recip(double, double r) { return r; }
+__device__ __forceinline__ float tab_recip(float v, double r) {
+  const float q = (float)r;
+  return __builtin_fmaf(__builtin_fmaf(-v, q, 1.0f), q, q);
+}
+
 // Reproducible sums.  Each double term is truncated to a multiple of 2^-80
 // and split into four signed 32-bit limbs accumulated in int64: integer
 // addition is associative, so the total is independent of the order and of
@@ -342,7 +350,9 @@ struct c3d_ctx {
   int* cln_fb = nullptr;
   double les_fcoe[9] = {};
   void* d_lesmet = nullptr;
-  void* les_arr[2] = {nullptr, nullptr};  // elimination scratch of the uy and uz LES solves
+  // uy's and uz's field-sized scratch (ux's is tmpA): checkpoints of the LES
+  // solves, convolved right-hand sides of the merged 2nd-order solves
+  void* les_arr[2] = {nullptr, nullptr};
   c3d::LesMet<double> lmd{};
   c3d::LesMet<float> lmf{};
 
@@ -418,11 +428,27 @@ int launch_diag(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int 
 int launch_diag_finalize(c3d_ctx* c, int nblocks, int what, int cfl_slot);
 
 // ---- launchers (k_adi.hip) ----
+// fields small enough that a substep's three convolutions and three y sweeps
+// run as one launch each (the bound above which fields stream through the
+// caches): at 64^3 one component's launch is a serial sweep on a few CUs
+inline bool adi3_fields(const Geom& g, size_t esize) {
+  return (double)g.nfield * esize < 64.0 * 1024 * 1024;
+}
+// reciprocals of the pivots of the y operator of component comp at substep ns
+inline const double* adi_recip(const c3d_ctx* c, int ns, int comp) {
+  const size_t L = (size_t)c->g.ny + 2;
+  return c->adi[ns - 1].d_xtaps + c->g.nx + c->g.nz + (comp == 1 ? 11 : 10) * L;
+}
 // comp: 0 ux (CN metrics), 1 uy (node metrics + wall row), 2 uz (CN metrics).
 // add_dpmdxns: 2nd order adds dpmdxns to RhsX during the x sweep; 4th order
 // (y solve only) subtracts dp1ns from RhsX as the sweep loads it
 int launch_adi(c3d_ctx* c, int comp, int ns, void* u, void* rhs, const void* duy_ym,
                int add_dpmdxns);
+// the three components' x-z convolutions and y sweeps of a 2nd-order substep in
+// two launches; *done = false (nothing launched) where the separate launches
+// apply: fields too large to gain, or no fused convolution
+int launch_adi3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
+                int add_dpmdxns, bool* done);
 int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
                   int add_dpmdxns);
 

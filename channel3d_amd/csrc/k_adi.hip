@@ -82,20 +82,17 @@ __global__ __launch_bounds__(ABX* ABY) void k_conv_z(Geom g, const double* __res
 constexpr int MAXMX = 32;
 
 // TIN: type of the right-hand side read (an FP32 solve of an FP64 right-hand
-// side); batches: blockIdx.y selects the field, bf reals apart in f and out.
-template <typename T, int MZ, bool ADD, bool NTS = false, typename TIN = T>
-__global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restrict__ xt, int mx,
-                                                 const double* __restrict__ zt,
-                                                 const TIN* __restrict__ f, T* __restrict__ out,
-                                                 const DevScalars* __restrict__ sc, int kchunk,
-                                                 int gxb, int gyb, long long bf) {
+// side); adding: the right-hand side is shifted by add.
+template <typename T, int MZ, bool NTS, typename TIN>
+__device__ __forceinline__ void conv_xz_body(const Geom& g, const double* __restrict__ xt, int mx,
+                                             const double* __restrict__ zt,
+                                             const TIN* __restrict__ f, T* __restrict__ out,
+                                             bool adding, T add, int kchunk, int gxb, int gyb,
+                                             T (*sm)[64 + 2 * MAXMX]) {
   // the convolutions replace the reference's periodic Thomas solves, so their
   // rounding differs from it regardless: fused multiply-adds are allowed here
 #pragma clang fp contract(fast)
   constexpr int NZT = 2 * MZ + 1;
-  f += bf * blockIdx.y;
-  out += bf * blockIdx.y;
-  __shared__ T sm[4][64 + 2 * MAXMX];
   const int nbl = gridDim.x;
   const int lb = xcd_remap(blockIdx.x, nbl);
   const int bx = lb % gxb, by = (lb / gxb) % gyb, bz = lb / (gxb * gyb);
@@ -106,7 +103,6 @@ __global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restric
   const bool rowok = jc <= g.ny;
   const bool active = rowok && i < nx;
   const int k0 = bz * kchunk, k1 = min(nz, k0 + kchunk);
-  const T add = ADD ? (T)sc->dpmdxns : T(0);
   // a staged row holds 64 + 2 mx <= 128 values: two per thread
   // x positions this thread stages (periodic), fixed for the whole march
   int ix[2];
@@ -146,7 +142,7 @@ __global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restric
   load(wrapk(kn), raw);
   auto step = [&]() -> T {
 #pragma unroll
-    for (int q = 0; q < 2; ++q) sm[ty][tx + 64 * q] = ADD ? raw[q] + add : raw[q];
+    for (int q = 0; q < 2; ++q) sm[ty][tx + 64 * q] = adding ? raw[q] + add : raw[q];
     if (pend_at >= 0) C3D_ST_ONCE(pend, &out[pend_at]);  // written once
     pend_at = -1;
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -181,6 +177,37 @@ __global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restric
     }
   }
   if (pend_at >= 0) C3D_ST_ONCE(pend, &out[pend_at]);
+}
+
+// batches: blockIdx.y selects the field, bf reals apart in f and out.
+template <typename T, int MZ, bool ADD, bool NTS = false, typename TIN = T>
+__global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restrict__ xt, int mx,
+                                                 const double* __restrict__ zt,
+                                                 const TIN* __restrict__ f, T* __restrict__ out,
+                                                 const DevScalars* __restrict__ sc, int kchunk,
+                                                 int gxb, int gyb, long long bf) {
+  __shared__ T sm[4][64 + 2 * MAXMX];
+  conv_xz_body<T, MZ, NTS, TIN>(g, xt, mx, zt, f + bf * blockIdx.y, out + bf * blockIdx.y, ADD,
+                                ADD ? (T)sc->dpmdxns : T(0), kchunk, gxb, gyb, sm);
+}
+
+// the three components of a substep in one launch (blockIdx.y = component),
+// add: the ux right-hand side carries the constant-flow-rate shift
+template <typename T>
+struct Conv3 {
+  const T* f[3];
+  T* out[3];
+};
+template <typename T, int MZ>
+__global__ __launch_bounds__(256) void k_conv_xz3(Geom g, const double* __restrict__ xt, int mx,
+                                                  const double* __restrict__ zt, Conv3<T> a,
+                                                  const DevScalars* __restrict__ sc, int add,
+                                                  int kchunk, int gxb, int gyb) {
+  __shared__ T sm[4][64 + 2 * MAXMX];
+  const int d = blockIdx.y;
+  const bool adding = d == 0 && add != 0;
+  conv_xz_body<T, MZ, false, T>(g, xt, mx, zt, a.f[d], a.out[d], adding,
+                                adding ? (T)sc->dpmdxns : T(0), kchunk, gxb, gyb, sm);
 }
 
 // Thomas sweeps along y with shared factors: a(j), vecm(j), arrmn(j) for
@@ -299,6 +326,11 @@ __global__ __launch_bounds__(256) void k_adi_y(Geom g, const double* __restrict_
 // column, so NTH changes only the grouping): 256, or 64 on grids with few
 // lines, where 256-line workgroups would leave CUs idle.
 constexpr int YNT = 256;
+// a segment's rows carry the guard against rows past the last; it is the top one
+template <bool G, bool TOP>
+struct SegKind {
+  static constexpr bool guard = G, top = TOP;
+};
 // One line's sweep: ck is the workgroup's LDS checkpoint array
 // [segment][NTH threads], tid the thread's column, line < nx*nz.
 template <typename T, int C, int WALL, bool SHIFT, bool NTS, bool SET, typename TU, bool FY,
@@ -306,6 +338,7 @@ template <typename T, int C, int WALL, bool SHIFT, bool NTS, bool SET, typename 
 __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __restrict__ ta,
                                               const double* __restrict__ tvecm,
                                               const double* __restrict__ tarr,
+                                              const double* __restrict__ trv,
                                               const T* __restrict__ r, TU* __restrict__ u,
                                               const T* __restrict__ duy,
                                               const DevScalars* __restrict__ sc,
@@ -323,11 +356,11 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
   // the compiler waits for every outstanding load (the prefetched segment
   // included), so the other segments run unguarded (G false).  With FY (ny a
   // multiple of C) the top segment is whole too.
-  using Gd = std::integral_constant<bool, !FY>;
-  using Un = std::false_type;
+  using Gd = SegKind<!FY, true>;
+  using Un = SegKind<false, false>;
   // rows s*C+1 .. s*C+C of the right-hand side (0 past the last row)
   auto load = [&](T* y, int s, auto gv) {
-    constexpr bool G = decltype(gv)::value;
+    constexpr bool G = decltype(gv)::guard;
     const int lo = s * C + 1;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
@@ -336,7 +369,7 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
     }
   };
   auto loadu = [&](TU* uv, int s, auto gv) {
-    constexpr bool G = decltype(gv)::value;
+    constexpr bool G = decltype(gv)::guard;
     const int lo = s * C + 1;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
@@ -344,20 +377,18 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
       uv[q] = (!SET && (!G || j <= ny)) ? C3D_LD_ONCE(&u[base + sj * j]) : TU(0);  // once
     }
   };
-  // forward recurrence of segment s from f (the value at the row below it)
+  // forward recurrence of segment s from f (the value at the row below it, 0
+  // below row 1)
   auto fwd = [&](T* y, int s, T& f, auto gv) {
-    constexpr bool G = decltype(gv)::value;
+    constexpr bool G = decltype(gv)::guard;
     const int lo = s * C + 1;
-    if (s == 0) {
-      if (WALLROW) y[0] = wallv;
-      f = y[0] / (T)tvecm[1];
-      y[0] = f;
-    }
+    if (WALLROW && s == 0) y[0] = wallv;
 #pragma unroll
     for (int q = 0; q < C; ++q) {
       const int j = lo + q;
-      if ((s > 0 || q > 0) && (!G || j <= ny)) {
-        f = (y[q] - (T)ta[j] * f) / (T)tvecm[j];
+      if (!G || j <= ny) {
+        const T v = (T)tvecm[j];
+        f = quot(y[q] - (T)ta[j] * f, v, tab_recip(v, trv[j]));
         y[q] = f;
       }
     }
@@ -365,12 +396,12 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
   // substitution through segment s (forward values in y, u in uv)
   T x = T(0);
   auto back = [&](const T* y, const TU* uv, int s, auto gv) {
-    constexpr bool G = decltype(gv)::value;
+    constexpr bool G = decltype(gv)::guard;
     const int lo = s * C + 1;
 #pragma unroll
     for (int q = C - 1; q >= 0; --q) {
       const int j = lo + q;
-      if (j < ny) x = y[q] - (T)tarr[j + 1] * x;
+      if (!decltype(gv)::top || j < ny) x = y[q] - (T)tarr[j + 1] * x;
       if (!G || j <= ny) C3D_ST_ONCE(SET ? (TU)x : uv[q] + (TU)x, &u[base + sj * j]);
     }
   };
@@ -441,6 +472,7 @@ template <typename T, int C, int WALL, bool SHIFT, bool NTS = false, bool SET = 
 __global__ __launch_bounds__(NTH) void k_adi_y_ck(Geom g, const double* __restrict__ ta,
                                                   const double* __restrict__ tvecm,
                                                   const double* __restrict__ tarr,
+                                                  const double* __restrict__ trv,
                                                   const T* __restrict__ r, TU* __restrict__ u,
                                                   const T* __restrict__ duy,
                                                   const DevScalars* __restrict__ sc,
@@ -449,7 +481,8 @@ __global__ __launch_bounds__(NTH) void k_adi_y_ck(Geom g, const double* __restri
   const int tid = threadIdx.x;
   const long long line = (long long)blockIdx.x * NTH + tid;
   if (line >= (long long)g.nx * g.nz) return;
-  adi_y_ck_line<T, C, WALL, SHIFT, NTS, SET, TU, FY, NTH>(g, ta, tvecm, tarr, r + bf * blockIdx.y,
+  adi_y_ck_line<T, C, WALL, SHIFT, NTS, SET, TU, FY, NTH>(g, ta, tvecm, tarr, trv,
+                                                          r + bf * blockIdx.y,
                                                           u + bf * blockIdx.y, duy, sc,
                                                           (T*)ck_raw, tid, line);
 }
@@ -462,32 +495,38 @@ __global__ __launch_bounds__(NTH) void k_adi_y_ck(Geom g, const double* __restri
 // waiting on each line's serial sweep when the grid has few lines.
 template <typename T>
 struct AdiY3 {
-  const double* t[3][3];  // per component: ta, tvecm, tarr
   const T* r[3];
   T* u[3];
   const T* duy;
 };
 
+// c*: the cell operator's tables (ux, uz), p*: the node operator's (uy), as
+// restrict arguments so that they come through scalar loads (from a struct
+// they were vector loads, which queue behind the prefetched segment and drain
+// it): 192x128x160 0.064 -> 0.057 ms (4N words at 6.6 TB/s, partly from the
+// last-level cache), the three components at 64^3 3 x 0.015 ms in launches of
+// their own, 0.013 ms here
 template <typename T, int C, bool SHIFT, bool NTS, bool FY, int NTH>
-__global__ __launch_bounds__(NTH) void k_adi_y3(Geom g, AdiY3<T> a,
-                                                const DevScalars* __restrict__ sc) {
+__global__ __launch_bounds__(NTH) void k_adi_y3(
+    Geom g, const double* __restrict__ ca, const double* __restrict__ cvecm,
+    const double* __restrict__ carr, const double* __restrict__ crv,
+    const double* __restrict__ pa, const double* __restrict__ pvecm,
+    const double* __restrict__ parr, const double* __restrict__ prv, AdiY3<T> a,
+    const DevScalars* __restrict__ sc) {
   extern __shared__ unsigned char ck_raw[];
   const int tid = threadIdx.x;
   const long long line = (long long)blockIdx.x * NTH + tid;
   if (line >= (long long)g.nx * g.nz) return;
   T* ck = (T*)ck_raw;
   if (blockIdx.y == 0)
-    adi_y_ck_line<T, C, 0, SHIFT, NTS, false, T, FY, NTH>(g, a.t[0][0], a.t[0][1], a.t[0][2],
-                                                          a.r[0], a.u[0], nullptr, sc, ck, tid,
-                                                          line);
+    adi_y_ck_line<T, C, 0, SHIFT, NTS, false, T, FY, NTH>(g, ca, cvecm, carr, crv, a.r[0], a.u[0],
+                                                          nullptr, sc, ck, tid, line);
   else if (blockIdx.y == 1)
-    adi_y_ck_line<T, C, 1, false, NTS, false, T, FY, NTH>(g, a.t[1][0], a.t[1][1], a.t[1][2],
-                                                          a.r[1], a.u[1], a.duy, sc, ck, tid,
-                                                          line);
+    adi_y_ck_line<T, C, 1, false, NTS, false, T, FY, NTH>(g, pa, pvecm, parr, prv, a.r[1], a.u[1],
+                                                          a.duy, sc, ck, tid, line);
   else
-    adi_y_ck_line<T, C, 0, false, NTS, false, T, FY, NTH>(g, a.t[2][0], a.t[2][1], a.t[2][2],
-                                                          a.r[2], a.u[2], nullptr, sc, ck, tid,
-                                                          line);
+    adi_y_ck_line<T, C, 0, false, NTS, false, T, FY, NTH>(g, ca, cvecm, carr, crv, a.r[2], a.u[2],
+                                                          nullptr, sc, ck, tid, line);
 }
 
 // lines per workgroup of the checkpointed sweep: 64 below 256 workgroups of
@@ -500,9 +539,11 @@ static int y_threads_for(const c3d_ctx* c) {
 
 // y solve + update of one component
 template <typename T>
-static int y_solve(c3d_ctx* c, const c3d_ctx::AdiTab& tb, int comp, void* rhs, void* u,
-                   const void* duy_ym, bool shift) {
+static int y_solve(c3d_ctx* c, int ns, int comp, void* rhs, void* u, const void* duy_ym,
+                   bool shift) {
   const Geom& g = c->g;
+  const auto& tb = c->adi[ns - 1];
+  const double* rv = adi_recip(c, ns, comp);
   dim3 gy((g.nx + 63) / 64, (g.nz + 3) / 4), by(64, 4);
   double* const* yt = comp == 1 ? tb.d_yp : tb.d_yc;
   const DevScalars* sc = (const DevScalars*)c->d_sc;
@@ -517,15 +558,15 @@ static int y_solve(c3d_ctx* c, const c3d_ctx::AdiTab& tb, int comp, void* rhs, v
       constexpr int N_ = decltype(nthc)::value;
       if (comp == 1)
         hipLaunchKernelGGL((k_adi_y_ck<T, CSEG, 1, false, NT_, false, T, FY, N_>), gy, by,
-                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], (const T*)rhs, (T*)u,
+                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], rv, (const T*)rhs, (T*)u,
                            (const T*)duy_ym, sc, 0LL);
       else if (shift)
         hipLaunchKernelGGL((k_adi_y_ck<T, CSEG, 0, true, NT_, false, T, FY, N_>), gy, by,
-                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], (const T*)rhs, (T*)u,
+                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], rv, (const T*)rhs, (T*)u,
                            (const T*)nullptr, sc, 0LL);
       else
         hipLaunchKernelGGL((k_adi_y_ck<T, CSEG, 0, false, NT_, false, T, FY, N_>), gy, by,
-                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], (const T*)rhs, (T*)u,
+                           ck_bytes, c->stream, g, yt[0], yt[1], yt[2], rv, (const T*)rhs, (T*)u,
                            (const T*)nullptr, sc, 0LL);
     };
     // whole segments only (ny a multiple of the segment): the guard-free sweep
@@ -573,17 +614,28 @@ static bool xz_fusable(const Geom& g, const c3d_ctx::AdiTab& tb) {
          2 * mx + 1 < g.nx;
 }
 
+// z planes per workgroup of the fused convolution, nf fields side by side: about
+// 4096 workgroups, and runs long against the 2 mz planes of lead-in; on small
+// grids shorter runs, down to 8 planes, so that most CUs hold a wavefront per
+// SIMD (64^3: 3 x 0.015 ms with one launch and 24-plane runs per component,
+// 0.011 ms for the three in one launch of 8-plane runs)
+static int conv_kchunk(const Geom& g, int mz, int nf) {
+  const int tiles = ((g.nx + 63) / 64) * ((g.ny + 3) / 4) * nf;
+  int nch = (4096 + tiles - 1) / tiles;
+  int kc = (g.nz + nch - 1) / nch;
+  int lo = 4 * mz + 8;
+  if ((long long)tiles * ((g.nz + lo - 1) / lo) < 256) lo = 8;
+  if (kc < lo) kc = lo;
+  return kc > g.nz ? g.nz : kc;
+}
+
 template <typename T, bool ADD>
 static bool launch_xz_fused(c3d_ctx* c, const c3d_ctx::AdiTab& tb, const void* rhs) {
   const Geom& g = c->g;
   const int mx = -tb.xlo, mz = -tb.zlo;
   if (!xz_fusable(g, tb)) return false;
   const int gxb = (g.nx + 63) / 64, gyb = (g.ny + 3) / 4;
-  int nch = (4096 + gxb * gyb - 1) / (gxb * gyb);
-  nch = nch < 1 ? 1 : nch;
-  int kchunk = (g.nz + nch - 1) / nch;
-  if (kchunk < 4 * mz + 8) kchunk = 4 * mz + 8;
-  if (kchunk > g.nz) kchunk = g.nz;
+  const int kchunk = conv_kchunk(g, mz, 1);
   const int gzb = (g.nz + kchunk - 1) / kchunk;
   const dim3 grid(gxb * gyb * gzb), blk(64, 4);
   switch (mz) {
@@ -616,7 +668,7 @@ static int adi_t(c3d_ctx* c, int comp, int ns, void* u, void* rhs, const void* d
   // in place (src/CFD_4th/m_TScheme.f90:443-549)
   if (c->order == 4) {
     prof_begin(c, ST_ADI_Y, &ev);
-    if ((rc = y_solve<T>(c, tb, comp, rhs, u, duy_ym, add != 0))) return rc;
+    if ((rc = y_solve<T>(c, ns, comp, rhs, u, duy_ym, add != 0))) return rc;
     prof_end(c, ST_ADI_Y, ev, 3.0 * N * c->esize);
     return C3D_OK;
   }
@@ -628,7 +680,7 @@ static int adi_t(c3d_ctx* c, int comp, int ns, void* u, void* rhs, const void* d
     C3D_HIP(hipGetLastError());
     prof_end(c, ST_ADI_XZ, ev, 2.0 * N * c->esize);
     prof_begin(c, ST_ADI_Y, &ev);
-    if ((rc = y_solve<T>(c, tb, comp, c->tmpA, u, duy_ym, false))) return rc;
+    if ((rc = y_solve<T>(c, ns, comp, c->tmpA, u, duy_ym, false))) return rc;
     prof_end(c, ST_ADI_Y, ev, 3.0 * N * c->esize);
     return C3D_OK;
   }
@@ -652,7 +704,7 @@ static int adi_t(c3d_ctx* c, int comp, int ns, void* u, void* rhs, const void* d
   prof_end(c, ST_ADI_Z, ev, 2.0 * N * c->esize);
   // y sweep + update
   prof_begin(c, ST_ADI_Y, &ev);
-  if ((rc = y_solve<T>(c, tb, comp, rhs, u, duy_ym, false))) return rc;
+  if ((rc = y_solve<T>(c, ns, comp, rhs, u, duy_ym, false))) return rc;
   prof_end(c, ST_ADI_Y, ev, 3.0 * N * c->esize);
   return C3D_OK;
 }
@@ -686,8 +738,6 @@ static void adi_y3_t(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], c
   const size_t ck_bytes = y3_ck_bytes(c);
   AdiY3<T> a;
   for (int d = 0; d < 3; ++d) {
-    double* const* yt = d == 1 ? tb.d_yp : tb.d_yc;
-    for (int q = 0; q < 3; ++q) a.t[d][q] = yt[q];
     a.r[d] = (const T*)rhs[d];
     a.u[d] = (T*)u[d];
   }
@@ -698,8 +748,9 @@ static void adi_y3_t(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], c
     constexpr bool SH = decltype(shc)::value, NT_ = decltype(ntc)::value,
                    FY = decltype(fyc)::value;
     constexpr int N_ = decltype(nthc)::value;
-    hipLaunchKernelGGL((k_adi_y3<T, CSEG, SH, NT_, FY, N_>), gy, by, ck_bytes, c->stream, g, a,
-                       sc);
+    hipLaunchKernelGGL((k_adi_y3<T, CSEG, SH, NT_, FY, N_>), gy, by, ck_bytes, c->stream, g,
+                       tb.d_yc[0], tb.d_yc[1], tb.d_yc[2], adi_recip(c, ns, 0), tb.d_yp[0],
+                       tb.d_yp[1], tb.d_yp[2], adi_recip(c, ns, 1), a, sc);
   };
   using N64 = std::integral_constant<int, 64>;
   using N256 = std::integral_constant<int, YNT>;
@@ -740,6 +791,62 @@ int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], cons
     if ((rc = launch_adi(c, d, ns, u[d], rhs[d], d == 1 ? duy_ym : nullptr,
                          d == 0 ? add_dpmdxns : 0)))
       return rc;
+  return C3D_OK;
+}
+
+template <typename T>
+static bool conv3_t(c3d_ctx* c, const c3d_ctx::AdiTab& tb, void* const rhs[3],
+                    void* const out[3], int add) {
+  const Geom& g = c->g;
+  const int mx = -tb.xlo, mz = -tb.zlo;
+  const int gxb = (g.nx + 63) / 64, gyb = (g.ny + 3) / 4;
+  const int kchunk = conv_kchunk(g, mz, 3);
+  const dim3 grid(gxb * gyb * ((g.nz + kchunk - 1) / kchunk), 3), blk(64, 4);
+  Conv3<T> a;
+  for (int d = 0; d < 3; ++d) {
+    a.f[d] = (const T*)rhs[d];
+    a.out[d] = (T*)out[d];
+  }
+  switch (mz) {
+#define XZ(M)                                                                                  \
+  case M:                                                                                      \
+    hipLaunchKernelGGL((k_conv_xz3<T, M>), grid, blk, 0, c->stream, g, tb.d_xtaps, mx,          \
+                       tb.d_ztaps, a, (const DevScalars*)c->d_sc, add, kchunk, gxb, gyb);       \
+    break;
+    XZ(0) XZ(1) XZ(2) XZ(3) XZ(4) XZ(5) XZ(6) XZ(7) XZ(8) XZ(9) XZ(10) XZ(11) XZ(12)
+#undef XZ
+    default: return false;
+  }
+  return true;
+}
+
+int launch_adi3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
+                int add_dpmdxns, bool* done) {
+  const Geom& g = c->g;
+  *done = false;
+  if (ns < 1 || ns > 3 || !duy_ym) {
+    set_error("adi3: substep 1..3 with duy_ym");
+    return C3D_ERR_ARG;
+  }
+  const auto& tb = c->adi[ns - 1];
+  if (c->order != 2 || !adi3_fields(g, c->esize) || !c->les_arr[0] || !c->les_arr[1] ||
+      !xz_fusable(g, tb) || c->ymode != YS_CHECKPOINT || y3_ck_bytes(c) > 64 * 1024)
+    return C3D_OK;
+  const double N = (double)g.nx * g.ny * g.nz;
+  void* const out[3] = {c->tmpA, c->les_arr[0], c->les_arr[1]};
+  hipEvent_t ev;
+  prof_begin(c, ST_ADI_XZ, &ev);
+  if (!(c->prec == C3D_FP64 ? conv3_t<double>(c, tb, rhs, out, add_dpmdxns)
+                            : conv3_t<float>(c, tb, rhs, out, add_dpmdxns)))
+    return C3D_OK;
+  C3D_HIP(hipGetLastError());
+  prof_end(c, ST_ADI_XZ, ev, 6.0 * N * c->esize);
+  prof_begin(c, ST_ADI_Y, &ev);
+  if (c->prec == C3D_FP64) adi_y3_t<double>(c, ns, u, out, duy_ym, false);
+  else adi_y3_t<float>(c, ns, u, out, duy_ym, false);
+  C3D_HIP(hipGetLastError());
+  prof_end(c, ST_ADI_Y, ev, 9.0 * N * c->esize);
+  *done = true;
   return C3D_OK;
 }
 
@@ -895,11 +1002,7 @@ static int xz_batch(c3d_ctx* c, const c3d_ctx::AdiTab& tb, const void* rhs, void
   const Geom& g = c->g;
   const int mx = -tb.xlo, mz = -tb.zlo;
   const int gxb = (g.nx + 63) / 64, gyb = (g.ny + 3) / 4;
-  int nch = (4096 + gxb * gyb - 1) / (gxb * gyb);
-  nch = nch < 1 ? 1 : nch;
-  int kchunk = (g.nz + nch - 1) / nch;
-  if (kchunk < 4 * mz + 8) kchunk = 4 * mz + 8;
-  if (kchunk > g.nz) kchunk = g.nz;
+  const int kchunk = conv_kchunk(g, mz, 1);  // per field
   const int gzb = (g.nz + kchunk - 1) / kchunk;
   const dim3 grid(gxb * gyb * gzb, nb), blk(64, 4);
   const DevScalars* sc = (const DevScalars*)c->d_sc;
@@ -926,9 +1029,11 @@ static int xz_batch(c3d_ctx* c, const c3d_ctx::AdiTab& tb, const void* rhs, void
 // y sweeps of a batch: rhs (T, the convolved right-hand side) -> du (double),
 // SET: du = x, else du += x
 template <typename T, bool SET>
-static int y_batch(c3d_ctx* c, const c3d_ctx::AdiTab& tb, int comp, const void* rhs, void* du,
-                   int nb, long long bf) {
+static int y_batch(c3d_ctx* c, int ns, int comp, const void* rhs, void* du, int nb,
+                   long long bf) {
   const Geom& g = c->g;
+  const auto& tb = c->adi[ns - 1];
+  const double* rv = adi_recip(c, ns, comp);
   constexpr int CSEG = 16;
   const size_t ck_bytes = (size_t)((g.ny + CSEG - 1) / CSEG) * YNT * sizeof(T);
   if (ck_bytes > 64 * 1024) {
@@ -942,7 +1047,7 @@ static int y_batch(c3d_ctx* c, const c3d_ctx::AdiTab& tb, int comp, const void* 
     constexpr bool NT_ = decltype(ntc)::value;
     constexpr int W_ = decltype(wallc)::value;
     hipLaunchKernelGGL((k_adi_y_ck<T, CSEG, W_, false, NT_, SET, double>), gy, by, ck_bytes,
-                       c->stream, g, yt[0], yt[1], yt[2], (const T*)rhs, (double*)du,
+                       c->stream, g, yt[0], yt[1], yt[2], rv, (const T*)rhs, (double*)du,
                        (const T*)nullptr, sc, bf);
   };
   using W0 = std::integral_constant<int, 0>;
@@ -977,7 +1082,7 @@ int run_helmholtz_batch(c3d_ctx* c, int comp, int ns, int nb, const void* rhs, v
     if ((rc = xz_batch<double, double>(c, tb, rhs, c->btmp, nb, bf))) return rc;
     prof_end(c, ST_ADI_XZ, ev, 2.0 * N * 8);
     prof_begin(c, ST_ADI_Y, &ev);
-    if ((rc = y_batch<double, true>(c, tb, comp, c->btmp, du, nb, bf))) return rc;
+    if ((rc = y_batch<double, true>(c, ns, comp, c->btmp, du, nb, bf))) return rc;
     prof_end(c, ST_ADI_Y, ev, 2.0 * N * 8);
     return C3D_OK;
   }
@@ -985,7 +1090,7 @@ int run_helmholtz_batch(c3d_ctx* c, int comp, int ns, int nb, const void* rhs, v
   if ((rc = xz_batch<float, double>(c, tb, rhs, c->btmp, nb, bf))) return rc;
   prof_end(c, ST_ADI_XZ, ev, N * (8 + 4));
   prof_begin(c, ST_ADI_Y, &ev);
-  if ((rc = y_batch<float, true>(c, tb, comp, c->btmp, du, nb, bf))) return rc;
+  if ((rc = y_batch<float, true>(c, ns, comp, c->btmp, du, nb, bf))) return rc;
   prof_end(c, ST_ADI_Y, ev, N * (4 + 8));
   const double beta = 0.5 * c->aconst[ns - 1] * c->p.xnu * c->dt;
   const double wxo = -beta * c->rdx2, wxc = beta * c->rdx2 * 2.0 + 1.0;
@@ -1014,7 +1119,7 @@ int run_helmholtz_batch(c3d_ctx* c, int comp, int ns, int nb, const void* rhs, v
     if ((rc = xz_batch<float, float>(c, tb, c->bres, c->btmp, nb, bf))) return rc;
     prof_end(c, ST_ADI_XZ, ev, 2.0 * N * 4);
     prof_begin(c, ST_ADI_Y, &ev);
-    if ((rc = y_batch<float, false>(c, tb, comp, c->btmp, du, nb, bf))) return rc;
+    if ((rc = y_batch<float, false>(c, ns, comp, c->btmp, du, nb, bf))) return rc;
     prof_end(c, ST_ADI_Y, ev, N * (4 + 16));
   }
   return C3D_OK;
