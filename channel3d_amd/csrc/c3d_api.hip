@@ -1238,6 +1238,17 @@ extern "C" int c3d_SetBC_and_UpdateHalo(c3d_ctx* c, void* ux, void* uy, void* uz
 static int read_scalars(c3d_ctx* c) {
   C3D_HIP(hipMemcpyAsync(&c->h_sc, c->d_sc, sizeof(DevScalars), hipMemcpyDeviceToHost, c->stream));
   C3D_HIP(hipStreamSynchronize(c->stream));
+  // a maximum is its plain field (a finalising kernel's) or its slots (a step's);
+  // whichever was not written last is zero
+  DevScalars& h = c->h_sc;
+  double* const field[RED_N] = {nullptr, nullptr, nullptr, nullptr, &h.divmax1, &h.divmax2,
+                                &h.vmax[0], &h.vmax[1], &h.vmax[2], &h.uddxmax[0], &h.uddxmax[1]};
+  for (int w = RED_DIV1; w < RED_N; ++w)
+    for (int q = 0; q < RED_SLOTS; ++q) {
+      double v;
+      std::memcpy(&v, &h.red[q][w], sizeof v);
+      if (v > *field[w]) *field[w] = v;
+    }
   return prof_harvest(c);
 }
 
@@ -1424,7 +1435,7 @@ extern "C" int c3d_CheckDivergence(c3d_ctx* c, const void* ux, const void* uy, c
                                    double* divmax) {
   CHECK_CTX(c);
   if (!divmax) return C3D_ERR_ARG;
-  int rc = c->order == 4 ? launch_div4(c, ux, uy, uz) : launch_diag(c, ux, uy, uz, 2, 0);
+  int rc = c->order == 4 ? launch_div4(c, ux, uy, uz, false) : launch_diag(c, ux, uy, uz, 2, 0);
   if (!rc) rc = read_scalars(c);
   if (rc) return rc;
   *divmax = c->h_sc.divmax2;
@@ -1453,16 +1464,24 @@ extern "C" int c3d_CalcUxAver(c3d_ctx* c, const void* ux, double* uxaver) {
 // ===========================================================================
 // fused, device-resident step (m_ChannelSystem.f90:73-130)
 // ===========================================================================
-// one substep of the 4th-order ChannelIterate (src/CFD_4th/m_ChannelSystem.f90:105-143)
-static int substep4(c3d_ctx* c, int ns) {
+// One substep in ChannelIterate's order.  The small routines run inside their
+// neighbours: Update_uy_ym with the clearing of the reductions (substep_begin),
+// SetBC_and_UpdateHaloForPrSrc where the pressure source reads uy, the
+// flow-rate and divergence reductions in the kernels that produce them, the
+// final SetBC_and_UpdateHalo(_pr) in the projection.  At 64^3 each of them cost
+// a launch of about 5 us, nine of a substep's nineteen (step 0.169 -> 0.124 ms).
+// next_slot >= 0: the first substep of a step (see launch_substep_begin).
+
+// 4th order (src/CFD_4th/m_ChannelSystem.f90:105-143)
+static int substep4(c3d_ctx* c, int ns, int next_slot) {
   int rc;
   void** s = c->state;
   if ((rc = c3d_PMcoeUpdate(c, ns))) return rc;
-  if ((rc = launch_update_uy_ym(c, s[C3D_UY_YM], s[C3D_DUY_YM]))) return rc;
+  if ((rc = launch_substep_begin(c, next_slot))) return rc;
   const int flow = c->p.is_ux_const != 0;
   // clcRhsXYZ: RhsX -> RealArr1, RhsY -> RealArr2, RhsZ -> RealHalo (:111-117)
   if ((rc = launch_rhs4(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR], s[C3D_ARR1], s[C3D_ARR2],
-                        s[C3D_HALOARR], s[C3D_HISTX], s[C3D_HISTY], s[C3D_HISTZ], flow)))
+                        s[C3D_HALOARR], s[C3D_HISTX], s[C3D_HISTY], s[C3D_HISTZ], flow ? 2 : 0)))
     return rc;
   // clcU1Hat..U3Hat (:120-122) in one launch; RhsX's flow-rate shift is
   // applied as the y sweep loads it
@@ -1472,62 +1491,61 @@ static int substep4(c3d_ctx* c, int ns) {
     if ((rc = launch_adi_y3(c, ns, u, r, s[C3D_DUY_YM], flow))) return rc;
   }
   // :126-130
-  if ((rc = launch_bc4_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
-  if ((rc = launch_prsrc4(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], 0.0))) return rc;
+  if ((rc = launch_prsrc4(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], 0.0, true))) return rc;
   if ((rc = run_ppe(c, s[C3D_ARR1], s[C3D_HALOARR]))) return rc;
-  // :133-136, the Neumann ghosts of phi applied inside the projection
-  if ((rc = launch_proj4(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR], 1, 1, 1)))
-    return rc;
-  // :138-139
-  if ((rc = launch_bc4_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 1))) return rc;
-  return launch_bc_pr(c, s[C3D_PR]);
+  // :133-139, the Neumann ghosts of phi applied inside the projection
+  return launch_proj4_walls(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR]);
 }
 
-// one substep of the LES scheme (m_ChannelSystem.f90:91-125 with the
-// pointers of m_TScheme.f90:185-203); nut was evaluated at the step start
-static int substep_les(c3d_ctx* c, int ns) {
+// the pressure source and solve into RealHalo; pr: corrected by -nu/2 div
+static int substep_pressure(c3d_ctx* c, void* pr) {
+  int rc;
+  void** s = c->state;
+  if (c->ppe_sweeps < 0 && fft_size_compiled(c->g.nk) && !c->g.fftrt) {
+    // clcPrSrc fused into the first pass of clcPPE (RealArr1 is not written);
+    // on large grids the wall rows of uy are set before it
+    if (c->g.nt && (rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0)))
+      return rc;
+    if ((rc = launch_prsrc_fft_x(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], pr))) return rc;
+    return run_ppe_from_spectrum(c, s[C3D_HALOARR]);
+  }
+  // x lengths with a run-time plan and the refined solve: a source pass
+  if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
+  if ((rc = launch_prsrc(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], pr, 0.0))) return rc;
+  return run_ppe(c, s[C3D_ARR1], s[C3D_HALOARR]);
+}
+
+// the LES scheme (m_ChannelSystem.f90:91-125 with the pointers of
+// m_TScheme.f90:185-203); nut was evaluated at the step start
+static int substep_les(c3d_ctx* c, int ns, int next_slot) {
   int rc;
   void** s = c->state;
   if ((rc = c3d_PMcoeUpdate(c, ns))) return rc;
-  if ((rc = launch_update_uy_ym(c, s[C3D_UY_YM], s[C3D_DUY_YM]))) return rc;
+  if ((rc = launch_substep_begin(c, next_slot))) return rc;
   if ((rc = launch_rhs_les(c, 7, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR], s[C3D_ARR1],
                            s[C3D_ARR2], s[C3D_HALOARR], s[C3D_HISTX], s[C3D_HISTY], s[C3D_HISTZ],
                            1)))
     return rc;
-  // the three wall-normal solves in one launch (the ux solve's elimination
-  // scratch in tmpA, the others' in the LES scratch fields); the
-  // constant-flow-rate shift of RhsX is applied as the ux solve loads it
+  // the three wall-normal solves in one launch (the ux solve's checkpoints in
+  // tmpA, the others' in the scratch fields); the constant-flow-rate shift of
+  // RhsX is applied as the ux solve loads it
   {
     void* const u[3] = {s[C3D_UX], s[C3D_UY], s[C3D_UZ]};
     void* const r[3] = {s[C3D_ARR1], s[C3D_ARR2], s[C3D_HALOARR]};
     if ((rc = launch_les_y3(c, u, r, s[C3D_DUY_YM], c->p.is_ux_const))) return rc;
   }
-  if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
-  if (c->ppe_sweeps < 0 && fft_size_compiled(c->g.nk) && !c->g.fftrt) {
-    if ((rc = launch_prsrc_fft_x(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], nullptr))) return rc;
-    if ((rc = run_ppe_from_spectrum(c, s[C3D_HALOARR]))) return rc;
-  } else {
-    if ((rc = launch_prsrc(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], nullptr, 0.0)))
-      return rc;
-    if ((rc = run_ppe(c, s[C3D_ARR1], s[C3D_HALOARR]))) return rc;
-  }
-  if ((rc = launch_bc_pr(c, s[C3D_HALOARR]))) return rc;
-  if ((rc = launch_proj(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], nullptr, 1, 0, 0)))
-    return rc;
-  if ((rc = launch_prupd_les(c, s[C3D_PR], s[C3D_HALOARR]))) return rc;
-  if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 1))) return rc;
-  return launch_bc_pr(c, s[C3D_PR]);
+  if ((rc = substep_pressure(c, nullptr))) return rc;
+  return launch_proj_les(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR]);
 }
 
-extern "C" int c3d_substep(c3d_ctx* c, int ns) {
-  CHECK_CTX(c);
+static int substep(c3d_ctx* c, int ns, int next_slot) {
   c->cfl_valid = false;  // step_body validates it again after its last substep
-  if (c->order == 4) return substep4(c, ns);
-  if (c->les_type) return substep_les(c, ns);
+  if (c->order == 4) return substep4(c, ns, next_slot);
+  if (c->les_type) return substep_les(c, ns, next_slot);
   int rc;
   void** s = c->state;
   if ((rc = c3d_PMcoeUpdate(c, ns))) return rc;
-  if ((rc = launch_update_uy_ym(c, s[C3D_UY_YM], s[C3D_DUY_YM]))) return rc;
+  if ((rc = launch_substep_begin(c, next_slot))) return rc;
   // RhsX -> RealArr1, RhsY -> RealArr2, RhsZ -> RealHalo (:97-100)
   if ((rc = launch_rhs(c, 7, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR], s[C3D_ARR1], s[C3D_ARR2],
                        s[C3D_HALOARR], s[C3D_HISTX], s[C3D_HISTY], s[C3D_HISTZ], 1)))
@@ -1538,30 +1556,28 @@ extern "C" int c3d_substep(c3d_ctx* c, int ns) {
     void* const u[3] = {s[C3D_UX], s[C3D_UY], s[C3D_UZ]};
     void* const r[3] = {s[C3D_ARR1], s[C3D_ARR2], s[C3D_HALOARR]};
     bool done = false;
-    if ((rc = launch_adi3(c, ns, u, r, s[C3D_DUY_YM], c->p.is_ux_const, &done))) return rc;
+    if ((rc = launch_adi3(c, ns, u, r, s[C3D_DUY_YM], &done))) return rc;
+    if (!done && c->p.is_ux_const && (rc = launch_bulk_slots(c))) return rc;
     for (int d = 0; d < 3 && !done; ++d)
       if ((rc = launch_adi(c, d, ns, u[d], r[d], d == 1 ? s[C3D_DUY_YM] : nullptr,
                            d == 0 ? c->p.is_ux_const : 0)))
         return rc;
   }
   // :110-114
-  if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
-  if (c->ppe_sweeps < 0 && fft_size_compiled(c->g.nk) && !c->g.fftrt) {
-    // clcPrSrc fused into the first pass of clcPPE (RealArr1 is not written);
-    // x lengths with a run-time plan take the separate source kernel below
-    if ((rc = launch_prsrc_fft_x(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR]))) return rc;
-    if ((rc = run_ppe_from_spectrum(c, s[C3D_HALOARR]))) return rc;
-  } else {
-    if ((rc = launch_prsrc(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], s[C3D_PR], 0.0)))
-      return rc;
-    if ((rc = run_ppe(c, s[C3D_ARR1], s[C3D_HALOARR]))) return rc;
-  }
-  // :115-121, the Neumann ghost of phi applied inside the projection
+  if ((rc = substep_pressure(c, s[C3D_PR]))) return rc;
+  // :115-124, the Neumann ghost of phi applied inside the projection; large grids
+  // set the wall ghosts in launches of their own (see k_proj)
+  if (!c->g.nt)
+    return launch_proj_walls(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR]);
   if ((rc = launch_proj(c, s[C3D_HALOARR], s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_PR], 1, 1, 1)))
     return rc;
-  // :123-124
   if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 1))) return rc;
   return launch_bc_pr(c, s[C3D_PR]);
+}
+
+extern "C" int c3d_substep(c3d_ctx* c, int ns) {
+  CHECK_CTX(c);
+  return substep(c, ns, -1);
 }
 
 static int step_body(c3d_ctx* c) {
@@ -1576,16 +1592,16 @@ static int step_body(c3d_ctx* c) {
   if (c->les_type &&
       (rc = launch_sgs(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_NUT])))
     return rc;
+  const int next = c->cfl_slot ^ 1;
   for (int ns = 1; ns <= c->iadvance; ++ns)
-    if ((rc = c3d_substep(c, ns))) return rc;
+    if ((rc = substep(c, ns, ns == 1 ? next : -1))) return rc;
   // CheckDivergence, CalcVmax (:127-130) and the next step's CFL, one pass
   // (order 4: the divergence with the 4th-order differences in a pass of its own)
-  const int next = c->cfl_slot ^ 1;
   if (c->order == 4) {
-    if ((rc = launch_div4(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ]))) return rc;
-    if ((rc = launch_diag(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], 5, next))) return rc;
+    if ((rc = launch_div4(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], true))) return rc;
+    if ((rc = launch_diag_close(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], 5, next))) return rc;
   } else {
-    if ((rc = launch_diag(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], 7, next))) return rc;
+    if ((rc = launch_diag_close(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], 7, next))) return rc;
   }
   c->last_cfl_slot = c->cfl_slot;
   c->cfl_slot = next;

@@ -193,7 +193,100 @@ struct DevScalars {
   double uxaver;
   double dp1ns;       // 4th order: pmAlpha * dpmdxns, subtracted from RhsX
   double pad[3];
+  // Reductions of the fused substep and of a step's closing pass: RED_SLOTS
+  // partial results on cache lines of their own, since one address takes an
+  // atomic every few ns and the workgroups of a small grid end together.
+  // Words of a line: the flow-rate integral's four limbs, then maxima (the bits
+  // of non-negative doubles, which order like integers).
+  unsigned long long red[16][16];
 };
+constexpr int RED_SLOTS = 16;
+enum { RED_BULK = 0, RED_DIV1 = 4, RED_DIV2, RED_VX, RED_VY, RED_VZ, RED_CFL0, RED_CFL1, RED_N };
+
+// The reductions run inside the kernels that produce them: a workgroup adds its
+// limbs (integers: any order, the same sum) or raises a maximum, without
+// waiting for either; k_substep_begin clears them, the kernel that needs the
+// flow-rate shift forms it from the slots, and the maxima are combined where
+// the host reads them.
+__device__ inline void bulk_add(DevScalars* sc, const long long* v) {
+  unsigned long long* s = sc->red[blockIdx.x % RED_SLOTS];
+  for (int l = 0; l < 4; ++l)
+    if (v[l]) atomicAdd(&s[RED_BULK + l], (unsigned long long)v[l]);
+}
+__device__ inline void raise_max(DevScalars* sc, int word, double v) {
+  atomicMax(&sc->red[blockIdx.x % RED_SLOTS][word],
+            (unsigned long long)__double_as_longlong(v));
+}
+// a value that a finalising kernel wrote replaces what the slots hold of it
+__device__ inline void drop_max(DevScalars* sc, int word) {
+  for (int q = 0; q < RED_SLOTS; ++q) sc->red[q][word] = 0;
+}
+// what turns the integral into the shift (m_TSchemeFIMP_inc.f90:61-74; 4th
+// order m_TScheme.f90:392-407)
+struct Bulk {
+  int on;                    // 0: the shift is in DevScalars already
+  double nxnz, len, ubulk, alphaC, dt;
+  double xnu, alpha;         // 4th order
+  int order, reset_aver;
+};
+// the shift of RhsX; the one caller with `keep` also records it and the pressure
+// gradients
+__device__ inline double bulk_shift(const Bulk& b, DevScalars* sc, bool keep) {
+  if (!b.on) return b.order == 4 ? sc->dp1ns : sc->dpmdxns;
+  long long tot[4] = {0, 0, 0, 0};
+  for (int q = 0; q < RED_SLOTS; ++q)
+    for (int l = 0; l < 4; ++l) tot[l] += (long long)sc->red[q][RED_BULK + l];
+  if (b.order == 4) {
+    const double d = b.xnu * fix_value(tot) / b.nxnz / b.len;
+    if (keep) {
+      sc->dpmdxns = sc->PrGradNow = d;
+      sc->dp1ns = b.alpha * d;
+      sc->PrGradAver = (b.reset_aver ? 0.0 : sc->PrGradAver) + d * b.alphaC;
+    }
+    return b.alpha * d;
+  }
+  const double s1 = fix_value(tot) / b.nxnz / b.len;
+  const double d = b.alphaC * (b.ubulk - s1), now = (b.ubulk - s1) / b.dt;
+  if (keep) {
+    sc->s1tot1 = s1;
+    sc->dpmdxns = d;
+    sc->PrGradNow = now;
+    sc->PrGradAver = (b.reset_aver ? 0.0 : sc->PrGradAver) + b.alphaC * now;
+  }
+  return d;
+}
+
+// wall values of the velocity, m_BC_and_Halo.f90; order 4: noslip_p = channel
+struct WallBC {
+  int bcym, bcyp;
+  double uxm, uym, uzm, uxp, uyp, uzp;  // wall values
+  double dyp1, dypn;                    // dyp(1), dyp(nyp)
+};
+// The wall ghosts that rows 1, 2 and ny determine (SetBC_and_UpdateHalo,
+// m_BC_and_Halo.f90:232-344), from cell c's new velocity; returns uy(jc) itself,
+// the wall value in row 1.
+template <typename T>
+__device__ __forceinline__ T walls_vel(const Geom& g, const WallBC& b, int jc, long long c, T u,
+                                       T v, T w, T* ux, T* uy, T* uz) {
+  const T ym = (T)b.uym, yp = (T)b.uyp;
+  if (jc == g.ny) {
+    const long long t = c + g.nx;
+    const bool ns = b.bcyp == C3D_BC_NOSLIP;
+    ux[t] = ns ? (T)b.uxp * T(2) - u : (T)b.uxp * (T)b.dypn + u;
+    uz[t] = ns ? (T)b.uzp * T(2) - w : (T)b.uzp * (T)b.dypn + w;
+    uy[t] = yp;
+    uy[t + g.nx] = yp * T(2) - v;
+  }
+  if (jc == 2) uy[c - 2 * (long long)g.nx] = ym * T(2) - v;
+  if (jc == 1) {
+    const long long t = c - g.nx;
+    const bool ns = b.bcym == C3D_BC_NOSLIP;
+    ux[t] = ns ? (T)b.uxm * T(2) - u : u - (T)b.uxm * (T)b.dyp1;
+    uz[t] = ns ? (T)b.uzm * T(2) - w : w - (T)b.uzm * (T)b.dyp1;
+    v = ym;
+  }
+  return v;
+}
 
 // 4th-order x/z stencil constants (src/CFD_4th/m_MeshAndMetries.f90:87-91)
 // and the per-substep scalars of the 4th-order routines
@@ -408,6 +501,15 @@ int prof_begin(c3d_ctx* c, int stage, hipEvent_t* ev);
 int prof_end(c3d_ctx* c, int stage, hipEvent_t ev, double bytes);
 
 // ---- launchers (k_stencil.hip) ----
+WallBC make_wallbc(const c3d_ctx* c);
+// what turns the fused substep's flow-rate integral into the shift of RhsX
+Bulk make_bulk(const c3d_ctx* c);
+// Update_uy_ym of the state and the clearing of the substep's reductions;
+// next_slot >= 0 (a step's first substep): also of the closing diagnostics,
+// whose CFL goes to that slot
+int launch_substep_begin(c3d_ctx* c, int next_slot);
+// dpmdxns / dp1ns from the slots, for consumers that read DevScalars
+int launch_bulk_slots(c3d_ctx* c);
 int launch_rhs(c3d_ctx* c, int mask, const void* ux, const void* uy, const void* uz,
                const void* pr, void* rx, void* ry, void* rz, void* hx, void* hy, void* hz,
                int want_bulk);
@@ -421,6 +523,12 @@ int launch_bc_pr(c3d_ctx* c, void* pr);
 int launch_update_uy_ym(c3d_ctx* c, void* uy_ym, void* duy_ym);
 int launch_proj(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr,
                 int do_vel, int do_pr, int ghost_from_interior);
+// velocity and pressure update with every wall ghost that SetBC_and_UpdateHalo
+// and SetBC_and_UpdateHalo_pr would set
+int launch_proj_walls(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr);
+// the closing diagnostics into the slots that k_substep_begin cleared
+int launch_diag_close(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
+                      int cfl_slot);
 // what: bit0 CFL, bit1 divergence, bit2 vmax, bit3 ux average; cfl_slot selects
 // the uddxmax slot written
 int launch_diag(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
@@ -448,7 +556,7 @@ int launch_adi(c3d_ctx* c, int comp, int ns, void* u, void* rhs, const void* duy
 // two launches; *done = false (nothing launched) where the separate launches
 // apply: fields too large to gain, or no fused convolution
 int launch_adi3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
-                int add_dpmdxns, bool* done);
+                bool* done);
 int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
                   int add_dpmdxns);
 
@@ -460,13 +568,16 @@ Coef4<T> make_coef4(const c3d_ctx* c);
 int launch_rhs4(c3d_ctx* c, const void* ux, const void* uy, const void* uz, const void* pr,
                 void* rx, void* ry, void* rz, void* hx, void* hy, void* hz, int want_flow);
 int launch_sub_dp1ns(c3d_ctx* c, void* rx);
+// walls: uy's wall rows taken as the wall values (the substep's
+// SetBC_and_UpdateHaloForPrSrc), max |div| into its slots
 int launch_prsrc4(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* prsrc,
-                  double alpha_override);
+                  double alpha_override, bool walls = false);
 int launch_proj4(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
                  int do_pr, int ghost_from_interior);
 int launch_bc4_vel(c3d_ctx* c, void* ux, void* uy, void* uz, const void* uy_ym, int full);
 // CheckDivergence with the 4th-order x/z differences -> DevScalars::divmax2
-int launch_div4(c3d_ctx* c, const void* ux, const void* uy, const void* uz);
+int launch_div4(c3d_ctx* c, const void* ux, const void* uy, const void* uz, bool closing);
+int launch_proj4_walls(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr);
 
 // ---- launchers (k_les.hip, LES layer of the 2nd-order path) ----
 // eddy viscosity of the context's model into nut, wall ghosts included
@@ -487,6 +598,9 @@ int launch_les_y3(c3d_ctx* c, void* const u[3], void* const rhs[3], const void* 
                   int add_dpmdxns);
 // pressure += (1 - pmBetaT d/dy nut d/dy) phi; phi's wall ghosts must be set
 int launch_prupd_les(c3d_ctx* c, void* pr, const void* phi);
+// FluidVelUpdate, PressureUpdate_PIMP_LES and every wall ghost in one pass (phi's
+// own Neumann ghosts applied on the fly)
+int launch_proj_les(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr);
 
 // ---- launchers (k_stats.hip) ----
 int launch_stat(c3d_ctx* c, const void* ux, const void* uy, const void* uz, const void* pr);
@@ -506,8 +620,8 @@ int launch_tridiag(c3d_ctx* c, void* spec, void* ck, const Batch& b = Batch());
 int run_ppe(c3d_ctx* c, void* prsrc, void* phi);
 // the pressure source (with the -nu/2 div pressure correction when pr is
 // given) fused into the x forward pass of the FP64-solve pressure equation;
-// the source lands in the spectral array only, max |div| in divmax1.  Then
-// run_ppe_from_spectrum finishes the solve into phi.
+// the source lands in the spectral array only, max |div| in its slots.
+// SetBC_and_UpdateHaloForPrSrc is part of it.  Then run_ppe_from_spectrum finishes the solve into phi.
 int launch_prsrc_fft_x(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* pr);
 int run_ppe_from_spectrum(c3d_ctx* c, void* phi);
 // FP32 transforms of the mixed-precision solve

@@ -191,8 +191,8 @@ __global__ __launch_bounds__(256) void k_conv_xz(Geom g, const double* __restric
                                 ADD ? (T)sc->dpmdxns : T(0), kchunk, gxb, gyb, sm);
 }
 
-// the three components of a substep in one launch (blockIdx.y = component),
-// add: the ux right-hand side carries the constant-flow-rate shift
+// the three components of a substep in one launch (blockIdx.y = component); the
+// ux right-hand side carries the constant-flow-rate shift, formed here
 template <typename T>
 struct Conv3 {
   const T* f[3];
@@ -201,13 +201,15 @@ struct Conv3 {
 template <typename T, int MZ>
 __global__ __launch_bounds__(256) void k_conv_xz3(Geom g, const double* __restrict__ xt, int mx,
                                                   const double* __restrict__ zt, Conv3<T> a,
-                                                  const DevScalars* __restrict__ sc, int add,
-                                                  int kchunk, int gxb, int gyb) {
+                                                  DevScalars* sc, Bulk bk, int kchunk, int gxb,
+                                                  int gyb) {
   __shared__ T sm[4][64 + 2 * MAXMX];
   const int d = blockIdx.y;
-  const bool adding = d == 0 && add != 0;
+  const bool adding = d == 0 && bk.on;
+  const bool keep = blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0;
   conv_xz_body<T, MZ, false, T>(g, xt, mx, zt, a.f[d], a.out[d], adding,
-                                adding ? (T)sc->dpmdxns : T(0), kchunk, gxb, gyb, sm);
+                                adding ? (T)bulk_shift(bk, sc, keep) : T(0), kchunk, gxb, gyb,
+                                sm);
 }
 
 // Thomas sweeps along y with shared factors: a(j), vecm(j), arrmn(j) for
@@ -340,8 +342,7 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
                                               const double* __restrict__ tarr,
                                               const double* __restrict__ trv,
                                               const T* __restrict__ r, TU* __restrict__ u,
-                                              const T* __restrict__ duy,
-                                              const DevScalars* __restrict__ sc,
+                                              const T* __restrict__ duy, double dp1ns,
                                               T* __restrict__ ck, int tid, long long line) {
   const int i = (int)(line % g.nx), k = (int)(line / g.nx);
   constexpr bool WALLROW = WALL != 0;
@@ -349,7 +350,7 @@ __device__ __forceinline__ void adi_y_ck_line(const Geom& g, const double* __res
   const int nseg = (ny + C - 1) / C;
   const long long base = (long long)i + g.plane * k;
   const long long sj = g.nx;
-  const T shift = SHIFT ? (T)sc->dp1ns : T(0);
+  const T shift = SHIFT ? (T)dp1ns : T(0);
   const T wallv = WALL == 1 ? duy[i + (long long)g.nx * k] : T(0);
   // The per-row guards (rows past ny) are needed in the top segment only; a
   // guarded load or store is a branch of its own, and across such branches
@@ -483,7 +484,8 @@ __global__ __launch_bounds__(NTH) void k_adi_y_ck(Geom g, const double* __restri
   if (line >= (long long)g.nx * g.nz) return;
   adi_y_ck_line<T, C, WALL, SHIFT, NTS, SET, TU, FY, NTH>(g, ta, tvecm, tarr, trv,
                                                           r + bf * blockIdx.y,
-                                                          u + bf * blockIdx.y, duy, sc,
+                                                          u + bf * blockIdx.y, duy,
+                                                          SHIFT ? sc->dp1ns : 0.0,
                                                           (T*)ck_raw, tid, line);
 }
 
@@ -511,22 +513,23 @@ __global__ __launch_bounds__(NTH) void k_adi_y3(
     Geom g, const double* __restrict__ ca, const double* __restrict__ cvecm,
     const double* __restrict__ carr, const double* __restrict__ crv,
     const double* __restrict__ pa, const double* __restrict__ pvecm,
-    const double* __restrict__ parr, const double* __restrict__ prv, AdiY3<T> a,
-    const DevScalars* __restrict__ sc) {
+    const double* __restrict__ parr, const double* __restrict__ prv, AdiY3<T> a, Bulk bk,
+    DevScalars* sc) {
   extern __shared__ unsigned char ck_raw[];
   const int tid = threadIdx.x;
   const long long line = (long long)blockIdx.x * NTH + tid;
   if (line >= (long long)g.nx * g.nz) return;
   T* ck = (T*)ck_raw;
+  const double sh = SHIFT && blockIdx.y == 0 ? bulk_shift(bk, sc, line == 0) : 0.0;
   if (blockIdx.y == 0)
     adi_y_ck_line<T, C, 0, SHIFT, NTS, false, T, FY, NTH>(g, ca, cvecm, carr, crv, a.r[0], a.u[0],
-                                                          nullptr, sc, ck, tid, line);
+                                                          nullptr, sh, ck, tid, line);
   else if (blockIdx.y == 1)
     adi_y_ck_line<T, C, 1, false, NTS, false, T, FY, NTH>(g, pa, pvecm, parr, prv, a.r[1], a.u[1],
-                                                          a.duy, sc, ck, tid, line);
+                                                          a.duy, 0.0, ck, tid, line);
   else
     adi_y_ck_line<T, C, 0, false, NTS, false, T, FY, NTH>(g, ca, cvecm, carr, crv, a.r[2], a.u[2],
-                                                          nullptr, sc, ck, tid, line);
+                                                          nullptr, 0.0, ck, tid, line);
 }
 
 // lines per workgroup of the checkpointed sweep: 64 below 256 workgroups of
@@ -732,6 +735,7 @@ static void adi_y3_t(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], c
                      bool shift) {
   const Geom& g = c->g;
   const auto& tb = c->adi[ns - 1];
+  const Bulk bk = make_bulk(c);
   constexpr int CSEG = Y3SEG;
   const long long lines = (long long)g.nx * g.nz;
   const int nth = y_threads_for(c);
@@ -743,14 +747,13 @@ static void adi_y3_t(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], c
   }
   a.duy = (const T*)duy;
   const dim3 gy((unsigned)((lines + nth - 1) / nth), 3), by(nth);
-  const DevScalars* sc = (const DevScalars*)c->d_sc;
   auto launch = [&](auto shc, auto ntc, auto fyc, auto nthc) {
     constexpr bool SH = decltype(shc)::value, NT_ = decltype(ntc)::value,
                    FY = decltype(fyc)::value;
     constexpr int N_ = decltype(nthc)::value;
     hipLaunchKernelGGL((k_adi_y3<T, CSEG, SH, NT_, FY, N_>), gy, by, ck_bytes, c->stream, g,
                        tb.d_yc[0], tb.d_yc[1], tb.d_yc[2], adi_recip(c, ns, 0), tb.d_yp[0],
-                       tb.d_yp[1], tb.d_yp[2], adi_recip(c, ns, 1), a, sc);
+                       tb.d_yp[1], tb.d_yp[2], adi_recip(c, ns, 1), a, bk, c->d_sc);
   };
   using N64 = std::integral_constant<int, 64>;
   using N256 = std::integral_constant<int, YNT>;
@@ -786,7 +789,9 @@ int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], cons
     prof_end(c, ST_ADI_Y, ev, 9.0 * N * c->esize);
     return C3D_OK;
   }
+  // the separate sweeps read the shift from DevScalars
   int rc;
+  if (add_dpmdxns && (rc = launch_bulk_slots(c))) return rc;
   for (int d = 0; d < 3; ++d)
     if ((rc = launch_adi(c, d, ns, u[d], rhs[d], d == 1 ? duy_ym : nullptr,
                          d == 0 ? add_dpmdxns : 0)))
@@ -796,7 +801,7 @@ int launch_adi_y3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], cons
 
 template <typename T>
 static bool conv3_t(c3d_ctx* c, const c3d_ctx::AdiTab& tb, void* const rhs[3],
-                    void* const out[3], int add) {
+                    void* const out[3], const Bulk& bk) {
   const Geom& g = c->g;
   const int mx = -tb.xlo, mz = -tb.zlo;
   const int gxb = (g.nx + 63) / 64, gyb = (g.ny + 3) / 4;
@@ -811,7 +816,7 @@ static bool conv3_t(c3d_ctx* c, const c3d_ctx::AdiTab& tb, void* const rhs[3],
 #define XZ(M)                                                                                  \
   case M:                                                                                      \
     hipLaunchKernelGGL((k_conv_xz3<T, M>), grid, blk, 0, c->stream, g, tb.d_xtaps, mx,          \
-                       tb.d_ztaps, a, (const DevScalars*)c->d_sc, add, kchunk, gxb, gyb);       \
+                       tb.d_ztaps, a, c->d_sc, bk, kchunk, gxb, gyb);                           \
     break;
     XZ(0) XZ(1) XZ(2) XZ(3) XZ(4) XZ(5) XZ(6) XZ(7) XZ(8) XZ(9) XZ(10) XZ(11) XZ(12)
 #undef XZ
@@ -821,7 +826,7 @@ static bool conv3_t(c3d_ctx* c, const c3d_ctx::AdiTab& tb, void* const rhs[3],
 }
 
 int launch_adi3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const void* duy_ym,
-                int add_dpmdxns, bool* done) {
+                bool* done) {
   const Geom& g = c->g;
   *done = false;
   if (ns < 1 || ns > 3 || !duy_ym) {
@@ -836,8 +841,9 @@ int launch_adi3(c3d_ctx* c, int ns, void* const u[3], void* const rhs[3], const 
   void* const out[3] = {c->tmpA, c->les_arr[0], c->les_arr[1]};
   hipEvent_t ev;
   prof_begin(c, ST_ADI_XZ, &ev);
-  if (!(c->prec == C3D_FP64 ? conv3_t<double>(c, tb, rhs, out, add_dpmdxns)
-                            : conv3_t<float>(c, tb, rhs, out, add_dpmdxns)))
+  const Bulk bk = make_bulk(c);
+  if (!(c->prec == C3D_FP64 ? conv3_t<double>(c, tb, rhs, out, bk)
+                            : conv3_t<float>(c, tb, rhs, out, bk)))
     return C3D_OK;
   C3D_HIP(hipGetLastError());
   prof_end(c, ST_ADI_XZ, ev, 6.0 * N * c->esize);

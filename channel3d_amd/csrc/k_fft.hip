@@ -306,8 +306,13 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd(Geom g, const TIN* __restrict
 // (m_TScheme.f90:246-276; without PCORR clcPrSrcOther, :213-241) evaluated
 // for the two x points of every complex element as the first FFT pass loads
 // it, so the source never goes through HBM.  Same expressions and order as
-// the stand-alone source kernel, without contraction; the per-block max
-// |div| goes to partials[blockIdx.x].
+// the stand-alone source kernel, without contraction; each workgroup raises
+// the divmax1 slots to its max |div|.  On grids
+// that fit in the caches (not NTS) uy's two wall rows are not read but taken as
+// the wall values, which SetBC_and_UpdateHaloForPrSrc (m_BC_and_Halo.f90:349-405)
+// would have put there in a launch of its own, half the time of this kernel at
+// 64^3; the selects cost more than that launch on large ones (768x384x576: 1.59
+// -> 1.85 ms).
 // ---------------------------------------------------------------------------
 template <typename T>
 struct DivArgs {
@@ -317,7 +322,8 @@ struct DivArgs {
   T* pr;
   const T* rdyp;
   T rdx, rdz, sudtal, xnuhm;
-  double* partials;
+  T vym, vyp;       // uy on the walls, in place of its rows 1 and ny+1
+  DevScalars* sc;   // its divmax1 slots take max |div|
 };
 
 // calls of the first pass's input accessor per thread (its butterflies per
@@ -337,6 +343,7 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd_div(Geom g, DivArgs<T> d,
   __shared__ T2 sm[LINES * LDN];
   __shared__ long long rb[LINES], rkp[LINES];
   __shared__ T rdy[LINES];
+  __shared__ int wall[LINES];  // 1: the row has the lower wall, 2: the upper
   __shared__ double wmax[FNT / 64];
   const int row0 = blockIdx.x * LINES;
   const int tid = threadIdx.x;
@@ -345,8 +352,10 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd_div(Geom g, DivArgs<T> d,
     const int row = row0 + tid;
     long long o = -1, okp = 0;
     T sy = T(0);
+    int wl = 0;
     if (row < g.ny * g.nz) {
       const int jc = row % g.ny + 1, k = row / g.ny;
+      wl = (jc == 1 ? 1 : 0) | (jc == g.ny ? 2 : 0);
       const int kp = k == g.nz - 1 ? 0 : k + 1;
       o = (long long)nx * jc + g.plane * k;
       okp = (long long)nx * jc + g.plane * kp;
@@ -355,6 +364,7 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd_div(Geom g, DivArgs<T> d,
     rb[tid] = o;
     rkp[tid] = okp;
     rdy[tid] = sy;
+    wall[tid] = wl;
   }
   __syncthreads();
   double dm = 0.0;
@@ -376,12 +386,18 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd_div(Geom g, DivArgs<T> d,
     }
     const long long rowkp = rkp[l];
     const T sucaj = rdy[l];
+    const int wl = wall[l];
     T val[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int i = 2 * m + h, ip = i == nx - 1 ? 0 : i + 1;
       const long long c = rowc + i;
-      const T rdiv = (d.ux[rowc + ip] - d.ux[c]) * d.rdx + (d.uy[c + nx] - d.uy[c]) * sucaj +
+      T v0 = d.uy[c], v1 = d.uy[c + nx];
+      if (!NTS) {
+        v0 = wl & 1 ? d.vym : v0;
+        v1 = wl & 2 ? d.vyp : v1;
+      }
+      const T rdiv = (d.ux[rowc + ip] - d.ux[c]) * d.rdx + (v1 - v0) * sucaj +
                      (d.uz[rowkp + i] - d.uz[c]) * d.rdz;
       dm = fmax(dm, (double)fabs(rdiv));
       val[h] = d.sudtal * rdiv;
@@ -408,7 +424,7 @@ __global__ __launch_bounds__(FNT) void k_fft_x_fwd_div(Geom g, DivArgs<T> d,
   if (tid == 0) {
     double r = 0.0;
     for (int q = 0; q < FNT / 64; ++q) r = fmax(r, wmax[q]);
-    d.partials[blockIdx.x] = r;
+    raise_max(d.sc, RED_DIV1, r);
   }
 }
 
@@ -819,7 +835,7 @@ static int fft_x_fwd_t(c3d_ctx* c, const void* in, void* spec, const Batch& b) {
 
 template <typename T, bool NTS>
 static int prsrc_fft_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* pr,
-                       double alpha, int* nblocks) {
+                       double alpha) {
   using T2 = typename CT<T>::t;
   const Geom& g = c->g;
   const int nrows = g.ny * g.nz;
@@ -829,16 +845,13 @@ static int prsrc_fft_t(c3d_ctx* c, const void* ux, const void* uy, const void* u
   d.rdx = (T)c->rdx; d.rdz = (T)c->rdz;
   d.sudtal = (T)(1.0 / alpha);
   d.xnuhm = (T)(-0.5 * c->p.xnu);
-  d.partials = c->d_partials;
+  d.vym = (T)c->p.uybc[2];
+  d.vyp = (T)c->p.uybc[3];
+  d.sc = c->d_sc;
   switch (g.fftrt ? 0 : g.nk) {
 #define X(n_)                                                                                    \
   case n_: {                                                                                     \
     const int nb = (nrows + xlines(n_) - 1) / xlines(n_);                                       \
-    if (nb > c->max_partials) {                                                                  \
-      set_error("prsrc_fft: too many workgroups for the partials buffer");                       \
-      return C3D_ERR_ARG;                                                                        \
-    }                                                                                            \
-    *nblocks = nb;                                                                               \
     if (pr)                                                                                      \
       hipLaunchKernelGGL((k_fft_x_fwd_div<T, n_, true, NTS>), dim3(nb), dim3(FNT), 0, c->stream, g,  \
                          d, (T2*)c->spec, (const T2*)c->tw_x, (const T2*)c->tw_xr);              \
@@ -1033,13 +1046,12 @@ int launch_fft_x_fwd(c3d_ctx* c, const void* in, void* spec, const Batch& b) {
 int launch_prsrc_fft_x(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* pr) {
   hipEvent_t ev;
   prof_begin(c, ST_PRSRC_FFT, &ev);
-  int nb = 0;
-  int rc = c->prec == C3D_FP64 ? (c->g.nt ? prsrc_fft_t<double, true>(c, ux, uy, uz, pr, c->pmAlpha, &nb) : prsrc_fft_t<double, false>(c, ux, uy, uz, pr, c->pmAlpha, &nb))
-                               : (c->g.nt ? prsrc_fft_t<float, true>(c, ux, uy, uz, pr, c->pmAlpha, &nb) : prsrc_fft_t<float, false>(c, ux, uy, uz, pr, c->pmAlpha, &nb));
+  int rc = c->prec == C3D_FP64 ? (c->g.nt ? prsrc_fft_t<double, true>(c, ux, uy, uz, pr, c->pmAlpha) : prsrc_fft_t<double, false>(c, ux, uy, uz, pr, c->pmAlpha))
+                               : (c->g.nt ? prsrc_fft_t<float, true>(c, ux, uy, uz, pr, c->pmAlpha) : prsrc_fft_t<float, false>(c, ux, uy, uz, pr, c->pmAlpha));
   if (rc) return rc;
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   prof_end(c, ST_PRSRC_FFT, ev, (pr ? 6.0 : 4.0) * N * c->esize);
-  return launch_max_finalize(c, nb, 0);
+  return C3D_OK;
 }
 
 int launch_fft_x_inv(c3d_ctx* c, const void* spec, void* out, double scale, const Batch& b) {

@@ -117,7 +117,8 @@ __global__ __launch_bounds__(BX* RHS_WY, 1) void k_rhs(Geom g, Metrics<T> m, Coe
                                                       T* __restrict__ rx, T* __restrict__ ry,
                                                       T* __restrict__ rz, T* __restrict__ hx,
                                                       T* __restrict__ hy, T* __restrict__ hz,
-                                                      double* __restrict__ partials, int kchunk) {
+                                                      double* __restrict__ partials,
+                                                      DevScalars* sc, int kchunk) {
   constexpr int WY = RHS_WY, LW = BX + 2, LP = LW * (WY + 2);  // one field's tile plane
   constexpr int NT = BX * WY, NS = (LP + NT - 1) / NT;         // staging slots per thread
   __shared__ T sb[3][4][LP];
@@ -287,8 +288,12 @@ __global__ __launch_bounds__(BX* RHS_WY, 1) void k_rhs(Geom g, Metrics<T> m, Coe
   if (MASK & 1) {
     block_sum_fix(s1, shf);
     if (tid == 0) {
-      long long* pf = (long long*)partials + 4LL * blockIdx.x;
-      for (int q = 0; q < 4; ++q) pf[q] = s1[q];
+      if (MASK == 7) {  // the fused substep's integral
+        bulk_add(sc, s1);
+      } else {
+        long long* pf = (long long*)partials + 4LL * blockIdx.x;
+        for (int q = 0; q < 4; ++q) pf[q] = s1[q];
+      }
     }
   }
 }
@@ -368,7 +373,8 @@ __global__ __launch_bounds__(BX* BY) void k_prsrc(Geom g, Metrics<T> m, T rdx, T
     partials[blockIdx.x] = r;
 }
 
-__global__ void k_max_finalize(const double* __restrict__ partials, int n, double* out) {
+__global__ void k_max_finalize(const double* __restrict__ partials, int n, double* out,
+                               DevScalars* sc, int word) {
   __shared__ double sh[1024];
   const int t = threadIdx.x;
   double s = 0.0;
@@ -379,7 +385,10 @@ __global__ void k_max_finalize(const double* __restrict__ partials, int n, doubl
     if (t < w) sh[t] = fmax(sh[t], sh[t + w]);
     __syncthreads();
   }
-  if (t == 0) *out = sh[0];
+  if (t == 0) {
+    *out = sh[0];
+    drop_max(sc, word);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -387,12 +396,6 @@ __global__ void k_max_finalize(const double* __restrict__ partials, int n, doubl
 // full=0: SetBC_and_UpdateHaloForPrSrc (:349-405, only the uy wall nodes).
 // One thread per (i,k) wall column.
 // ---------------------------------------------------------------------------
-struct WallBC {
-  int bcym, bcyp;
-  double uxm, uym_unused, uzm, uxp, uyp, uzp;  // wall values
-  double dyp1, dypn;                           // dyp(1), dyp(nyp)
-};
-
 template <typename T>
 __global__ void k_bc_vel(Geom g, WallBC b, T* __restrict__ ux, T* __restrict__ uy,
                          T* __restrict__ uz, const T* __restrict__ uy_ym, int full) {
@@ -442,6 +445,38 @@ __global__ void k_bc_pr(Geom g, T* __restrict__ pr) {
   pr[fidx(g, i, 0, k)] = pr[fidx(g, i, 1, k)];
 }
 
+// the first launch of a fused substep: Update_uy_ym of the state, and zero into
+// the reductions that its kernels add to
+template <typename T>
+__global__ void k_substep_begin(int n, T uybc, T* __restrict__ uy_ym, T* __restrict__ duy_ym,
+                                DevScalars* sc, int next_slot) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n) {
+    const T d = uy_ym[q];
+    uy_ym[q] = uybc;
+    duy_ym[q] = uybc - d;
+  }
+  if (blockIdx.x == 0) {
+    // entries of this substep, and on a step's first of its closing pass
+    auto mine = [&](int w) {
+      return w <= RED_DIV1 || (next_slot >= 0 && (w <= RED_VZ || w == RED_CFL0 + next_slot));
+    };
+    for (int l = threadIdx.x; l < RED_SLOTS * RED_N; l += blockDim.x)
+      if (mine(l % RED_N)) sc->red[l / RED_N][l % RED_N] = 0;
+    if (threadIdx.x == 0) {
+      sc->divmax1 = 0.0;
+      if (next_slot >= 0) {
+        sc->divmax2 = sc->vmax[0] = sc->vmax[1] = sc->vmax[2] = 0.0;
+        sc->uddxmax[next_slot] = 0.0;
+      }
+    }
+  }
+}
+
+__global__ void k_bulk_slots(Bulk b, DevScalars* sc) {
+  if (threadIdx.x == 0) bulk_shift(b, sc, true);
+}
+
 // Update_uy_ym_CH (m_FlowType_Channel.f90:120-130)
 template <typename T>
 __global__ void k_update_uy_ym(int n, T uybc, T* __restrict__ uy_ym, T* __restrict__ duy_ym) {
@@ -463,12 +498,17 @@ __global__ void k_update_uy_ym(int n, T uybc, T* __restrict__ uy_ym, T* __restri
 // cannot be waited for without also waiting for the store), and every load
 // is unconditional (the ghost row is read and then selected).  phi one plane
 // down is the previous plane's own value.
+//
+// WALLS: the wall ghosts of SetBC_and_UpdateHalo and SetBC_and_UpdateHalo_pr
+// (m_BC_and_Halo.f90:232-344, 410-456) are written from the row's new values by
+// the wavefronts of rows 1, 2 and ny, which have them in registers, instead of
+// by two launches that read the rows again (about 5 us each at any size).
 // ---------------------------------------------------------------------------
 constexpr int PKCH = 16;
 
-template <typename T, bool VEL, bool PRS, bool GHOST, bool NTS = false>
+template <typename T, bool VEL, bool PRS, bool GHOST, bool NTS = false, bool WALLS = false>
 __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2, T rdzEta2,
-                                                 T alpha, const T* __restrict__ phi,
+                                                 T alpha, WallBC wb, const T* __restrict__ phi,
                                                  T* __restrict__ ux, T* __restrict__ uy,
                                                  T* __restrict__ uz, T* __restrict__ pr) {
   CELL_BLOCK();
@@ -495,7 +535,8 @@ __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2
     }
     if (PRS) a.p = C3D_LD_ONCE(&pr[c]);
   };
-  auto update = [&](int k, const Plane& a, T phz) {
+  auto update = [&](int k, const Plane& a, T phz, auto wallv) {
+    constexpr bool WALL = decltype(wallv)::value;
     // keep the scheduler from moving this plane's stores above the loads of
     // the next plane issued just before
     __builtin_amdgcn_sched_barrier(0);
@@ -503,33 +544,48 @@ __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2
     const T locphi = a.ph;
     if (VEL) {
       const T phy = (GHOST && jc == 1) ? locphi : a.phy;
-      C3D_ST_ONCE(a.u - (locphi - a.phx) * rdxEta2, &ux[c]);
-      C3D_ST_ONCE(a.v - (locphi - phy) * sucacEta2, &uy[c]);
-      C3D_ST_ONCE(a.w - (locphi - phz) * rdzEta2, &uz[c]);
+      const T un = a.u - (locphi - a.phx) * rdxEta2;
+      T vn = a.v - (locphi - phy) * sucacEta2;
+      const T wn = a.w - (locphi - phz) * rdzEta2;
+      if (WALL) {
+        vn = walls_vel(g, wb, jc, c, un, vn, wn, ux, uy, uz);
+        if (jc == 1) pr[c - g.nx] = a.p + locphi;
+        if (jc == g.ny) pr[c + g.nx] = a.p + locphi;
+      }
+      C3D_ST_ONCE(un, &ux[c]);
+      C3D_ST_ONCE(vn, &uy[c]);
+      C3D_ST_ONCE(wn, &uz[c]);
     }
     if (PRS) C3D_ST_ONCE(a.p + locphi, &pr[c]);
   };
-  T phz = VEL ? phi[row + g.plane * wrapm(k0, g.nz) + i] : T(0);  // phi one plane down
-  // two plane buffers in alternating roles (a copy between them would wait
-  // for the loads, and with them for the stores issued since)
-  Plane a, b;
-  fetch(k0, a);
-  int k = k0;
-  for (; k + 2 < k1; k += 2) {
-    fetch(k + 1, b);
-    update(k, a, phz);
-    phz = a.ph;
-    fetch(k + 2, a);
-    update(k + 1, b, phz);
-    phz = b.ph;
-  }
-  if (k + 1 < k1) {  // a holds plane k; one more plane after it
-    fetch(k + 1, b);
-    update(k, a, phz);
-    update(k + 1, b, a.ph);
-  } else {
-    update(k, a, phz);
-  }
+  auto march = [&](auto wallv) {
+    T phz = VEL ? phi[row + g.plane * wrapm(k0, g.nz) + i] : T(0);  // phi one plane down
+    // two plane buffers in alternating roles (a copy between them would wait
+    // for the loads, and with them for the stores issued since)
+    Plane a, b;
+    fetch(k0, a);
+    int k = k0;
+    for (; k + 2 < k1; k += 2) {
+      fetch(k + 1, b);
+      update(k, a, phz, wallv);
+      phz = a.ph;
+      fetch(k + 2, a);
+      update(k + 1, b, phz, wallv);
+      phz = b.ph;
+    }
+    if (k + 1 < k1) {  // a holds plane k; one more plane after it
+      fetch(k + 1, b);
+      update(k, a, phz, wallv);
+      update(k + 1, b, a.ph, wallv);
+    } else {
+      update(k, a, phz, wallv);
+    }
+  };
+  // a wavefront is one row: the rows that write no ghost take a loop without the
+  // tests.  768x384x576: 2.46 ms without WALLS, 2.56 with the tests in every
+  // row, 2.51 so; large grids therefore keep the two launches, 0.017 ms there.
+  if (WALLS && (jc <= 2 || jc == g.ny)) march(std::true_type{});
+  else march(std::false_type{});
 }
 
 // ---------------------------------------------------------------------------
@@ -537,13 +593,16 @@ __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2
 // CalcVmax :80-104, CalcUxAver :250-270.  One pass; WHAT selects outputs.
 // partials layout: [6][nblocks]: cfl, div, vx, vy, vz, uxsum
 // ---------------------------------------------------------------------------
-template <typename T, int WHAT>
+// CLOSE: the step's closing pass, into the slots that k_substep_begin cleared
+// instead of partials.
+template <typename T, int WHAT, bool CLOSE = false>
 __global__ __launch_bounds__(BX* BY) void k_diag(Geom g, Metrics<T> m, T rdx, T rdz,
                                                  const T* __restrict__ ux,
                                                  const T* __restrict__ uy,
                                                  const T* __restrict__ uz,
                                                  const double* __restrict__ dyp,
-                                                 double* __restrict__ partials, int nblocks) {
+                                                 double* __restrict__ partials, int nblocks,
+                                                 DevScalars* sc, int cfl_slot) {
   __shared__ double sh[8];
   CELL_BLOCK();
   const int i = cbx * BX + threadIdx.x;
@@ -585,6 +644,22 @@ __global__ __launch_bounds__(BX* BY) void k_diag(Geom g, Metrics<T> m, T rdx, T 
   }
   const int b = blockIdx.x;
   double r;
+  if (CLOSE) {
+    const bool lead = threadIdx.x == 0 && threadIdx.y == 0;
+    auto raise = [&](double v, int word, double scale) {
+      const double q = block_max(v, sh);
+      if (lead) raise_max(sc, word, q * scale);
+      __syncthreads();
+    };
+    if (WHAT & 1) raise(cfl, RED_CFL0 + cfl_slot, 0.5);
+    if (WHAT & 2) raise(dv, RED_DIV2, 1.0);
+    if (WHAT & 4) {
+      raise(vx, RED_VX, 1.0);
+      raise(vy, RED_VY, 1.0);
+      raise(vz, RED_VZ, 1.0);
+    }
+    return;
+  }
   if (WHAT & 1) { r = block_max(cfl, sh); if (threadIdx.x == 0 && threadIdx.y == 0) partials[0 * (long long)nblocks + b] = r; __syncthreads(); }
   if (WHAT & 2) { r = block_max(dv, sh); if (threadIdx.x == 0 && threadIdx.y == 0) partials[1 * (long long)nblocks + b] = r; __syncthreads(); }
   if (WHAT & 4) {
@@ -627,6 +702,9 @@ __global__ void k_diag_finalize(const double* __restrict__ partials, int n, int 
     __syncthreads();
   }
   if (t == 0) {
+    for (int w = 0; w < 5; ++w)
+      if (what & (w == 0 ? 1 : w == 1 ? 2 : 4))
+        drop_max(sc, w == 0 ? RED_CFL0 + cfl_slot : RED_DIV2 + w - 1);
     if (what & 1) sc->uddxmax[cfl_slot] = sh[0][0] * 0.5;
     if (what & 2) sc->divmax2 = sh[1][0];
     if (what & 4) { sc->vmax[0] = sh[2][0]; sc->vmax[1] = sh[3][0]; sc->vmax[2] = sh[4][0]; }
@@ -664,13 +742,17 @@ template <>
 const Metrics<float>& mets<float>(c3d_ctx* c) { return c->mf; }
 
 // z run of the RHS kernel: long enough to amortise the two lead-in planes,
-// short enough to give the device a few thousand workgroups
+// short enough to give the device a few thousand workgroups; on small grids down
+// to 4 planes, until every CU has two workgroups (64^3: 0.029 ms with 16 planes,
+// 64 workgroups; 0.014 ms with 4)
 static int rhs_kchunk(const Geom& g) {
   const int tiles = ((g.nx + BX - 1) / BX) * ((g.ny + RHS_WY - 1) / RHS_WY);
   int nch = (4096 + tiles - 1) / tiles;
   if (nch < 1) nch = 1;
   int kc = (g.nz + nch - 1) / nch;
-  if (kc < 16) kc = 16;
+  int lo = 16;
+  while (lo > 4 && tiles * ((g.nz + lo - 1) / lo) < 512) lo /= 2;
+  if (kc < lo) kc = lo;
   return kc > g.nz ? g.nz : kc;
 }
 static int rhs_nblocks(const Geom& g) {
@@ -692,11 +774,11 @@ static int rhs_t(c3d_ctx* c, int mask, const void* ux, const void* uy, const voi
   if (g.nt)                                                                                    \
     hipLaunchKernelGGL((k_rhs<T, M, true>), grid, blk, 0, c->stream, g, m, cf, U(ux), U(uy),    \
                        U(uz), U(pr), W(rx), W(ry), W(rz), W(hx), W(hy), W(hz), c->d_partials,  \
-                       kc);                                                                    \
+                       c->d_sc, kc);                                                           \
   else                                                                                         \
     hipLaunchKernelGGL((k_rhs<T, M, false>), grid, blk, 0, c->stream, g, m, cf, U(ux), U(uy),   \
                        U(uz), U(pr), W(rx), W(ry), W(rz), W(hx), W(hy), W(hz), c->d_partials,  \
-                       kc)
+                       c->d_sc, kc)
   switch (mask) {
     case 1: RHS_LAUNCH(1); break;
     case 2: RHS_LAUNCH(2); break;
@@ -721,7 +803,8 @@ int launch_rhs(c3d_ctx* c, int mask, const void* ux, const void* uy, const void*
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   const int ncomp = (mask & 1) + ((mask >> 1) & 1) + ((mask >> 2) & 1);
   prof_end(c, st, ev, (ncomp == 3 ? 13.0 : 6.0) * N * c->esize);
-  if (want_bulk && (mask & 1) && c->p.is_ux_const)
+  // the fused right-hand sides (mask 7) leave the integral in its slots
+  if (want_bulk && mask == 1 && c->p.is_ux_const)
     return launch_bulk_finalize(c, rhs_nblocks(c->g), c->cur_ns == 1);
   return C3D_OK;
 }
@@ -783,16 +866,16 @@ int launch_prsrc(c3d_ctx* c, const void* ux, const void* uy, const void* uz, voi
 int launch_max_finalize(c3d_ctx* c, int nblocks, int slot) {
   double* out = slot == 0 ? &c->d_sc->divmax1 : &c->d_sc->divmax2;
   hipLaunchKernelGGL(k_max_finalize, dim3(1), dim3(1024), 0, c->stream, c->d_partials, nblocks,
-                     out);
+                     out, c->d_sc, slot == 0 ? RED_DIV1 : RED_DIV2);
   C3D_HIP(hipGetLastError());
   return C3D_OK;
 }
 
-static WallBC make_wallbc(c3d_ctx* c) {
+WallBC make_wallbc(const c3d_ctx* c) {
   WallBC b;
   b.bcym = c->p.bc[2];
   b.bcyp = c->p.bc[3];
-  b.uxm = c->p.uxbc[2]; b.uym_unused = c->p.uybc[2]; b.uzm = c->p.uzbc[2];
+  b.uxm = c->p.uxbc[2]; b.uym = c->p.uybc[2]; b.uzm = c->p.uzbc[2];
   b.uxp = c->p.uxbc[3]; b.uyp = c->p.uybc[3]; b.uzp = c->p.uzbc[3];
   b.dyp1 = c->met[C3D_M_DYP][1];
   b.dypn = c->met[C3D_M_DYP][c->g.ny + 1];
@@ -830,6 +913,46 @@ int launch_bc_pr(c3d_ctx* c, void* pr) {
   return C3D_OK;
 }
 
+Bulk make_bulk(const c3d_ctx* c) {
+  Bulk b{};
+  b.on = c->p.is_ux_const != 0;
+  b.nxnz = (double)c->g.nx * (double)c->g.nz;
+  b.len = c->order == 4 ? c->p.yly : c->p.ybulk2 - c->p.ybulk1;
+  b.ubulk = c->p.ubulk;
+  b.alphaC = c->pmAlphaC;
+  b.dt = c->dt;
+  b.xnu = c->p.xnu;
+  b.alpha = c->pmAlpha;
+  b.order = c->order;
+  b.reset_aver = c->cur_ns == 1;
+  return b;
+}
+
+int launch_bulk_slots(c3d_ctx* c) {
+  hipEvent_t ev;
+  prof_begin(c, ST_BULK, &ev);
+  hipLaunchKernelGGL(k_bulk_slots, dim3(1), dim3(64), 0, c->stream, make_bulk(c), c->d_sc);
+  C3D_HIP(hipGetLastError());
+  prof_end(c, ST_BULK, ev, 0.0);
+  return C3D_OK;
+}
+
+int launch_substep_begin(c3d_ctx* c, int next_slot) {
+  const int n = c->g.nx * c->g.nz;
+  const double v = c->order == 4 ? 0.0 : c->p.uybc[2];
+  const dim3 grid((n + 255) / 256), blk(256);
+  if (c->prec == C3D_FP64)
+    hipLaunchKernelGGL(k_substep_begin<double>, grid, blk, 0, c->stream, n, v,
+                       (double*)c->state[C3D_UY_YM], (double*)c->state[C3D_DUY_YM], c->d_sc,
+                       next_slot);
+  else
+    hipLaunchKernelGGL(k_substep_begin<float>, grid, blk, 0, c->stream, n, (float)v,
+                       (float*)c->state[C3D_UY_YM], (float*)c->state[C3D_DUY_YM], c->d_sc,
+                       next_slot);
+  C3D_HIP(hipGetLastError());
+  return C3D_OK;
+}
+
 int launch_update_uy_ym(c3d_ctx* c, void* uy_ym, void* duy_ym) {
   const int n = c->g.nx * c->g.nz;
   // the 4th-order code sets the wall value to zero (src/CFD_4th/m_FlowCase.f90:162-172)
@@ -846,21 +969,26 @@ int launch_update_uy_ym(c3d_ctx* c, void* uy_ym, void* duy_ym) {
 
 template <typename T>
 static int proj_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int vel,
-                  int prs, int ghost) {
+                  int prs, int ghost, bool walls) {
   const Geom& g = c->g;
+  const WallBC wb = make_wallbc(c);
   const T a = (T)c->pmAlpha;
   const T rdxE = (T)(c->rdx * c->pmAlpha), rdzE = (T)(c->rdz * c->pmAlpha);
   const dim3 grid(ncell_blocks(g, PKCH));
 #define PROJ_LAUNCH(V, P, G)                                                                   \
   if (g.nt)                                                                                    \
     hipLaunchKernelGGL((k_proj<T, V, P, G, true>), grid, dim3(BX, BY), 0, c->stream, g,        \
-                       mets<T>(c), rdxE, rdzE, a, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,      \
+                       mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,  \
                        (T*)pr);                                                                \
   else                                                                                         \
     hipLaunchKernelGGL((k_proj<T, V, P, G, false>), grid, dim3(BX, BY), 0, c->stream, g,       \
-                       mets<T>(c), rdxE, rdzE, a, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,      \
+                       mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,  \
                        (T*)pr)
-  if (vel && prs && ghost) PROJ_LAUNCH(true, true, true);
+  if (walls) {
+    hipLaunchKernelGGL((k_proj<T, true, true, true, false, true>), grid, dim3(BX, BY), 0,
+                       c->stream, g, mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy,
+                       (T*)uz, (T*)pr);
+  } else if (vel && prs && ghost) PROJ_LAUNCH(true, true, true);
   else if (vel && prs) PROJ_LAUNCH(true, true, false);
   else if (vel && ghost) PROJ_LAUNCH(true, false, true);
   else if (vel) PROJ_LAUNCH(true, false, false);
@@ -870,18 +998,54 @@ static int proj_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, voi
   return C3D_OK;
 }
 
-int launch_proj(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
-                int do_pr, int ghost_from_interior) {
+static int proj(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
+                int do_pr, int ghost_from_interior, bool walls) {
   hipEvent_t ev;
   const int st = (do_vel && do_pr) ? ST_PROJ : do_vel ? ST_VELUPD : ST_PRUPD;
   prof_begin(c, st, &ev);
   int rc = c->prec == C3D_FP64
-               ? proj_t<double>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior)
-               : proj_t<float>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior);
+               ? proj_t<double>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, walls)
+               : proj_t<float>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, walls);
   if (rc) return rc;
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   const double words = (do_vel && do_pr) ? 9.0 : do_vel ? 7.0 : 3.0;
   prof_end(c, st, ev, words * N * c->esize);
+  return C3D_OK;
+}
+
+int launch_proj(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
+                int do_pr, int ghost_from_interior) {
+  return proj(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, false);
+}
+
+int launch_proj_walls(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr) {
+  return proj(c, phi, ux, uy, uz, pr, 1, 1, 1, true);
+}
+
+template <typename T>
+static int diag_close_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
+                        int cfl_slot) {
+  const Geom& g = c->g;
+  const int nb = ncell_blocks(g, KCHD);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(BX, BY), 0, c->stream, g, mets<T>(c), (T)c->rdx,
+                       (T)c->rdz, (const T*)ux, (const T*)uy, (const T*)uz,
+                       (const double*)c->d_dyp, c->d_partials, nb, c->d_sc, cfl_slot);
+  };
+  if (what == 7) launch(k_diag<T, 7, true>);
+  else launch(k_diag<T, 5, true>);
+  C3D_HIP(hipGetLastError());
+  return C3D_OK;
+}
+
+int launch_diag_close(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
+                      int cfl_slot) {
+  hipEvent_t ev;
+  prof_begin(c, ST_DIAG, &ev);
+  int rc = c->prec == C3D_FP64 ? diag_close_t<double>(c, ux, uy, uz, what, cfl_slot)
+                               : diag_close_t<float>(c, ux, uy, uz, what, cfl_slot);
+  if (rc) return rc;
+  prof_end(c, ST_DIAG, ev, 3.0 * (double)c->g.nx * c->g.ny * c->g.nz * c->esize);
   return C3D_OK;
 }
 
@@ -895,7 +1059,7 @@ static int diag_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, in
 #define DIAG_LAUNCH(W)                                                                           \
   hipLaunchKernelGGL((k_diag<T, W>), dgrid, dim3(BX, BY), 0, c->stream, g, mets<T>(c),           \
                      (T)c->rdx, (T)c->rdz, (const T*)ux, (const T*)uy, (const T*)uz, dyp,        \
-                     c->d_partials, nb)
+                     c->d_partials, nb, c->d_sc, cfl_slot)
   switch (what) {
     case 1: DIAG_LAUNCH(1); break;
     case 2: DIAG_LAUNCH(2); break;

@@ -82,7 +82,8 @@ __device__ __forceinline__ double block_max4(double v, double* sh) {
 // clcRhsXYZ (m_TScheme.f90:189-438, the branch without scalar or particle
 // coupling).  RhsX (:243-290), RhsY (:293-330), RhsZ (:333-370); with
 // want_flow the block partial of s3tot = sum (d11+d33+d22) dyp (:271) is
-// accumulated as reproducible fixed-point limbs.
+// accumulated as reproducible fixed-point limbs (2: into the fused substep's
+// slots).
 //
 // A wavefront owns 64 x cells of one row and marches a run of z planes.
 //  - z: every value along the own column (u, v, w, p, uy one row up, and the
@@ -113,7 +114,8 @@ __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef
                                                    T* __restrict__ rx, T* __restrict__ ry,
                                                    T* __restrict__ rz, T* __restrict__ hx,
                                                    T* __restrict__ hy, T* __restrict__ hz,
-                                                   double* __restrict__ partials, int want_flow,
+                                                   double* __restrict__ partials,
+                                                   DevScalars* sc, int want_flow,
                                                    int kchunk) {
   __shared__ long long shf[8][4];
   enum { RU, RV, RW, RP, RVP, RUM, RIZ, RW2, NROW };
@@ -392,8 +394,12 @@ __global__ __launch_bounds__(B4X* B4Y, 2) void k_rhs4(Geom g, Metrics<T> m, Coef
   if (want_flow) {
     block_fix4(s3, shf);
     if (threadIdx.x == 0 && threadIdx.y == 0) {
-      long long* pf = (long long*)partials + 4LL * blockIdx.x;
-      for (int q = 0; q < 4; ++q) pf[q] = s3[q];
+      if (want_flow == 2) {
+        bulk_add(sc, s3);
+      } else {
+        long long* pf = (long long*)partials + 4LL * blockIdx.x;
+        for (int q = 0; q < 4; ++q) pf[q] = s3[q];
+      }
     }
   }
 }
@@ -445,8 +451,12 @@ __global__ void k_sub_dp1ns(Geom g, T* __restrict__ f, const DevScalars* sc) {
 // clcPrSrc (m_TScheme.f90:114-143) and CheckDivergence (m_Tools.f90:54-81):
 // div = Dx4 ux + (uy(j+1)-uy(j)) rdyp + Dz4 uz; WRITE stores prsrc = div/pmAlpha
 // ---------------------------------------------------------------------------
-template <typename T, bool WRITE>
+// MAXTO: the workgroups raise the slots of `word` instead of writing partials.  WALLS: uy on
+// the walls is vym / vyp whatever its rows hold (the substep's
+// SetBC_and_UpdateHaloForPrSrc).
+template <typename T, bool WRITE, bool MAXTO, bool WALLS>
 __global__ __launch_bounds__(B4X* B4Y) void k_div4(Geom g, Metrics<T> m, Coef4<T> cf, T sudtal,
+                                                   T vym, T vyp, DevScalars* sc, int word,
                                                    const T* __restrict__ ux_, const T* __restrict__ uy_,
                                                    const T* __restrict__ uz_, T* __restrict__ prsrc,
                                                    double* __restrict__ partials) {
@@ -460,7 +470,12 @@ __global__ __launch_bounds__(B4X* B4Y) void k_div4(Geom g, Metrics<T> m, Coef4<T
     for (int k = k0; k < k1; ++k) {
       const T dudx = cf.dx1 * ux(i - 1, jc, k) + cf.dx2 * ux(i, jc, k) + cf.dx3 * ux(i + 1, jc, k) +
                      cf.dx4 * ux(i + 2, jc, k);
-      const T dvdy = (uy(i, jc + 1, k) - uy(i, jc, k)) * sucaj;
+      T v0 = uy(i, jc, k), v1 = uy(i, jc + 1, k);
+      if (WALLS) {
+        v0 = jc == 1 ? vym : v0;
+        v1 = jc == g.ny ? vyp : v1;
+      }
+      const T dvdy = (v1 - v0) * sucaj;
       const T dwdz = cf.dz1 * uz(i, jc, k - 1) + cf.dz2 * uz(i, jc, k) + cf.dz3 * uz(i, jc, k + 1) +
                      cf.dz4 * uz(i, jc, k + 2);
       const T rdiv = dudx + dvdy + dwdz;
@@ -469,10 +484,14 @@ __global__ __launch_bounds__(B4X* B4Y) void k_div4(Geom g, Metrics<T> m, Coef4<T
     }
   }
   const double r = block_max4(dm, sh);
-  if (threadIdx.x == 0 && threadIdx.y == 0) partials[blockIdx.x] = r;
+  if (threadIdx.x == 0 && threadIdx.y == 0) {
+    if (MAXTO) raise_max(sc, word, r);
+    else partials[blockIdx.x] = r;
+  }
 }
 
-__global__ void k_max4_finalize(const double* __restrict__ partials, int n, double* out) {
+__global__ void k_max4_finalize(const double* __restrict__ partials, int n, double* out,
+                                DevScalars* sc, int word) {
   __shared__ double sh[1024];
   const int t = threadIdx.x;
   double s = 0.0;
@@ -483,7 +502,10 @@ __global__ void k_max4_finalize(const double* __restrict__ partials, int n, doub
     if (t < w) sh[t] = fmax(sh[t], sh[t + w]);
     __syncthreads();
   }
-  if (t == 0) *out = sh[0];
+  if (t == 0) {
+    *out = sh[0];
+    drop_max(sc, word);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -492,9 +514,18 @@ __global__ void k_max4_finalize(const double* __restrict__ partials, int n, doub
 // Neumann ghosts of SetBC_and_UpdateHalo_pr (phi(0)=phi(1),
 // phi(nyp)=phi(nyc)) are applied on the fly.
 // ---------------------------------------------------------------------------
-template <typename T, bool VEL, bool PRS, bool GHOST>
+// WALLS: the ghosts that SetBC_and_UpdateHalo (4th, m_BC_and_Halo.f90:51-96) and
+// SetBC_and_UpdateHalo_pr would set, written by rows 1 and ny from their new
+// values instead of by two more launches.
+struct WallBC4 {
+  int channel;                       // 1: FT_CH, 0: FT_HC
+  double uxm, uzm, uxp, uyp, uzp;    // wall values (ym / yp)
+};
+
+template <typename T, bool VEL, bool PRS, bool GHOST, bool WALLS = false>
 __global__ __launch_bounds__(B4X* B4Y) void k_proj4(Geom g, Metrics<T> m, Coef4<T> cf, T alpha,
-                                                    T beta, const T* __restrict__ phi_,
+                                                    T beta, WallBC4 wb,
+                                                    const T* __restrict__ phi_,
                                                     T* __restrict__ ux, T* __restrict__ uy,
                                                     T* __restrict__ uz, T* __restrict__ pr) {
   CELL4_BLOCK(K4CH);
@@ -514,13 +545,29 @@ __global__ __launch_bounds__(B4X* B4Y) void k_proj4(Geom g, Metrics<T> m, Coef4<
       const T dpdy = (pc - pm) * sucac;
       const T dpdz = cf.dz1 * ph(i, jc, k - 2) + cf.dz2 * ph(i, jc, k - 1) + cf.dz3 * pc +
                      cf.dz4 * ph(i, jc, k + 1);
-      ux[c] = ux[c] - alpha * dpdx;
-      uy[c] = uy[c] - alpha * dpdy;
-      uz[c] = uz[c] - alpha * dpdz;
+      const T un = ux[c] - alpha * dpdx, wn = uz[c] - alpha * dpdz;
+      T vn = uy[c] - alpha * dpdy;
+      if (WALLS && jc == g.ny) {
+        const long long t = c + g.nx;
+        ux[t] = wb.channel ? (T)wb.uxp * T(2) - un : un;
+        uy[t] = wb.channel ? (T)wb.uyp : T(0);
+        uz[t] = wb.channel ? (T)wb.uzp * T(2) - wn : wn;
+      }
+      if (WALLS && jc == 1) {
+        ux[c - g.nx] = (T)wb.uxm * T(2) - un;
+        vn = T(0);  // uy_ym of the 4th-order code
+        uz[c - g.nx] = (T)wb.uzm * T(2) - wn;
+      }
+      ux[c] = un;
+      uy[c] = vn;
+      uz[c] = wn;
     }
     if (PRS) {
       const T pp = (GHOST && jc == g.ny) ? pc : ph(i, jc + 1, k);
-      pr[c] = pr[c] + pmBetap * pp + pmBetac * pc + pmBetam * pm;
+      const T pn = pr[c] + pmBetap * pp + pmBetac * pc + pmBetam * pm;
+      if (WALLS && jc == 1) pr[c - g.nx] = pn;
+      if (WALLS && jc == g.ny) pr[c + g.nx] = pn;
+      pr[c] = pn;
     }
   }
 }
@@ -530,11 +577,6 @@ __global__ __launch_bounds__(B4X* B4Y) void k_proj4(Geom g, Metrics<T> m, Coef4<
 // SetBC_and_UpdateHalo (:51-96), full=0 SetBC_and_UpdateHaloForPrSrc
 // (:101-134).  Channel (no-slip top) or half channel (free-slip top).
 // ---------------------------------------------------------------------------
-struct WallBC4 {
-  int channel;                       // 1: FT_CH, 0: FT_HC
-  double uxm, uzm, uxp, uyp, uzp;    // wall values (ym / yp)
-};
-
 template <typename T>
 __global__ void k_bc4_vel(Geom g, WallBC4 b, T* __restrict__ ux, T* __restrict__ uy,
                           T* __restrict__ uz, const T* __restrict__ uy_ym, int full) {
@@ -603,16 +645,16 @@ static int rhs4_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, co
   const int kc = march_kchunk((long long)((g.nx + B4X - 1) / B4X) * ((g.ny + B4Y - 1) / B4Y * B4Y),
                               g.nz, 4);
   const int nb = nblocks4(g, kc);
-  if (want_flow && 4 * nb > c->max_partials) {
+  if (want_flow == 1 && 4 * nb > c->max_partials) {
     set_error("rhs4: partial buffer too small");
     return C3D_ERR_ARG;
   }
   hipLaunchKernelGGL((k_rhs4<T>), dim3(nb), dim3(B4X, B4Y), 0, c->stream, g, mets4<T>(c),
                      make_coef4<T>(c), (const double*)c->d_dyp, (const T*)ux, (const T*)uy,
                      (const T*)uz, (const T*)pr, (T*)rx, (T*)ry, (T*)rz, (T*)hx, (T*)hy, (T*)hz,
-                     c->d_partials, want_flow, kc);
+                     c->d_partials, c->d_sc, want_flow, kc);
   C3D_HIP(hipGetLastError());
-  if (want_flow) {
+  if (want_flow == 1) {
     hipLaunchKernelGGL(k_flow4_finalize, dim3(1), dim3(1024), 0, c->stream, c->d_partials, nb,
                        c->d_sc, c->p.xnu, (double)(g.nx * g.nz), c->p.yly, c->pmAlpha, c->pmAlphaC,
                        c->cur_ns == 1);
@@ -646,62 +688,94 @@ int launch_sub_dp1ns(c3d_ctx* c, void* rx) {
   return C3D_OK;
 }
 
-template <typename T, bool WRITE>
+// word: the slots that max |div| goes to (raise), or whose plain field it goes to
+template <typename T, bool WRITE, bool WALLS>
 static int div4_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* prsrc,
-                  T sudtal, double* out) {
+                  T sudtal, int word, bool raise) {
   const Geom& g = c->g;
   const int nb = nblocks4(g, 4 * K4CH);
-  if (nb > c->max_partials) {
+  if (!raise && nb > c->max_partials) {
     set_error("div4: partial buffer too small");
     return C3D_ERR_ARG;
   }
-  hipLaunchKernelGGL((k_div4<T, WRITE>), dim3(nb), dim3(B4X, B4Y), 0, c->stream, g, mets4<T>(c),
-                     make_coef4<T>(c), sudtal, (const T*)ux, (const T*)uy, (const T*)uz, (T*)prsrc,
-                     c->d_partials);
+  const T vyp = (T)(c->p.bc[3] == C3D_BC_NOSLIP ? c->p.uybc[3] : 0.0);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(nb), dim3(B4X, B4Y), 0, c->stream, g, mets4<T>(c),
+                       make_coef4<T>(c), sudtal, T(0), vyp, c->d_sc, word, (const T*)ux, (const T*)uy,
+                       (const T*)uz, (T*)prsrc, c->d_partials);
+  };
+  if (raise) {
+    launch(k_div4<T, WRITE, true, WALLS>);
+    C3D_HIP(hipGetLastError());
+    return C3D_OK;
+  }
+  launch(k_div4<T, WRITE, false, WALLS>);
   C3D_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_max4_finalize, dim3(1), dim3(1024), 0, c->stream, c->d_partials, nb, out);
+  hipLaunchKernelGGL(k_max4_finalize, dim3(1), dim3(1024), 0, c->stream, c->d_partials, nb,
+                     word == RED_DIV1 ? &c->d_sc->divmax1 : &c->d_sc->divmax2, c->d_sc, word);
   C3D_HIP(hipGetLastError());
   return C3D_OK;
 }
 
 int launch_prsrc4(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* prsrc,
-                  double alpha_override) {
+                  double alpha_override, bool walls) {
   hipEvent_t ev;
   prof_begin(c, ST_PRSRC, &ev);
   const double alpha = alpha_override > 0.0 ? alpha_override : c->pmAlpha;
-  double* out = &((DevScalars*)c->d_sc)->divmax1;
-  int rc = c->prec == C3D_FP64
-               ? div4_t<double, true>(c, ux, uy, uz, prsrc, 1.0 / alpha, out)
-               : div4_t<float, true>(c, ux, uy, uz, prsrc, (float)(1.0 / alpha), out);
+  const int out = RED_DIV1;
+  int rc;
+  if (c->prec == C3D_FP64)
+    rc = walls ? div4_t<double, true, true>(c, ux, uy, uz, prsrc, 1.0 / alpha, out, true)
+               : div4_t<double, true, false>(c, ux, uy, uz, prsrc, 1.0 / alpha, out, false);
+  else
+    rc = walls ? div4_t<float, true, true>(c, ux, uy, uz, prsrc, (float)(1.0 / alpha), out, true)
+               : div4_t<float, true, false>(c, ux, uy, uz, prsrc, (float)(1.0 / alpha), out, false);
   if (rc) return rc;
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   prof_end(c, ST_PRSRC, ev, 4.0 * N * c->esize);
   return C3D_OK;
 }
 
-int launch_div4(c3d_ctx* c, const void* ux, const void* uy, const void* uz) {
+int launch_div4(c3d_ctx* c, const void* ux, const void* uy, const void* uz, bool closing) {
   hipEvent_t ev;
   prof_begin(c, ST_DIAG, &ev);
-  double* out = &((DevScalars*)c->d_sc)->divmax2;
-  int rc = c->prec == C3D_FP64 ? div4_t<double, false>(c, ux, uy, uz, nullptr, 0.0, out)
-                               : div4_t<float, false>(c, ux, uy, uz, nullptr, 0.f, out);
+  const int out = RED_DIV2;
+  int rc = c->prec == C3D_FP64
+               ? div4_t<double, false, false>(c, ux, uy, uz, nullptr, 0.0, out, closing)
+               : div4_t<float, false, false>(c, ux, uy, uz, nullptr, 0.f, out, closing);
   if (rc) return rc;
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   prof_end(c, ST_DIAG, ev, 3.0 * N * c->esize);
   return C3D_OK;
 }
 
+static WallBC4 make_wallbc4(const c3d_ctx* c) {
+  WallBC4 b;
+  b.channel = c->p.bc[3] == C3D_BC_NOSLIP ? 1 : 0;
+  b.uxm = c->p.uxbc[2];
+  b.uzm = c->p.uzbc[2];
+  b.uxp = c->p.uxbc[3];
+  b.uyp = c->p.uybc[3];
+  b.uzp = c->p.uzbc[3];
+  return b;
+}
+
 template <typename T>
 static int proj4_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int vel,
-                   int prs, int ghost) {
+                   int prs, int ghost, bool walls) {
   const Geom& g = c->g;
+  const WallBC4 wb = make_wallbc4(c);
   const dim3 grid(nblocks4(g, K4CH)), blk(B4X, B4Y);
   const T alpha = (T)c->pmAlpha, beta = (T)c->pmBeta;
   const Coef4<T> cf = make_coef4<T>(c);
 #define PROJ4(V, P, G)                                                                          \
   hipLaunchKernelGGL((k_proj4<T, V, P, G>), grid, blk, 0, c->stream, g, mets4<T>(c), cf, alpha, \
-                     beta, (const T*)phi, (T*)ux, (T*)uy, (T*)uz, (T*)pr)
-  if (vel && prs) {
+                     beta, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz, (T*)pr)
+  if (walls) {
+    hipLaunchKernelGGL((k_proj4<T, true, true, true, true>), grid, blk, 0, c->stream, g,
+                       mets4<T>(c), cf, alpha, beta, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,
+                       (T*)pr);
+  } else if (vel && prs) {
     if (ghost) PROJ4(true, true, true); else PROJ4(true, true, false);
   } else if (vel) {
     if (ghost) PROJ4(true, false, true); else PROJ4(true, false, false);
@@ -713,15 +787,15 @@ static int proj4_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, vo
   return C3D_OK;
 }
 
-int launch_proj4(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
-                 int do_pr, int ghost_from_interior) {
+static int proj4(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
+                 int do_pr, int ghost_from_interior, bool walls) {
   if (!do_vel && !do_pr) return C3D_OK;
   const int st = (do_vel && do_pr) ? ST_PROJ : do_vel ? ST_VELUPD : ST_PRUPD;
   hipEvent_t ev;
   prof_begin(c, st, &ev);
   int rc = c->prec == C3D_FP64
-               ? proj4_t<double>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior)
-               : proj4_t<float>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior);
+               ? proj4_t<double>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, walls)
+               : proj4_t<float>(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, walls);
   if (rc) return rc;
   const double N = (double)c->g.nx * c->g.ny * c->g.nz;
   const double words = (do_vel && do_pr) ? 9.0 : do_vel ? 7.0 : 3.0;
@@ -729,15 +803,18 @@ int launch_proj4(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void
   return C3D_OK;
 }
 
+int launch_proj4(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr, int do_vel,
+                 int do_pr, int ghost_from_interior) {
+  return proj4(c, phi, ux, uy, uz, pr, do_vel, do_pr, ghost_from_interior, false);
+}
+
+int launch_proj4_walls(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr) {
+  return proj4(c, phi, ux, uy, uz, pr, 1, 1, 1, true);
+}
+
 int launch_bc4_vel(c3d_ctx* c, void* ux, void* uy, void* uz, const void* uy_ym, int full) {
   const Geom& g = c->g;
-  WallBC4 b;
-  b.channel = c->p.bc[3] == C3D_BC_NOSLIP ? 1 : 0;
-  b.uxm = c->p.uxbc[2];
-  b.uzm = c->p.uzbc[2];
-  b.uxp = c->p.uxbc[3];
-  b.uyp = c->p.uybc[3];
-  b.uzp = c->p.uzbc[3];
+  const WallBC4 b = make_wallbc4(c);
   hipEvent_t ev;
   prof_begin(c, ST_BC, &ev);
   const dim3 grid((g.nx + 255) / 256, g.nz), blk(256);
