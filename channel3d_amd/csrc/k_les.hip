@@ -763,11 +763,11 @@ __global__ __launch_bounds__(LBX* LBY) void k_prupd_les(Geom g, Metrics<T> m, T 
 // 0.235 + 0.143 + 0.016 ms at 384x192x288, now 0.354 ms; 5 launches fewer a
 // substep at 96x96x72.
 // ---------------------------------------------------------------------------
-constexpr int PLKCH = 16;
+constexpr int PLKCH = 16;  // longest z run
 
 template <typename T, bool NTS>
 __global__ __launch_bounds__(LBX* LBY) void k_proj_les(Geom g, Metrics<T> m, T rdxE, T rdzE,
-                                                       T alpha, T bt, WallBC wb,
+                                                       T alpha, T bt, WallBC wb, int kchunk,
                                                        const T* __restrict__ nut,
                                                        const T* __restrict__ phi,
                                                        T* __restrict__ ux, T* __restrict__ uy,
@@ -777,7 +777,7 @@ __global__ __launch_bounds__(LBX* LBY) void k_proj_les(Geom g, Metrics<T> m, T r
   const int i = (lb % gxb) * LBX + threadIdx.x;
   const int jc = ((lb / gxb) % gyb) * LBY + threadIdx.y + 1;
   if (i >= g.nx || jc > g.ny) return;
-  const int k0 = (lb / (gxb * gyb)) * PLKCH, k1 = min(g.nz, k0 + PLKCH);
+  const int k0 = (lb / (gxb * gyb)) * kchunk, k1 = min(g.nz, k0 + kchunk);
   const int im = wm(i, g.nx);
   const T sucac = m.rdyc[jc] * alpha;
   const T metr1 = m.rdyp[jc] * m.rdyc[jc], metr2 = m.rdyp[jc] * m.rdyc[jc + 1];
@@ -1029,13 +1029,16 @@ int launch_les_y3(c3d_ctx* c, void* const u[3], void* const rhs[3], const void* 
 template <typename T>
 static int proj_les_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr) {
   const Geom& g = c->g;
-  const dim3 grid(((g.nx + LBX - 1) / LBX) * ((g.ny + LBY - 1) / LBY) *
-                  ((g.nz + PLKCH - 1) / PLKCH)),
-      blk(LBX, LBY);
+  // down to two planes a run until every CU has four workgroups (the rule of the
+  // second-order projection)
+  const int tiles = ((g.nx + LBX - 1) / LBX) * ((g.ny + LBY - 1) / LBY);
+  int kc = PLKCH;
+  while (kc > 2 && tiles * ((g.nz + kc - 1) / kc) < 1024) kc /= 2;
+  const dim3 grid(tiles * ((g.nz + kc - 1) / kc)), blk(LBX, LBY);
   auto launch = [&](auto ntc) {
     hipLaunchKernelGGL((k_proj_les<T, decltype(ntc)::value>), grid, blk, 0, c->stream, g, met<T>(c),
                        (T)(c->rdx * c->pmAlpha), (T)(c->rdz * c->pmAlpha), (T)c->pmAlpha,
-                       (T)c->pmBetaT, make_wallbc(c), (const T*)c->state[C3D_NUT], (const T*)phi,
+                       (T)c->pmBetaT, make_wallbc(c), kc, (const T*)c->state[C3D_NUT], (const T*)phi,
                        (T*)ux, (T*)uy, (T*)uz, (T*)pr);
   };
   if (g.nt) launch(std::true_type{});

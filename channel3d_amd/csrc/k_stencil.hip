@@ -13,7 +13,7 @@
 namespace c3d {
 
 constexpr int BX = 64, BY = 4, KCH = 8;
-constexpr int KCHD = 64;  // z run of the diagnostics (fewer partials to combine)
+constexpr int KCHD = 64;  // longest z run of the diagnostics (fewer partials to combine)
 
 template <typename T>
 struct Fld {
@@ -492,7 +492,7 @@ __global__ void k_update_uy_ym(int n, T uybc, T* __restrict__ uy_ym, T* __restri
 // (m_TSchemeFIMP_inc.f90:1371-1386).  With ghost_from_interior the Neumann
 // ghost phi(0)=phi(1) of SetBC_and_UpdateHalo_pr is applied on the fly.
 //
-// A thread walks a run of PKCH z planes of its (i, j) column.  Plane k+1's
+// A thread walks a run of up to PKCH z planes of its (i, j) column.  Plane k+1's
 // words are requested before plane k's results are stored (the hardware
 // counts loads and stores on one counter, so a load issued after a store
 // cannot be waited for without also waiting for the store), and every load
@@ -508,7 +508,8 @@ constexpr int PKCH = 16;
 
 template <typename T, bool VEL, bool PRS, bool GHOST, bool NTS = false, bool WALLS = false>
 __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2, T rdzEta2,
-                                                 T alpha, WallBC wb, const T* __restrict__ phi,
+                                                 T alpha, WallBC wb, int kchunk,
+                                                 const T* __restrict__ phi,
                                                  T* __restrict__ ux, T* __restrict__ uy,
                                                  T* __restrict__ uz, T* __restrict__ pr) {
   CELL_BLOCK();
@@ -517,7 +518,7 @@ __global__ __launch_bounds__(BX* BY) void k_proj(Geom g, Metrics<T> m, T rdxEta2
   if (i >= g.nx || jc > g.ny) return;
   const int im = wrapm(i, g.nx);
   const T sucacEta2 = m.rdyc[jc] * alpha;
-  const int k0 = cbz * PKCH, k1 = min(g.nz, k0 + PKCH);
+  const int k0 = cbz * kchunk, k1 = min(g.nz, k0 + kchunk);
   const long long row = (long long)g.nx * jc;
   struct Plane {
     T ph, phx, phy, u, v, w, p;
@@ -602,7 +603,7 @@ __global__ __launch_bounds__(BX* BY) void k_diag(Geom g, Metrics<T> m, T rdx, T 
                                                  const T* __restrict__ uz,
                                                  const double* __restrict__ dyp,
                                                  double* __restrict__ partials, int nblocks,
-                                                 DevScalars* sc, int cfl_slot) {
+                                                 DevScalars* sc, int cfl_slot, int kchunk) {
   __shared__ double sh[8];
   CELL_BLOCK();
   const int i = cbx * BX + threadIdx.x;
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(BX* BY) void k_diag(Geom g, Metrics<T> m, T rdx, T 
     const int ip = wrapp(i, g.nx);
     const T rdyp = m.rdyp[jc];
     const double dy = dyp[jc];
-    const int k0 = cbz * KCHD, k1 = min(g.nz, (cbz + 1) * KCHD);
+    const int k0 = cbz * kchunk, k1 = min(g.nz, k0 + kchunk);
     // uz one plane up is the next plane's own value; unrolled so that
     // several planes' loads are in flight together
     T w = uz[(long long)g.nx * jc + g.plane * k0 + i];
@@ -720,6 +721,16 @@ __global__ void k_diag_finalize(const double* __restrict__ partials, int n, int 
 // ===========================================================================
 static inline int ncell_blocks(const Geom& g, int kch = KCH) {
   return ((g.nx + BX - 1) / BX) * ((g.ny + BY - 1) / BY) * ((g.nz + kch - 1) / kch);
+}
+// z run of a pass over the cells: `longest` planes, halved down to `shortest`
+// until every CU has four workgroups.  A longer run re-reads fewer lead-in
+// planes, which is worth nothing while CUs idle (64^3, one tile of 16 rows a
+// plane: projection 14.5 us with 16 planes, 8.7 with 2; closing diagnostics 19 us
+// with 64, 6.9 with 2); from 1024 workgroups on the lengths are the longest ones.
+static inline int short_kchunk(const Geom& g, int longest, int shortest) {
+  int kc = longest;
+  while (kc / 2 >= shortest && ncell_blocks(g, kc) < 1024) kc /= 2;
+  return kc;
 }
 static inline dim3 cell_grid(const Geom& g) { return dim3(ncell_blocks(g)); }
 
@@ -974,20 +985,21 @@ static int proj_t(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, voi
   const WallBC wb = make_wallbc(c);
   const T a = (T)c->pmAlpha;
   const T rdxE = (T)(c->rdx * c->pmAlpha), rdzE = (T)(c->rdz * c->pmAlpha);
-  const dim3 grid(ncell_blocks(g, PKCH));
+  const int kc = short_kchunk(g, PKCH, 2);
+  const dim3 grid(ncell_blocks(g, kc));
 #define PROJ_LAUNCH(V, P, G)                                                                   \
   if (g.nt)                                                                                    \
     hipLaunchKernelGGL((k_proj<T, V, P, G, true>), grid, dim3(BX, BY), 0, c->stream, g,        \
-                       mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,  \
-                       (T*)pr);                                                                \
+                       mets<T>(c), rdxE, rdzE, a, wb, kc, (const T*)phi, (T*)ux, (T*)uy,      \
+                       (T*)uz, (T*)pr);                                                                \
   else                                                                                         \
     hipLaunchKernelGGL((k_proj<T, V, P, G, false>), grid, dim3(BX, BY), 0, c->stream, g,       \
-                       mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy, (T*)uz,  \
-                       (T*)pr)
+                       mets<T>(c), rdxE, rdzE, a, wb, kc, (const T*)phi, (T*)ux, (T*)uy,      \
+                       (T*)uz, (T*)pr)
   if (walls) {
     hipLaunchKernelGGL((k_proj<T, true, true, true, false, true>), grid, dim3(BX, BY), 0,
-                       c->stream, g, mets<T>(c), rdxE, rdzE, a, wb, (const T*)phi, (T*)ux, (T*)uy,
-                       (T*)uz, (T*)pr);
+                       c->stream, g, mets<T>(c), rdxE, rdzE, a, wb, kc, (const T*)phi, (T*)ux,
+                       (T*)uy, (T*)uz, (T*)pr);
   } else if (vel && prs && ghost) PROJ_LAUNCH(true, true, true);
   else if (vel && prs) PROJ_LAUNCH(true, true, false);
   else if (vel && ghost) PROJ_LAUNCH(true, false, true);
@@ -1026,11 +1038,11 @@ template <typename T>
 static int diag_close_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
                         int cfl_slot) {
   const Geom& g = c->g;
-  const int nb = ncell_blocks(g, KCHD);
+  const int kc = short_kchunk(g, KCHD, 2), nb = ncell_blocks(g, kc);
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(nb), dim3(BX, BY), 0, c->stream, g, mets<T>(c), (T)c->rdx,
                        (T)c->rdz, (const T*)ux, (const T*)uy, (const T*)uz,
-                       (const double*)c->d_dyp, c->d_partials, nb, c->d_sc, cfl_slot);
+                       (const double*)c->d_dyp, c->d_partials, nb, c->d_sc, cfl_slot, kc);
   };
   if (what == 7) launch(k_diag<T, 7, true>);
   else launch(k_diag<T, 5, true>);
@@ -1053,13 +1065,14 @@ template <typename T>
 static int diag_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, int what,
                   int cfl_slot) {
   const Geom& g = c->g;
-  const int nb = ncell_blocks(g, KCHD);
+  // at least KCH planes a run: the partials were allocated for that many blocks
+  const int kc = short_kchunk(g, KCHD, KCH), nb = ncell_blocks(g, kc);
   const dim3 dgrid(nb);
   const double* dyp = c->d_dyp;
 #define DIAG_LAUNCH(W)                                                                           \
   hipLaunchKernelGGL((k_diag<T, W>), dgrid, dim3(BX, BY), 0, c->stream, g, mets<T>(c),           \
                      (T)c->rdx, (T)c->rdz, (const T*)ux, (const T*)uy, (const T*)uz, dyp,        \
-                     c->d_partials, nb, c->d_sc, cfl_slot)
+                     c->d_partials, nb, c->d_sc, cfl_slot, kc)
   switch (what) {
     case 1: DIAG_LAUNCH(1); break;
     case 2: DIAG_LAUNCH(2); break;
