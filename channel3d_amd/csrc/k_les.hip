@@ -95,143 +95,219 @@ __device__ __forceinline__ void nut_ghosts(const Geom& g, const LesCoef<T>& q, T
 }
 
 // ---------------------------------------------------------------------------
-// Clc_SGS_WALE (m_LESModels.f90:72-135)
+// Clc_SGS_WALE (m_LESModels.f90:72-135); Clc_SGS_MTS (:145-258) with
+// ClcVelStrainRate (:328-370).
+//
+// A workgroup owns 64 x 4 cells and marches a run of z planes.  Each plane of
+// u, v, w over the tile plus its halo (one cell, two above in x for the test
+// filter) passes once through LDS, two buffers in turn, requested a plane ahead;
+// the values at the planes a cell still needs stay in registers, so a plane
+// costs 19 LDS reads a thread.  The uz plane staged is one further up for MTS
+// (LZ = 2), whose residual on the face k+1 reaches k+2; that residual is the next
+// cell's at k, and the one quantity kept.  The squared residuals the reference
+// stores in Ktemp are formed by each cell for its other faces (same operands,
+// same operations).  Bound: HBM, 4 words per cell.
+// With every operand fetched on its own (MTS: over 90 loads a cell, both
+// residuals of each component from memory) MTS took 0.724 ms at 384x192x288,
+// WALE 0.026 ms at 96x96x72; now 0.284 (2.4 TB/s; FP64 latency of the square
+// roots and divisions at three wavefronts per SIMD is what remains) and 0.018 ms.
 // ---------------------------------------------------------------------------
 template <typename T>
-__global__ __launch_bounds__(LBX* LBY) void k_sgs_wale(Geom g, Metrics<T> m, LesMet<T> lm,
-                                                       LesCoef<T> q, const T* __restrict__ ux,
-                                                       const T* __restrict__ uy,
-                                                       const T* __restrict__ uz,
-                                                       T* __restrict__ nut) {
-  LES_CELL();
-  if (i >= g.nx || jc > g.ny) return;
-  const int nx = g.nx, nyh = g.nyh;
-  const int im = wm(i, nx), ip = wp(i, nx);
-  const int jm = jc - 1, jp = jc + 1;
-  const T caj = m.rdyp[jc];
-  const T cac1 = m.rdyc[jc];
-  const T cac2 = m.rdyc[jp];
-  const T cac12 = cac1 - cac2;
-  T CwDelta2 = T(0.325) * lm.delta[jc];
-  CwDelta2 = CwDelta2 * CwDelta2;
-  const T rdx = q.rdx, rdz = q.rdz;
-  for (int k = kz0; k < kz1; ++k) {
-    const int km = wm(k, g.nz), kp = wp(k, g.nz);
-    const T dudx = (A(ux, ip, jc, k) - A(ux, i, jc, k)) * rdx;
-    const T dudy = ((A(ux, ip, jp, k) + A(ux, i, jp, k)) * cac2 +
-                    (A(ux, ip, jc, k) + A(ux, i, jc, k)) * cac12 -
-                    (A(ux, ip, jm, k) + A(ux, i, jm, k)) * cac1) * T(0.25);
-    const T dudz = (A(ux, ip, jc, kp) + A(ux, i, jc, kp) - A(ux, ip, jc, km) - A(ux, i, jc, km)) *
-                   rdz * T(0.25);
-    const T dvdx = (A(uy, ip, jp, k) - A(uy, im, jp, k) + A(uy, ip, jc, k) - A(uy, im, jc, k)) *
-                   rdx * T(0.25);
-    const T dvdy = (A(uy, i, jp, k) - A(uy, i, jc, k)) * caj;
-    const T dvdz = (A(uy, i, jp, kp) + A(uy, i, jc, kp) - A(uy, i, jp, km) - A(uy, i, jc, km)) *
-                   rdz * T(0.25);
-    const T dwdx = (A(uz, ip, jc, kp) - A(uz, im, jc, kp) + A(uz, ip, jc, k) - A(uz, im, jc, k)) *
-                   rdx * T(0.25);
-    const T dwdy = ((A(uz, i, jp, kp) + A(uz, i, jp, k)) * cac2 +
-                    (A(uz, i, jc, kp) + A(uz, i, jc, k)) * cac12 -
-                    (A(uz, i, jm, kp) + A(uz, i, jm, k)) * cac1) * T(0.25);
-    const T dwdz = (A(uz, i, jc, kp) - A(uz, i, jc, k)) * rdz;
+__device__ __forceinline__ T filt_res(const T* F, const T* a, const T* b, const T* c) {
+  return F[0] * a[0] + F[1] * a[1] + F[2] * a[2] + F[3] * b[0] + F[4] * b[1] + F[5] * b[2] +
+         F[6] * c[0] + F[7] * c[1] + F[8] * c[2];
+}
 
-    const T S11 = dudx;
-    const T S12 = (dudy + dvdx) * T(0.5);
-    const T S13 = (dudz + dwdx) * T(0.5);
-    const T S22 = dvdy;
-    const T S23 = (dvdz + dwdy) * T(0.5);
-    const T S33 = dwdz;
-    const T SijSij = S11 * S11 + S22 * S22 + S33 * S33 + T(2) * (S12 * S12 + S13 * S13 + S23 * S23);
-
-    T Sd11 = dudx * dudx + dudy * dvdx + dudz * dwdx;
-    const T Sd12 = (dudx * dudy + dudy * dvdy + dudz * dwdy + dvdx * dudx + dvdy * dvdx + dvdz * dwdx) * T(0.5);
-    const T Sd13 = (dudx * dudz + dudy * dvdz + dudz * dwdz + dwdx * dudx + dwdy * dvdx + dwdz * dwdx) * T(0.5);
-    T Sd22 = dvdx * dudy + dvdy * dvdy + dvdz * dwdy;
-    const T Sd23 = (dvdx * dudz + dvdy * dvdz + dvdz * dwdz + dwdx * dudy + dwdy * dvdy + dwdz * dwdy) * T(0.5);
-    T Sd33 = dwdx * dudz + dwdy * dvdz + dwdz * dwdz;
-    const T SdTrace = (Sd11 + Sd22 + Sd33) / T(3);
-    Sd11 = Sd11 - SdTrace;
-    Sd22 = Sd22 - SdTrace;
-    Sd33 = Sd33 - SdTrace;
-    const T SdijSdij =
-        Sd11 * Sd11 + Sd22 * Sd22 + Sd33 * Sd33 + T(2) * (Sd12 * Sd12 + Sd13 * Sd13 + Sd23 * Sd23);
-    // the reference's powers (**1.5, **2.5, **1.25) of these non-negative
-    // sums through square roots: x^1.5 = x sqrt(x), x^2.5 = x^2 sqrt(x),
-    // x^1.25 = x sqrt(sqrt(x)), a few ulp from pow at a fraction of its cost
-    const T sdh = sqrt(SdijSdij), sh = sqrt(SijSij);
-    const T v = CwDelta2 * (SdijSdij * sdh) /
-                    (SijSij * SijSij * sh + SdijSdij * sqrt(sdh)) + q.xnu;
-    A(nut, i, jc, k) = v;
-    nut_ghosts(g, q, nut, i, jc, k, v);
+template <typename T, bool MTS>
+__global__ __launch_bounds__(LBX* LBY, 2) void k_sgs(Geom g, Metrics<T> m, LesMet<T> lm,
+                                                     LesCoef<T> q, const T* __restrict__ ux,
+                                                     const T* __restrict__ uy,
+                                                     const T* __restrict__ uz,
+                                                     T* __restrict__ nut, int kchunk) {
+  constexpr int LZ = MTS ? 2 : 1;
+  constexpr int LW = LBX + (MTS ? 3 : 2), LP = LW * (LBY + 2);
+  constexpr int NT = LBX * LBY, NS = (LP + NT - 1) / NT;
+  __shared__ T sb[2][3][LP];
+  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane(threadIdx.y);
+  const int tid = tx + LBX * ty;
+  const int nx = g.nx, ny = g.ny, nz = g.nz;
+  const int gxb = (nx + LBX - 1) / LBX, gyb = (ny + LBY - 1) / LBY;
+  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int i0 = (lb % gxb) * LBX, j0 = ((lb / gxb) % gyb) * LBY + 1;
+  const int k0 = (lb / (gxb * gyb)) * kchunk, k1 = min(nz, k0 + kchunk);
+  // staging slots as in the right-hand sides below
+  unsigned so[NS];
+  bool sl[NS];
+#pragma unroll
+  for (int s = 0; s < NS; ++s) {
+    const int e = tid + NT * s;
+    const int jj = e / LW, ii = e - jj * LW;
+    int i = i0 - 1 + ii;
+    i = i < 0 ? nx - 1 : (i >= nx ? i % nx : i);
+    sl[s] = e < LP;
+    so[s] = sl[s] ? (unsigned)(min(j0 - 1 + jj, ny + 1) * nx + i) * (unsigned)sizeof(T) : 0u;
   }
-}
-
-// ---------------------------------------------------------------------------
-// Clc_SGS_MTS (m_LESModels.f90:145-258) with ClcVelStrainRate (:328-370).
-// The squared test-filter residuals the reference stores in Ktemp are
-// recomputed per cell for both faces (same operands, same operations).
-// ---------------------------------------------------------------------------
-template <typename T>
-__device__ __forceinline__ T filt_res(const Geom& g, const LesCoef<T>& q, const T* u, int i, int j,
-                                      int k) {
-  const int nx = g.nx, nyh = g.nyh;
-  const int im = wm(i, nx), ip = wp(i, nx), km = wm(k, g.nz), kp = wp(k, g.nz);
-  const T* F = q.fc;
-  return F[0] * A(u, im, j, km) + F[1] * A(u, i, j, km) + F[2] * A(u, ip, j, km) +
-         F[3] * A(u, im, j, k) + F[4] * A(u, i, j, k) + F[5] * A(u, ip, j, k) +
-         F[6] * A(u, im, j, kp) + F[7] * A(u, i, j, kp) + F[8] * A(u, ip, j, kp);
-}
-
-template <typename T>
-__global__ __launch_bounds__(LBX* LBY) void k_sgs_mts(Geom g, Metrics<T> m, LesMet<T> lm,
-                                                      LesCoef<T> q, const T* __restrict__ ux,
-                                                      const T* __restrict__ uy,
-                                                      const T* __restrict__ uz,
-                                                      T* __restrict__ nut) {
-  LES_CELL();
-  if (i >= g.nx || jc > g.ny) return;
-  const int nx = g.nx, nyh = g.nyh;
-  const int im = wm(i, nx), ip = wp(i, nx);
-  const int jm = jc - 1, jp = jc + 1;
-  const T caj = m.rdyp[jc];
-  const T cac1 = m.rdyc[jc];
+  T st[3][NS];
+  // ux, uy of plane k+1 and uz of plane k+LZ, periodic
+  auto fetch = [&](int k) {
+    const int ka = (k + 1 + 2 * nz) % nz, kb = (k + LZ + 2 * nz) % nz;
+    const T* const f[3] = {ux + g.plane * ka, uy + g.plane * ka, uz + g.plane * kb};
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int s = 0; s < NS; ++s) st[a][s] = *(const T*)((const char*)f[a] + so[s]);
+  };
+  auto stage = [&](int buf) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+      if (sl[s]) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) sb[buf][a][tid + NT * s] = st[a][s];
+      }
+  };
+  const int jc = j0 + ty, jrow = min(jc, ny), jp = jrow + 1;
+  const int e = (ty + 1) * LW + tx + 1;
+  const int i = i0 + tx;
+  const bool live = i < nx && jc <= ny;
+  const T caj = m.rdyp[jrow];
+  const T cac1 = m.rdyc[jrow];
   const T cac2 = m.rdyc[jp];
   const T cac12 = cac1 - cac2;
-  const T rdelta = lm.rdelta[jc];
   const T rdx = q.rdx, rdz = q.rdz, oneEighth = T(0.125);
-  for (int k = kz0; k < kz1; ++k) {
-    const int km = wm(k, g.nz), kp = wp(k, g.nz);
-    const T st1 = (A(ux, ip, jc, k) - A(ux, i, jc, k)) * rdx;
-    const T st2 = (A(uy, i, jp, k) - A(uy, i, jc, k)) * caj;
-    const T st3 = (A(uz, i, jc, kp) - A(uz, i, jc, k)) * rdz;
-    const T st4 = oneEighth * ((A(uy, ip, jp, k) - A(uy, im, jp, k) + A(uy, ip, jc, k) - A(uy, im, jc, k)) * rdx +
-                               (A(ux, ip, jp, k) + A(ux, i, jp, k)) * cac2 +
-                               (A(ux, ip, jc, k) + A(ux, i, jc, k)) * cac12 -
-                               (A(ux, ip, jm, k) + A(ux, i, jm, k)) * cac1);
-    const T st5 = oneEighth * ((A(ux, ip, jc, kp) + A(ux, i, jc, kp) - A(ux, ip, jc, km) - A(ux, i, jc, km)) * rdz +
-                               (A(uz, ip, jc, kp) - A(uz, im, jc, kp) + A(uz, ip, jc, k) - A(uz, im, jc, k)) * rdx);
-    const T st6 = oneEighth * ((A(uy, i, jp, kp) + A(uy, i, jc, kp) - A(uy, i, jp, km) - A(uy, i, jc, km)) * rdz +
-                               (A(uz, i, jp, kp) + A(uz, i, jp, k)) * cac2 +
-                               (A(uz, i, jc, kp) + A(uz, i, jc, k)) * cac12 -
-                               (A(uz, i, jm, kp) + A(uz, i, jm, k)) * cac1);
-    const T strain =
-        sqrt(T(2) * (st1 * st1 + st2 * st2 + st3 * st3) + T(4) * (st4 * st4 + st5 * st5 + st6 * st6));
-    // Kes: ux residual on the faces i and i+1, uy on the nodes jc and jc+1,
-    // uz on the faces k and k+1 (:159-230)
-    const T rx0 = filt_res(g, q, ux, i, jc, k), rx1 = filt_res(g, q, ux, ip, jc, k);
-    T Kes = T(0.5) * (rx0 * rx0 + rx1 * rx1);
-    const T ry0 = filt_res(g, q, uy, i, jc, k), ry1 = filt_res(g, q, uy, i, jp, k);
-    Kes = Kes + T(0.5) * (ry0 * ry0 + ry1 * ry1);
-    const T rz0 = filt_res(g, q, uz, i, jc, k), rz1 = filt_res(g, q, uz, i, jc, kp);
-    Kes = Kes + T(0.5) * (rz0 * rz0 + rz1 * rz1);
-    T Ts = sqrt(Kes) * rdelta + strain / T(10);
-    if (Ts < T(1.00E-10))
-      Ts = T(0);
-    else
-      Ts = T(1) / Ts;
-    const T v = T(0.05) * Kes * Ts + q.xnu;
-    A(nut, i, jc, k) = v;
-    nut_ghosts(g, q, nut, i, jc, k, v);
+  const T rdelta = MTS ? lm.rdelta[jrow] : T(0);
+  T CwDelta2 = MTS ? T(0) : T(0.325) * lm.delta[jrow];
+  CwDelta2 = CwDelta2 * CwDelta2;
+  // [plane][x]: x = i-1, i, i+1, i+2.  ux and uy: planes k-1, k, k+1; ux on the
+  // rows beside: k, k+1; uz: k, k+1, k+LZ
+  T u[3][4], um[2][2], up[2][2], v[3][3], vp[3][3], w[LZ + 1][3], wm[LZ + 1], wp_[LZ + 1];
+  auto take = [&](int buf) {  // shift by a plane and append the staged one
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+#pragma unroll
+      for (int x = 0; x < 4; ++x) u[p][x] = u[p + 1][x];
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        v[p][x] = v[p + 1][x];
+        vp[p][x] = vp[p + 1][x];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      um[0][x] = um[1][x];
+      up[0][x] = up[1][x];
+    }
+#pragma unroll
+    for (int p = 0; p < LZ; ++p) {
+#pragma unroll
+      for (int x = 0; x < 3; ++x) w[p][x] = w[p + 1][x];
+      wm[p] = wm[p + 1];
+      wp_[p] = wp_[p + 1];
+    }
+    const T* U = sb[buf][0] + e;
+    const T* V = sb[buf][1] + e;
+    const T* W = sb[buf][2] + e;
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      u[2][x] = U[x - 1];
+      v[2][x] = V[x - 1];
+      vp[2][x] = V[LW + x - 1];
+      w[LZ][x] = W[x - 1];
+    }
+    if (MTS) u[2][3] = U[2];
+    um[1][0] = U[-LW]; um[1][1] = U[1 - LW];
+    up[1][0] = U[LW]; up[1][1] = U[1 + LW];
+    wm[LZ] = W[-LW];
+    wp_[LZ] = W[LW];
+  };
+  // the planes below the run
+  for (int k = k0 - LZ - 1; k < k0; ++k) {
+    fetch(k);
+    stage(k & 1);
+    __syncthreads();
+    take(k & 1);
+  }
+  T rz0 = T(0);
+  if (MTS) rz0 = filt_res(q.fc, w[0], w[1], w[LZ]);
+  fetch(k0);
+  stage(k0 & 1);
+  __syncthreads();
+  for (int k = k0; k < k1; ++k) {
+    fetch(k + 1);
+    take(k & 1);
+    const T dudx = (u[1][2] - u[1][1]) * rdx;
+    const T dvdy = (vp[1][1] - v[1][1]) * caj;
+    const T dwdz = (w[1][1] - w[0][1]) * rdz;
+    T nv;
+    if (MTS) {
+      const T st4 = oneEighth * ((vp[1][2] - vp[1][0] + v[1][2] - v[1][0]) * rdx +
+                                 (up[0][1] + up[0][0]) * cac2 + (u[1][2] + u[1][1]) * cac12 -
+                                 (um[0][1] + um[0][0]) * cac1);
+      const T st5 = oneEighth * ((u[2][2] + u[2][1] - u[0][2] - u[0][1]) * rdz +
+                                 (w[1][2] - w[1][0] + w[0][2] - w[0][0]) * rdx);
+      const T st6 = oneEighth * ((vp[2][1] + v[2][1] - vp[0][1] - v[0][1]) * rdz +
+                                 (wp_[1] + wp_[0]) * cac2 + (w[1][1] + w[0][1]) * cac12 -
+                                 (wm[1] + wm[0]) * cac1);
+      const T strain = sqrt(T(2) * (dudx * dudx + dvdy * dvdy + dwdz * dwdz) +
+                            T(4) * (st4 * st4 + st5 * st5 + st6 * st6));
+      // Kes: ux residual on the faces i and i+1, uy on the nodes jc and jc+1,
+      // uz on the faces k and k+1 (:159-230)
+      const T* F = q.fc;
+      const T rx0 = filt_res(F, u[0], u[1], u[2]);
+      const T rx1 = filt_res(F, u[0] + 1, u[1] + 1, u[2] + 1);
+      T Kes = T(0.5) * (rx0 * rx0 + rx1 * rx1);
+      const T ry0 = filt_res(F, v[0], v[1], v[2]), ry1 = filt_res(F, vp[0], vp[1], vp[2]);
+      Kes = Kes + T(0.5) * (ry0 * ry0 + ry1 * ry1);
+      const T rz1 = filt_res(F, w[0], w[1], w[LZ]);
+      Kes = Kes + T(0.5) * (rz0 * rz0 + rz1 * rz1);
+      rz0 = rz1;
+      T Ts = sqrt(Kes) * rdelta + strain / T(10);
+      if (Ts < T(1.00E-10))
+        Ts = T(0);
+      else
+        Ts = T(1) / Ts;
+      nv = T(0.05) * Kes * Ts + q.xnu;
+    } else {
+      const T dudy = ((up[0][1] + up[0][0]) * cac2 + (u[1][2] + u[1][1]) * cac12 -
+                      (um[0][1] + um[0][0]) * cac1) * T(0.25);
+      const T dudz = (u[2][2] + u[2][1] - u[0][2] - u[0][1]) * rdz * T(0.25);
+      const T dvdx = (vp[1][2] - vp[1][0] + v[1][2] - v[1][0]) * rdx * T(0.25);
+      const T dvdz = (vp[2][1] + v[2][1] - vp[0][1] - v[0][1]) * rdz * T(0.25);
+      const T dwdx = (w[1][2] - w[1][0] + w[0][2] - w[0][0]) * rdx * T(0.25);
+      const T dwdy = ((wp_[1] + wp_[0]) * cac2 + (w[1][1] + w[0][1]) * cac12 -
+                      (wm[1] + wm[0]) * cac1) * T(0.25);
+      const T S11 = dudx;
+      const T S12 = (dudy + dvdx) * T(0.5);
+      const T S13 = (dudz + dwdx) * T(0.5);
+      const T S22 = dvdy;
+      const T S23 = (dvdz + dwdy) * T(0.5);
+      const T S33 = dwdz;
+      const T SijSij = S11 * S11 + S22 * S22 + S33 * S33 + T(2) * (S12 * S12 + S13 * S13 + S23 * S23);
+  
+      T Sd11 = dudx * dudx + dudy * dvdx + dudz * dwdx;
+      const T Sd12 = (dudx * dudy + dudy * dvdy + dudz * dwdy + dvdx * dudx + dvdy * dvdx + dvdz * dwdx) * T(0.5);
+      const T Sd13 = (dudx * dudz + dudy * dvdz + dudz * dwdz + dwdx * dudx + dwdy * dvdx + dwdz * dwdx) * T(0.5);
+      T Sd22 = dvdx * dudy + dvdy * dvdy + dvdz * dwdy;
+      const T Sd23 = (dvdx * dudz + dvdy * dvdz + dvdz * dwdz + dwdx * dudy + dwdy * dvdy + dwdz * dwdy) * T(0.5);
+      T Sd33 = dwdx * dudz + dwdy * dvdz + dwdz * dwdz;
+      const T SdTrace = (Sd11 + Sd22 + Sd33) / T(3);
+      Sd11 = Sd11 - SdTrace;
+      Sd22 = Sd22 - SdTrace;
+      Sd33 = Sd33 - SdTrace;
+      const T SdijSdij =
+          Sd11 * Sd11 + Sd22 * Sd22 + Sd33 * Sd33 + T(2) * (Sd12 * Sd12 + Sd13 * Sd13 + Sd23 * Sd23);
+      // the reference's powers (**1.5, **2.5, **1.25) of these non-negative
+      // sums through square roots: x^1.5 = x sqrt(x), x^2.5 = x^2 sqrt(x),
+      // x^1.25 = x sqrt(sqrt(x)), a few ulp from pow at a fraction of its cost
+      const T sdh = sqrt(SdijSdij), sh = sqrt(SijSij);
+      nv = CwDelta2 * (SdijSdij * sdh) /
+               (SijSij * SijSij * sh + SdijSdij * sqrt(sdh)) + q.xnu;
+    }
+    stage((k + 1) & 1);
+    if (live) {
+      nut[fidx(g, i, jc, k)] = nv;
+      nut_ghosts(g, q, nut, i, jc, k, nv);
+    }
+    __syncthreads();
   }
 }
 
@@ -856,14 +932,15 @@ template <typename T>
 static int sgs_t(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* nut) {
   const Geom& g = c->g;
   const LesCoef<T> q = make_les_coef<T>(c);
-  if (c->les_type == 2)
-    hipLaunchKernelGGL(k_sgs_wale<T>, dim3(les_blocks(g)), dim3(LBX, LBY), 0, c->stream, g,
+  const int tiles = ((g.nx + LBX - 1) / LBX) * ((g.ny + LBY - 1) / LBY);
+  const int kc = march_kchunk((long long)tiles * LBY, g.nz, c->les_type == 2 ? 2 : 3);
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(tiles * ((g.nz + kc - 1) / kc)), dim3(LBX, LBY), 0, c->stream, g,
                        met<T>(c), lesmet<T>(c), q, (const T*)ux, (const T*)uy, (const T*)uz,
-                       (T*)nut);
-  else
-    hipLaunchKernelGGL(k_sgs_mts<T>, dim3(les_blocks(g)), dim3(LBX, LBY), 0, c->stream, g,
-                       met<T>(c), lesmet<T>(c), q, (const T*)ux, (const T*)uy, (const T*)uz,
-                       (T*)nut);
+                       (T*)nut, kc);
+  };
+  if (c->les_type == 2) launch(k_sgs<T, false>);
+  else launch(k_sgs<T, true>);
   C3D_HIP(hipGetLastError());
   return C3D_OK;
 }
