@@ -516,60 +516,111 @@ __global__ __launch_bounds__(FNT) void k_fft_z(Geom g, typename CT<T>::t* __rest
 // ===========================================================================
 // Any length 2^a 3^b 5^c: the radix plan is made from the length on the host
 // (the compile-time kernels' greedy choice: 8, then 4, 2, 3, 5) and the
-// kernels loop over it.  A workgroup stages its lines in LDS (dynamic, at
-// most 64 KiB), runs every pass in place there -- each pass reads all its
-// butterflies' inputs into registers, synchronises, then writes -- and
-// writes the result out.  Two LDS round trips more than the compiled
-// lengths' kernels, which fuse the first and last passes with the global
-// accesses; these kernels serve the lengths outside that list.
+// kernels loop over it.  A workgroup's lines pass through LDS (dynamic, at most
+// 64 KiB) as in the compiled lengths' kernels: the first pass reads its inputs
+// from HBM, all of a thread's loads in flight together, each pass reads all its
+// butterflies' inputs into registers, synchronises and writes in place, and the
+// last pass of the transforms that need no post-processing writes to HBM.  The
+// index divisions by run-time lengths are multiplications by reciprocals
+// prepared with the plan.  With staging copies before and after
+// (one load in flight per thread, two more LDS round trips and barriers), hardware
+// divisions and 16 values reserved per thread the four transforms of 200x150x100
+// took 25, 31, 34 and 25 us; now 10.8, 15.0, 17.5 and 19.4 (8 us of HBM time each).
 // ===========================================================================
 constexpr int GEN_MAXP = 24;   // passes: 2^24 exceeds every supported length
-constexpr int GEN_MAXE = 16;   // complex values a thread holds in one pass
+constexpr int GEN_MAXE = 8;    // complex values a thread carries: lines x n <= 8 x FNT
 constexpr int GEN_NMAX = 4095; // one line of (N+1) FP64 complex fits 64 KiB
+
+// x / d for x and d up to 2^16: with m = ceil(2^32 / d) the product exceeds
+// 2^32 x / d by less than x < 2^32 / d, too little to reach the next integer
+struct FastDiv {
+  unsigned d, m;
+  __device__ __forceinline__ int operator()(int x) const {
+    return d == 1 ? x : (int)__umulhi((unsigned)x, m);
+  }
+};
+static FastDiv make_fastdiv(int d) {
+  return {(unsigned)d, (unsigned)(((1ull << 32) + (unsigned)d - 1) / (unsigned)d)};
+}
 
 struct FftPlan {
   int n;                       // transform length
   int np;                      // passes
   int lines;                   // lines per workgroup
+  FastDiv dn, dn1, dl;         // by n, n + 1 and lines
   int r[GEN_MAXP];             // radix of each pass
+  FastDiv dnr[GEN_MAXP];       // by n / radix
+  FastDiv dns[GEN_MAXP];       // by the product of the radices before
+  int tws[GEN_MAXP];           // twiddle stride n / (that product x radix)
 };
 
 // lines per workgroup: the LDS tile (lines x (n+1) complex of esz bytes) at
-// most 64 KiB, lines x n at most 8 x FNT values so that every pass's
-// butterflies fit GEN_MAXE registers per thread, and at most `cap`
+// most 64 KiB, lines x n at most GEN_MAXE x FNT values, and at most `cap`
 static FftPlan make_plan(int n, size_t esz, int cap) {
   FftPlan pl{};
   pl.n = n;
   int m = n;
   while (m > 1 && pl.np < GEN_MAXP) {
     const int R = pick_radix(m);
-    pl.r[pl.np++] = R;
+    pl.r[pl.np] = R;
+    pl.dnr[pl.np] = make_fastdiv(n / R);
+    pl.dns[pl.np] = make_fastdiv(n / m);
     m /= R;
+    pl.tws[pl.np++] = m;
   }
   int lines = (int)(65536 / ((size_t)(n + 1) * esz));
-  lines = std::min(lines, 8 * FNT / n);
+  lines = std::min(lines, GEN_MAXE * FNT / n);
   pl.lines = std::max(1, std::min(lines, cap));
+  pl.dn = make_fastdiv(n);
+  pl.dn1 = make_fastdiv(n + 1);
+  pl.dl = make_fastdiv(pl.lines);
   return pl;
 }
 
-template <typename T2, int S, int R>
-__device__ __forceinline__ void gen_pass(T2* sm, int ldn, const T2* __restrict__ tw, int N,
-                                         int lines, int NS) {
-  constexpr int PMAX = GEN_MAXE / R;
-  const int NR = N / R, NB = lines * NR, TWS = N / (NS * R);
+// Pass q of the plan, after sub-transforms of length NS.  FIRST: inputs through
+// in() (loads for every butterfly of the thread before any arithmetic), no
+// twiddles.  LAST: outputs through out(), nothing to wait for.  The other side is
+// LDS.  LF: line-fastest butterflies on the HBM side.
+template <typename T2, int S, int R, bool FIRST, bool LAST, bool LF, class In, class Out>
+__device__ __forceinline__ void gen_pass(T2* sm, const T2* __restrict__ tw, const FftPlan& pl,
+                                         int q, int NS, int TWS, const In& in, const Out& out) {
+  constexpr int PMAX = (GEN_MAXE + R - 1) / R;
+  const int N = pl.n, lines = pl.lines, ldn = N + 1;
+  const int NR = (int)pl.dnr[q].d, NB = lines * NR;
   const int tid = threadIdx.x;
   T2 v[PMAX][R];
   int ln[PMAX], od[PMAX];
+  auto split = [&](int gb, int& line, int& jb) {
+    if (LF) {
+      jb = pl.dl(gb);
+      line = gb - jb * lines;
+    } else {
+      line = pl.dnr[q](gb);
+      jb = gb - line * NR;
+    }
+  };
+  if (FIRST) {
+#pragma unroll
+    for (int p = 0; p < PMAX; ++p) {
+      int line, jb;
+      split(min(tid + p * FNT, NB - 1), line, jb);
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[p][r] = in(line, jb + r * NR);
+    }
+  }
 #pragma unroll
   for (int p = 0; p < PMAX; ++p) {
     const int gb = tid + p * FNT;
     ln[p] = -1;
     if (gb < NB) {
-      const int line = gb / NR, j = gb - line * NR;
+      int line, jb;
+      split(gb, line, jb);
+      int k = 0, jn = jb;
+      if (!FIRST) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) v[p][r] = sm[line * ldn + j + r * NR];
-      const int k = j % NS;
-      if (NS > 1) {
+        for (int r = 0; r < R; ++r) v[p][r] = sm[line * ldn + jb + r * NR];
+        jn = pl.dns[q](jb);
+        k = jb - jn * NS;
 #pragma unroll
         for (int r = 1; r < R; ++r) {
           T2 w = tw[k * r * TWS];
@@ -579,33 +630,59 @@ __device__ __forceinline__ void gen_pass(T2* sm, int ldn, const T2* __restrict__
       }
       Dft<R, S, T2>::run(v[p]);
       ln[p] = line;
-      od[p] = (j / NS) * NS * R + k;
+      od[p] = jn * NS * R + k;
     }
   }
-  __syncthreads();
+  if (!FIRST && !LAST) __syncthreads();
 #pragma unroll
   for (int p = 0; p < PMAX; ++p) {
     if (ln[p] >= 0) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) sm[ln[p] * ldn + od[p] + r * NS] = v[p][r];
+      for (int r = 0; r < R; ++r) {
+        if (LAST) out(ln[p], od[p] + r * NS, v[p][r]);
+        else sm[ln[p] * ldn + od[p] + r * NS] = v[p][r];
+      }
     }
   }
-  __syncthreads();
+  if (!LAST) __syncthreads();
 }
 
-// the whole transform of the lines staged in sm (line stride ldn), in place
-template <typename T2, int S>
-__device__ void gen_fft(T2* sm, int ldn, const T2* __restrict__ tw, const FftPlan& pl) {
-  int NS = 1;
-  for (int q = 0; q < pl.np; ++q) {
-    switch (pl.r[q]) {
-      case 8: gen_pass<T2, S, 8>(sm, ldn, tw, pl.n, pl.lines, NS); break;
-      case 4: gen_pass<T2, S, 4>(sm, ldn, tw, pl.n, pl.lines, NS); break;
-      case 2: gen_pass<T2, S, 2>(sm, ldn, tw, pl.n, pl.lines, NS); break;
-      case 3: gen_pass<T2, S, 3>(sm, ldn, tw, pl.n, pl.lines, NS); break;
-      default: gen_pass<T2, S, 5>(sm, ldn, tw, pl.n, pl.lines, NS); break;
-    }
+// one pass by its radix
+template <typename T2, int S, bool FIRST, bool LAST, bool LF, class In, class Out>
+__device__ __forceinline__ void gen_radix(T2* sm, const T2* __restrict__ tw, const FftPlan& pl,
+                                          int q, int NS, const In& in, const Out& out) {
+  const int TWS = pl.tws[q];
+  switch (pl.r[q]) {
+    case 8: gen_pass<T2, S, 8, FIRST, LAST, LF>(sm, tw, pl, q, NS, TWS, in, out); break;
+    case 4: gen_pass<T2, S, 4, FIRST, LAST, LF>(sm, tw, pl, q, NS, TWS, in, out); break;
+    case 2: gen_pass<T2, S, 2, FIRST, LAST, LF>(sm, tw, pl, q, NS, TWS, in, out); break;
+    case 3: gen_pass<T2, S, 3, FIRST, LAST, LF>(sm, tw, pl, q, NS, TWS, in, out); break;
+    default: gen_pass<T2, S, 5, FIRST, LAST, LF>(sm, tw, pl, q, NS, TWS, in, out); break;
+  }
+}
+
+// The whole transform of a workgroup's lines (line stride n + 1 in sm): inputs
+// through in(line, index); outputs through out(line, index, value), or left in sm
+// behind a barrier (OUT_LDS).
+template <typename T2, int S, bool LF, bool OUT_LDS, class In, class Out>
+__device__ __forceinline__ void gen_fft(T2* sm, const T2* __restrict__ tw, const FftPlan& pl,
+                                        const In& in, const Out& out) {
+  gen_radix<T2, S, true, false, LF>(sm, tw, pl, 0, 1, in, out);
+  int NS = pl.r[0];
+  const int mid = OUT_LDS ? pl.np : pl.np - 1;
+  for (int q = 1; q < mid; ++q) {
+    gen_radix<T2, S, false, false, false>(sm, tw, pl, q, NS, in, out);
     NS *= pl.r[q];
+  }
+  if (OUT_LDS) return;
+  if (pl.np > 1) {
+    gen_radix<T2, S, false, true, LF>(sm, tw, pl, pl.np - 1, NS, in, out);
+    return;
+  }
+  // a single pass (lengths 2 to 5 and 8): its results are in sm
+  for (int e = threadIdx.x; e < pl.lines * pl.n; e += FNT) {
+    const int l = pl.dn(e), m = e - l * pl.n;
+    out(l, m, sm[l * (pl.n + 1) + m]);
   }
 }
 
@@ -627,21 +704,17 @@ __global__ __launch_bounds__(FNT) void k_fftg_x_fwd(Geom g, FftPlan pl, const TI
   const int nrows = g.ny * g.nz;
   row_offsets(g, row0, lines, rb);
   __syncthreads();
-  for (int e = threadIdx.x; e < lines * N; e += FNT) {
-    const int l = e / N, m = e - l * N;
+  // past the last row: the field's first row is read and zero taken (a branch
+  // would hold back the next element's load)
+  auto ld = [&](int l, int m) -> T2 {
     const long long b = rb[l];
-    T2 z = mk<T2>(0, 0);
-    if (b >= 0) {
-      const TI2 w = ((const TI2*)(in + b))[m];
-      z = mk<T2>((T)w.x, (T)w.y);
-    }
-    sm[l * ldn + m] = z;
-  }
-  __syncthreads();
-  gen_fft<T2, -1>(sm, ldn, tw, pl);
+    const TI2 w = ((const TI2*)(in + (b < 0 ? (long long)g.nx : b)))[m];
+    return b < 0 ? mk<T2>(0, 0) : mk<T2>((T)w.x, (T)w.y);
+  };
+  gen_fft<T2, -1, false, true>(sm, tw, pl, ld, [](int, int, const T2&) {});
   // X_k = (Z_k + conj Z_{N-k})/2 + w_k (Z_k - conj Z_{N-k})/(2i)
   for (int e = threadIdx.x; e < lines * (N + 1); e += FNT) {
-    const int l = e / (N + 1), k = e - l * (N + 1), row = row0 + l;
+    const int l = pl.dn1(e), k = e - l * (N + 1), row = row0 + l;
     if (row >= nrows) continue;
     const T2 zk = sm[l * ldn + (k == N ? 0 : k)];
     const T2 zn = sm[l * ldn + (k == 0 ? 0 : N - k)];
@@ -673,33 +746,27 @@ __global__ __launch_bounds__(FNT) void k_fftg_x_inv(Geom g, FftPlan pl,
   const int row0 = blockIdx.x * lines;
   const int nrows = g.ny * g.nz;
   row_offsets(g, row0, lines, rb);
-  // Z_k = (X_k + conj X_{N-k}) + i conj(w_k) (X_k - conj X_{N-k})
-  for (int e = threadIdx.x; e < lines * N; e += FNT) {
-    const int l = e / N, k = e - l * N, row = row0 + l;
-    T2 z = mk<T2>(0, 0);
-    if (row < nrows) {
-      const T2* sp = spec + (long long)g.P * row;
-      T2 xk = sp[k], xn = sp[N - k];
-      if (k == 0) {
-        xk.y = 0;
-        xn.y = 0;
-      }
-      const T2 a = mk<T2>(xk.x + xn.x, xk.y - xn.y);
-      const T2 b = mk<T2>(xk.x - xn.x, xk.y + xn.y);
-      T2 w = twr[k];
-      w.y = -w.y;
-      const T2 wb = cmul(w, b);
-      z = mk<T2>(a.x - wb.y, a.y + wb.x);
-    }
-    sm[l * ldn + k] = z;
-  }
   __syncthreads();
-  gen_fft<T2, 1>(sm, ldn, tw, pl);
-  for (int e = threadIdx.x; e < lines * N; e += FNT) {
-    const int l = e / N, m = e - l * N;
+  // Z_k = (X_k + conj X_{N-k}) + i conj(w_k) (X_k - conj X_{N-k}); past the last
+  // row: the last row is read and zero taken
+  auto ld = [&](int l, int k) -> T2 {
+    const bool live = row0 + l < nrows;
+    const T2* sp = spec + (long long)g.P * min(row0 + l, nrows - 1);
+    T2 xk = sp[k], xn = sp[N - k];
+    T2 w = twr[k];
+    if (k == 0) {
+      xk.y = 0;
+      xn.y = 0;
+    }
+    const T2 a = mk<T2>(xk.x + xn.x, xk.y - xn.y);
+    const T2 b = mk<T2>(xk.x - xn.x, xk.y + xn.y);
+    w.y = -w.y;
+    const T2 wb = cmul(w, b);
+    return live ? mk<T2>(a.x - wb.y, a.y + wb.x) : mk<T2>(0, 0);
+  };
+  auto st = [&](int l, int m, const T2& z) {
     const long long b = rb[l];
-    if (b < 0) continue;
-    const T2 z = sm[l * ldn + m];
+    if (b < 0) return;
     TO2* rp = (TO2*)(out + b);
     if (ACC) {
       const TO2 o = rp[m];
@@ -708,7 +775,8 @@ __global__ __launch_bounds__(FNT) void k_fftg_x_inv(Geom g, FftPlan pl,
       C3D_ST_ONCE((TOUT)z.x * scale, &rp[m].x);
       C3D_ST_ONCE((TOUT)z.y * scale, &rp[m].y);
     }
-  }
+  };
+  gen_fft<T2, 1, false, false>(sm, tw, pl, ld, st);
 }
 
 // z, in place: pl.lines consecutive kx of one y plane, all kz
@@ -726,21 +794,19 @@ __global__ __launch_bounds__(FNT) void k_fftg_z(Geom g, FftPlan pl,
   const int nl = min(lines, g.nk + 1 - kx0);
   const long long sk = (long long)g.P * g.ny;
   T2* base = spec + (long long)g.P * blockIdx.y + kx0;
-  for (int e = threadIdx.x; e < lines * N; e += FNT) {
-    const int l = e % lines, m = e / lines;
-    sm[l * ldn + m] = l < nl ? base[sk * m + l] : mk<T2>(0, 0);
-  }
-  __syncthreads();
-  gen_fft<T2, S>(sm, ldn, tw, pl);
-  for (int e = threadIdx.x; e < lines * N; e += FNT) {
-    const int l = e % lines, m = e / lines;
+  // past the last kx: the first one is read and zero taken
+  auto ld = [&](int l, int kz) -> T2 {
+    const T2 z = base[sk * kz + (l < nl ? l : 0)];
+    return l < nl ? z : mk<T2>(0, 0);
+  };
+  auto st = [&](int l, int kz, const T2& v) {
     if (l < nl) {
-      const T2 v = sm[l * ldn + m];
-      T2* d = &base[sk * m + l];
+      T2* d = &base[sk * kz + l];
       C3D_ST_ONCE(v.x, &d->x);
       C3D_ST_ONCE(v.y, &d->y);
     }
-  }
+  };
+  gen_fft<T2, S, true, false>(sm, tw, pl, ld, st);
 }
 
 template <typename T, typename TIN, bool NTS>
