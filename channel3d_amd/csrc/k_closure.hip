@@ -308,10 +308,30 @@ __device__ __forceinline__ void transpose4(const s4v* in, s4v* out,
   wave_sync();
 }
 
-// sum over the 16 lanes of a quarter (samples), result in every lane
+// sum over the 16 lanes of a quarter (samples), result in every lane: the
+// butterfly over lane distances 1, 2, 4, 8 by DPP (once a group's lanes hold
+// one value, mirrors reach the same partner value as the distances 4 and 8)
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  const int t = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true);
+  return v + __builtin_bit_cast(float, t);
+}
 __device__ __forceinline__ float quarter_sum(float v) {
-  for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v = dpp_add<0xB1>(v);   // quad_perm 1 0 3 2
+  v = dpp_add<0x4E>(v);   // quad_perm 2 3 0 1
+  v = dpp_add<0x141>(v);  // mirror within 8
+  return dpp_add<0x140>(v);  // mirror within 16
+}
+
+// Where the LDS copies of the parameter vector hold parameter p.  A row (one
+// input's 64 outputs) of the first three layers has its 16 groups of four outputs
+// permuted by the input: the lanes of a quarter write one group of 16
+// consecutive rows, which unpermuted all lie on the same four banks.
+__device__ __forceinline__ int par_slot(int p) {
+  const int l = p >= OFF_W[3] ? 3 : p >= OFF_W[2] ? 2 : p >= OFF_W[1] ? 1 : 0;
+  const int loc = p - (l == 3 ? OFF_W[3] : l == 2 ? OFF_W[2] : l == 1 ? OFF_W[1] : OFF_W[0]);
+  const bool sw = l < 3 && loc < (l == 0 ? NPAD : NH) * NH;
+  return sw ? p ^ ((loc / NH & 15) << 2) : p;
 }
 
 // Which samples a gradient evaluation reads: sample base + t (idx and key
@@ -354,6 +374,9 @@ __device__ __forceinline__ unsigned feistel_perm(unsigned x, unsigned n, int h, 
 // tiles.  At the end the four wavefronts add their sums into one LDS copy
 // of the parameter vector in a fixed order, and the workgroup writes it as
 // its partial (FP32) with its squared-error sum (FP64).
+// Bound: one wavefront per SIMD through the chain of layers (25.2 us at 16,384
+// samples, one tile each; 26.6 with the sums put unpermuted and the first gather
+// after the staging).
 constexpr int GWAVES = 4;
 __global__ __launch_bounds__(64 * GWAVES) void k_cl_grad(const float* __restrict__ X,
                                                          const float* __restrict__ Tg,
@@ -364,51 +387,21 @@ __global__ __launch_bounds__(64 * GWAVES) void k_cl_grad(const float* __restrict
                                                          const float* __restrict__ w,
                                                          float* __restrict__ partial,
                                                          double* __restrict__ lpart) {
-  __shared__ float red[NPARAM];
+  __shared__ __align__(16) float red[NPARAM];
   __shared__ unsigned short trs[GWAVES][4][16][20];
   __shared__ double lsh[GWAVES];
   // the step's bf16 fragments and biases, read from LDS at each use (kept in
   // registers across the tile loop they would push the accumulators out)
-  __shared__ s4v frag[(NFWD + NBWD) * 64];
+  // (sized for the second copy of the parameter vector as well, which is longer)
+  constexpr int NFRAG = (NFWD + NBWD) * 64, NFSH = NFRAG > (NPARAM + 1) / 2 ? NFRAG : (NPARAM + 1) / 2;
+  __shared__ __align__(16) s4v frag[NFSH];
   __shared__ float bsh[3 * NH + NOUT];
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, r = lane & 15;
-  {
-    // all loads issued before the LDS stores wait for them
-    constexpr int NF = (NFWD + NBWD) * 64, PER = (NF + 64 * GWAVES - 1) / (64 * GWAVES);
-    s4v tmp[PER];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int e = threadIdx.x + k * 64 * GWAVES;
-      if (e < NF) tmp[k] = e < NFWD * 64 ? fwd[e] : bwd[e - NFWD * 64];
-    }
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int e = threadIdx.x + k * 64 * GWAVES;
-      if (e < NF) frag[e] = tmp[k];
-    }
-  }
-  for (int e = threadIdx.x; e < 3 * NH + NOUT; e += 64 * GWAVES)
-    bsh[e] = w[e < NH ? OFF_B[0] + e : (e < 2 * NH ? OFF_B[1] + e - NH
-                                                   : (e < 3 * NH ? OFF_B[2] + e - 2 * NH
-                                                                 : OFF_B[3] + e - 3 * NH))];
-  __syncthreads();
-  const s4v* fw = frag;
-  const s4v* bw = frag + NFWD * 64;
-  const float* bias[4] = {bsh, bsh + NH, bsh + 2 * NH, bsh + 3 * NH};
-  unsigned short (*tr4)[16][20] = trs[wv];
-  unsigned short (*tr)[20] = trs[wv][0];
   const f4v zero = {0.f, 0.f, 0.f, 0.f};
-  f4v acc[40];
-  f4v bacc[13];  // bias sums: layer 1..3 tiles 0..3 at [4 L + ot], layer 4 at [12]
-#pragma unroll
-  for (int e = 0; e < 40; ++e) acc[e] = zero;
-#pragma unroll
-  for (int e = 0; e < 13; ++e) bacc[e] = zero;
-  const float coef = (float)(2.0 / (ntot * NOUT));
-  double lsum = 0.0;
   const long long ntile = (n + 15) / 16;
-  // the gathered inputs and targets of a tile; the next tile's are loaded
-  // while the current one runs
+  // the gathered inputs and targets of a tile; the first tile's are
+  // requested before the fragments are staged, the next tile's while the current
+  // one runs
   auto gather = [&](long long t, f4v& xv, f4v& tg, bool& ok) {
     const long long tl = t * 16 + r;
     ok = t < ntile && tl < n;
@@ -432,6 +425,39 @@ __global__ __launch_bounds__(64 * GWAVES) void k_cl_grad(const float* __restrict
   f4v xn, tn;
   bool okn;
   gather(t, xn, tn, okn);
+  {
+    // all loads issued before the LDS stores wait for them
+    constexpr int NF = NFRAG, PER = (NF + 64 * GWAVES - 1) / (64 * GWAVES);
+    s4v tmp[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = threadIdx.x + k * 64 * GWAVES;
+      if (e < NF) tmp[k] = e < NFWD * 64 ? fwd[e] : bwd[e - NFWD * 64];
+    }
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const int e = threadIdx.x + k * 64 * GWAVES;
+      if (e < NF) frag[e] = tmp[k];
+    }
+  }
+  for (int e = threadIdx.x; e < 3 * NH + NOUT; e += 64 * GWAVES)
+    bsh[e] = w[e < NH ? OFF_B[0] + e : (e < 2 * NH ? OFF_B[1] + e - NH
+                                                   : (e < 3 * NH ? OFF_B[2] + e - 2 * NH
+                                                                 : OFF_B[3] + e - 3 * NH))];
+  __syncthreads();
+  const s4v* fw = frag;
+  const s4v* bw = frag + NFWD * 64;
+  const float* bias[4] = {bsh, bsh + NH, bsh + 2 * NH, bsh + 3 * NH};
+  unsigned short (*tr4)[16][20] = trs[wv];
+  unsigned short (*tr)[20] = trs[wv][0];
+  f4v acc[40];
+  f4v bacc[13];  // bias sums: layer 1..3 tiles 0..3 at [4 L + ot], layer 4 at [12]
+#pragma unroll
+  for (int e = 0; e < 40; ++e) acc[e] = zero;
+#pragma unroll
+  for (int e = 0; e < 13; ++e) bacc[e] = zero;
+  const float coef = (float)(2.0 / (ntot * NOUT));
+  double lsum = 0.0;
   for (; t < ntile; t += tstride) {
     const f4v xv = xn, tg = tn;
     const bool ok = okn;
@@ -529,12 +555,17 @@ __global__ __launch_bounds__(64 * GWAVES) void k_cl_grad(const float* __restrict
 #pragma unroll
         for (int it = 0; it < nit; ++it) {
           const f4v a = acc[off + ot * nit + it];
+          if (l < 3) {  // four outputs of one input: par_slot's place of them
+            f4v* d = (f4v*)&dst[OFF_W[l] + (16 * it + r) * NH + ((16 * ot + 4 * q) ^ (r << 2))];
+            *d = first ? a : *d + a;
+          } else {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int out = 16 * ot + 4 * q + i, in = 16 * it + r;
-            if (out < OUTD[l] && in < IND[l]) {
-              float& d = dst[OFF_W[l] + in * OUTD[l] + out];
-              d = first ? a[i] : d + a[i];
+            for (int i = 0; i < 4; ++i) {
+              const int out = 4 * q + i, in = 16 * it + r;
+              if (out < OUTD[l]) {
+                float& d = dst[OFF_W[l] + in * OUTD[l] + out];
+                d = first ? a[i] : d + a[i];
+              }
             }
           }
         }
@@ -562,7 +593,10 @@ __global__ __launch_bounds__(64 * GWAVES) void k_cl_grad(const float* __restrict
   if (wv >= 2) put((wv & 1) ? cpyB : red, std::false_type{});
   __syncthreads();
   float* pp = partial + (long long)blockIdx.x * NPARAM;
-  for (int e = threadIdx.x; e < NPARAM; e += 64 * GWAVES) pp[e] = red[e] + cpyB[e];
+  for (int e = threadIdx.x; e < NPARAM; e += 64 * GWAVES) {
+    const int d = par_slot(e);
+    pp[e] = red[d] + cpyB[d];
+  }
   for (int o = 32; o > 0; o >>= 1) lsum += __shfl_down(lsum, o, 64);
   if (lane == 0) lsh[wv] = lsum;
   __syncthreads();
@@ -632,7 +666,8 @@ __global__ void k_cl_adam(float* __restrict__ w, const float* __restrict__ g,
 // the workgroup partials in k_cl_reduce's fixed order; Adam updates the
 // master, and the thread writes the master's bf16 value into the forward and
 // backward fragments that hold it (the layouts of k_cl_pack).  loss as
-// k_cl_reduce.
+// k_cl_reduce.  Bound: the latency of the partials (10 MB of L2 at 256
+// workgroups); with four of a thread's sixteen in flight 7.1 us, with all 4.8.
 __global__ __launch_bounds__(1024) void k_cl_reduce_adam(const float* __restrict__ partial,
                                                          int nwg,
                                                          const double* __restrict__ lpart,
@@ -647,17 +682,26 @@ __global__ __launch_bounds__(1024) void k_cl_reduce_adam(const float* __restrict
   const int t = threadIdx.x, pl = t & 63, bg = t >> 6;
   const int p = blockIdx.x * 64 + pl;
   double a[4] = {0.0, 0.0, 0.0, 0.0};
-  // four partials per iteration, loaded before they are added (independent
-  // loads in flight); partial b goes to accumulator ((b - bg) / 16) % 4
-  if (p < NPARAM)
-    for (int b = bg; b < nwg; b += 64) {
-      float v[4];
+  // the state's words are requested with the partials
+  const int pc = p < NPARAM ? p : NPARAM - 1;
+  float m0 = 0.0f, v0 = 0.0f, w0 = 0.0f;
+  if (bg == 0) {
+    m0 = m[pc];
+    v0 = v[pc];
+    w0 = w[pc];
+  }
+  // sixteen partials per iteration (all of a thread's at 256 workgroups),
+  // requested before they are added, past the last one the last again and zero
+  // taken (a guarded load is a branch that holds back the next); partial b goes to
+  // accumulator ((b - bg) / 16) % 4
+  for (int b = bg; b < nwg; b += 256) {
+    float x[16];
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        v[u] = b + 16 * u < nwg ? partial[(long long)(b + 16 * u) * NPARAM + p] : 0.0f;
+    for (int u = 0; u < 16; ++u)
+      x[u] = partial[(long long)min(b + 16 * u, nwg - 1) * NPARAM + pc];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) a[u] += (double)v[u];
-    }
+    for (int u = 0; u < 16; ++u) a[u % 4] += b + 16 * u < nwg ? (double)x[u] : 0.0;
+  }
   sh[bg][pl] = (a[0] + a[1]) + (a[2] + a[3]);
   __syncthreads();
   if (bg == 0 && p < NPARAM && !(p < OFF_B[0] && p / NH >= NIN)) {
@@ -665,11 +709,11 @@ __global__ __launch_bounds__(1024) void k_cl_reduce_adam(const float* __restrict
     for (int qq = 0; qq < 16; ++qq) sum += sh[qq][pl];
     const float gp = (float)sum;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float mp = b1 * m[p] + (1.0f - b1) * gp;
-    const float vp = b2 * v[p] + (1.0f - b2) * gp * gp;
+    const float mp = b1 * m0 + (1.0f - b1) * gp;
+    const float vp = b2 * v0 + (1.0f - b2) * gp * gp;
     m[p] = mp;
     v[p] = vp;
-    const float wn = w[p] - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
+    const float wn = w0 - lr * (mp / c1) / (sqrtf(vp / c2) + eps);
     w[p] = wn;
     // the weight's places in the bf16 fragments (biases have none)
     int l = 3;
