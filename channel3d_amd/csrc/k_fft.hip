@@ -525,7 +525,7 @@ __global__ __launch_bounds__(FNT) void k_fft_z(Geom g, typename CT<T>::t* __rest
 // prepared with the plan.  With staging copies before and after
 // (one load in flight per thread, two more LDS round trips and barriers), hardware
 // divisions and 16 values reserved per thread the four transforms of 200x150x100
-// took 25, 31, 34 and 25 us; now 10.8, 15.0, 17.5 and 19.4 (8 us of HBM time each).
+// took 25, 31, 34 and 25 us; now 11, 14, 17 and 14 (8 us of HBM time each).
 // ===========================================================================
 constexpr int GEN_MAXP = 24;   // passes: 2^24 exceeds every supported length
 constexpr int GEN_MAXE = 8;    // complex values a thread carries: lines x n <= 8 x FNT
@@ -602,6 +602,7 @@ __device__ __forceinline__ void gen_pass(T2* sm, const T2* __restrict__ tw, cons
   if (FIRST) {
 #pragma unroll
     for (int p = 0; p < PMAX; ++p) {
+      if (p * FNT >= NB) break;  // for the whole workgroup
       int line, jb;
       split(min(tid + p * FNT, NB - 1), line, jb);
 #pragma unroll
