@@ -1510,8 +1510,8 @@ static int substep_pressure(c3d_ctx* c, void* pr) {
     return run_ppe_from_spectrum(c, s[C3D_HALOARR]);
   }
   // x lengths with a run-time plan and the refined solve: a source pass
-  if ((rc = launch_bc_vel(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_UY_YM], 0))) return rc;
-  if ((rc = launch_prsrc(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], pr, 0.0))) return rc;
+  if ((rc = launch_prsrc(c, s[C3D_UX], s[C3D_UY], s[C3D_UZ], s[C3D_ARR1], pr, 0.0, true)))
+    return rc;
   return run_ppe(c, s[C3D_ARR1], s[C3D_HALOARR]);
 }
 

@@ -516,7 +516,7 @@ int launch_rhs(c3d_ctx* c, int mask, const void* ux, const void* uy, const void*
 int launch_bulk_finalize(c3d_ctx* c, int nblocks, int reset_aver);
 int launch_add_dpmdxns(c3d_ctx* c, void* rx);
 int launch_prsrc(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* prsrc,
-                 void* pr, double alpha_override);
+                 void* pr, double alpha_override, bool fused = false);
 int launch_max_finalize(c3d_ctx* c, int nblocks, int slot);
 int launch_bc_vel(c3d_ctx* c, void* ux, void* uy, void* uz, const void* uy_ym, int full);
 int launch_bc_pr(c3d_ctx* c, void* pr);

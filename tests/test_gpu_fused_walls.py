@@ -82,3 +82,12 @@ def test_fused_equals_routines(monkeypatch, kind, ny, nt):
         assert np.array_equal(a, b)
     assert out[0][1] == out[1][1]
     assert out[0][2] == out[1][2]
+
+
+@pytest.mark.parametrize("kind", ["channel", "freeslip", "les"])
+def test_fused_source_pass(monkeypatch, kind):
+    """the same where the x length has a run-time transform plan and the source
+    is a pass of its own"""
+    monkeypatch.setenv("C3D_FFT_PLAN", "runtime")
+    test_fused_equals_routines(monkeypatch, kind, 13, "0")
+    test_fused_equals_routines(monkeypatch, kind, 5, "1")
