@@ -434,6 +434,108 @@ __global__ __launch_bounds__(256) void k_tridiag_ck2(Geom g, PprRows(T),
                                 line_of(g, ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 1));
 }
 
+// The two-lane sweep with a line's forward values and factors kept in LDS (96
+// reals per row of a wavefront's 32 pairs) instead of checkpoints: the backward
+// pass substitutes at once where it otherwise runs each segment's elimination a
+// second time.  The same operations on the same operands, so the same values.
+// For grids with one or two wavefronts per CU: there the serial chain, not
+// traffic, is the time (64^3 19.4 -> 14.8 us, 96x96x72 24.9 -> 19.0, 150x101x108
+// 28.8 -> 22.6).  With more lines than that a second round of workgroups costs as
+// much as the first, and the checkpointed form holds more wavefronts.  PER:
+// workgroups that share a CU's LDS.
+template <typename T, int PER>
+constexpr int tri_lds_rows() {
+  return 159744 / (96 * PER * (int)sizeof(T));
+}
+
+template <typename T, int PER, bool NTS>
+__global__ __launch_bounds__(64) void k_tridiag_lds(Geom g, PprRows(T),
+                                                    typename CT2<T>::t* __restrict__ spec,
+                                                    long long bsp) {
+  constexpr int C = 16;
+  __shared__ T sf[tri_lds_rows<T, PER>() * 64];  // forward values of a lane
+  __shared__ T sa[tri_lds_rows<T, PER>() * 32];  // factors, one for a pair's two lanes
+  const int lane = threadIdx.x, part = lane & 1, pair = lane >> 1;
+  const Line ln = line_of(g, ((long long)blockIdx.x * 64 + lane) >> 1);
+  const int kx = ln.kx, kz = ln.kz;
+  if (kz >= g.nz) return;  // no barrier below: a lane reads what it wrote
+  const int ny = g.ny, top = (ny + C - 1) / C - 1;
+  const long long P2 = 2LL * g.P;
+  T* sp = (T*)(spec + bsp * blockIdx.y) + 2 * (kx + (long long)g.P * ny * kz) + part;
+  const T lx = wx[kx], lz = wz[kz];
+  const bool pin = (kx == 0 && kz == 0);
+  using Gd = std::true_type;  // the top segment: rows past the last one
+  using Un = std::false_type;
+  auto load = [&](T* y, int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+#pragma unroll
+    for (int q = 0; q < C; ++q)
+      if (!G || s * C + q < ny) y[q] = sp[P2 * (s * C + q)];
+  };
+  // Row 1 has nothing below: f = 0, vecm = 1 and cprev = 0 give its pivot and value
+  T vecm = T(1), rv = T(1), cprev = T(0), f = T(0);
+  auto run = [&](const T* y, int s, auto gv) {
+    constexpr bool G = decltype(gv)::value;
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+      const int j0 = s * C + q;
+      if (!G || j0 < ny) {
+        const int jr = j0 + 1;
+        const T arr = quot(cprev, vecm, rv);
+        const T a = am[jr];
+        T fj = y[q], cj = ap[jr];
+        vecm = ((ac[jr] + lx) + lz) - a * arr;
+        if (q == 0 && s == 0 && pin) {  // the gauge row
+          vecm = T(1);
+          fj = cj = T(0);
+        }
+        rv = quot_recip(vecm);
+        f = quot(fj - a * f, vecm, rv);
+        cprev = cj;
+        sf[j0 * 64 + lane] = f;
+        sa[j0 * 32 + pair] = arr;
+      }
+    }
+  };
+  T ya[C], yb[C];
+  if (top == 0) {
+    load(ya, 0, Gd{});
+    run(ya, 0, Gd{});
+  } else {
+    load(ya, 0, Un{});
+    int s = 0;
+    for (; s + 2 < top; s += 2) {  // each load a segment ahead
+      load(yb, s + 1, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
+      load(ya, s + 2, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(yb, s + 1, Un{});
+    }
+    if (s + 1 < top) {
+      load(yb, s + 1, Un{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
+      load(ya, top, Gd{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(yb, s + 1, Un{});
+      run(ya, top, Gd{});
+    } else {
+      load(yb, top, Gd{});
+      __builtin_amdgcn_sched_barrier(0);
+      run(ya, s, Un{});
+      run(yb, top, Gd{});
+    }
+  }
+  T x = f;
+  C3D_ST_ONCE(x, &sp[P2 * (ny - 1)]);
+#pragma unroll 16
+  for (int j0 = ny - 2; j0 >= 0; --j0) {
+    x = sf[j0 * 64 + lane] - sa[(j0 + 1) * 32 + pair] * x;
+    C3D_ST_ONCE(x, &sp[P2 * j0]);
+  }
+}
+
 // The one-lane form, which C3D_TRIDIAG_LANES=1 selects to compare with.  At
 // least 4 waves per SIMD: the FP64 body fits 128 VGPRs without spilling.
 // Batches: blockIdx.y selects the field; its spectrum starts bsp complex
@@ -480,6 +582,10 @@ static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
     hipLaunchKernelGGL(kern, grid, blk, 0, c->stream, g, PPR_OF(m), (typename CT2<T>::t*)spec,
                        (T*)ck, b.spec, b.ck);
   };
+  auto launch_lds = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)((nl * 2 + 63) / 64), b.n), dim3(64), 0, c->stream, g,
+                       PPR_OF(m), (typename CT2<T>::t*)spec, b.spec);
+  };
   // checkpoints: 3 reals per line and segment, in the spectral scratch
   const long long need = 3LL * ((g.ny + CSEG - 1) / CSEG) * g.P * g.nz;
   if (c->ymode == YS_STORE || need > (long long)g.P * g.ny * g.nz) {
@@ -487,6 +593,12 @@ static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
   } else if (c->tri_lanes == 1) {
     if (g.nt) launch(k_tridiag_ck<T, CSEG, true>, 256, 1);
     else launch(k_tridiag_ck<T, CSEG, false>, 256, 1);
+  } else if (c->tri_lanes == 0 && nl * b.n * 2 <= 512LL * 64 && g.ny <= tri_lds_rows<T, 2>()) {
+    if (g.nt) launch_lds(k_tridiag_lds<T, 2, true>);
+    else launch_lds(k_tridiag_lds<T, 2, false>);
+  } else if (c->tri_lanes == 0 && nl * b.n * 2 <= 256LL * 64 && g.ny <= tri_lds_rows<T, 1>()) {
+    if (g.nt) launch_lds(k_tridiag_lds<T, 1, true>);
+    else launch_lds(k_tridiag_lds<T, 1, false>);
   } else if (nl * b.n * 2 <= 1024LL * 64) {
     // at most a wavefront per SIMD: the lines' serial chains bound the sweep,
     // and single-wave workgroups of 16-row segments spread them over the most
