@@ -345,7 +345,7 @@ __global__ void k_add_scalar(Geom g, T* __restrict__ f, const DevScalars* sc) {
 // FUSED: the substep's form for x lengths without a fused source pass and for the
 // refined solve.  The wall nodes of uy are taken as the boundary values (the
 // projection writes them) and the maximum goes to the reduction slots, two
-// launches of about 5 us fewer (a lone 200x150x100 step about 23 us of 835 less).
+// launches of about 5 us fewer (a lone 150x101x108 step about 23 us of 835 less).
 template <typename T, bool PCORR, bool FUSED>
 __global__ __launch_bounds__(BX* BY) void k_prsrc(Geom g, Metrics<T> m, T rdx, T rdz, T sudtal,
                                                   T xnuhm, T vym, T vyp, DevScalars* sc,
@@ -765,17 +765,17 @@ template <>
 const Metrics<float>& mets<float>(c3d_ctx* c) { return c->mf; }
 
 // z run of the RHS kernel: long enough to amortise the two lead-in planes,
-// short enough to give the device a few thousand workgroups; on small grids down
-// to 4 planes, until every CU has two workgroups (64^3: 0.029 ms with 16 planes,
-// 64 workgroups; 0.014 ms with 4)
+// short enough to give the device a few thousand workgroups.  On grids that give
+// it only a few rounds of two workgroups per CU the rounds are counted: a last
+// round that is nearly empty costs as much as a full one (150x101x108: 546
+// workgroups of 16 planes 57.7 us, 468 of 18 planes 42.8 us; 64^3: 0.029 ms with
+// 16 planes, 64 workgroups; 0.014 ms with 4).
 static int rhs_kchunk(const Geom& g) {
   const int tiles = ((g.nx + BX - 1) / BX) * ((g.ny + RHS_WY - 1) / RHS_WY);
-  int nch = (4096 + tiles - 1) / tiles;
-  if (nch < 1) nch = 1;
+  if (tiles * ((g.nz + 15) / 16) < 2048) return march_kchunk((long long)tiles * RHS_WY, g.nz, 2);
+  const int nch = (4096 + tiles - 1) / tiles;
   int kc = (g.nz + nch - 1) / nch;
-  int lo = 16;
-  while (lo > 4 && tiles * ((g.nz + lo - 1) / lo) < 512) lo /= 2;
-  if (kc < lo) kc = lo;
+  if (kc < 16) kc = 16;
   return kc > g.nz ? g.nz : kc;
 }
 static int rhs_nblocks(const Geom& g) {
