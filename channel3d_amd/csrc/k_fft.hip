@@ -524,8 +524,8 @@ __global__ __launch_bounds__(FNT) void k_fft_z(Geom g, typename CT<T>::t* __rest
 // index divisions by run-time lengths are multiplications by reciprocals
 // prepared with the plan.  With staging copies before and after
 // (one load in flight per thread, two more LDS round trips and barriers), hardware
-// divisions and 16 values reserved per thread the four transforms of 200x150x100
-// took 25, 31, 34 and 25 us; now 11, 14, 17 and 14 (8 us of HBM time each).
+// divisions and 16 values reserved per thread the four transforms of 150x101x108
+// took 25, 31, 34 and 25 us; now 11, 14, 17 and 14 (4 us of HBM time each).
 // ===========================================================================
 constexpr int GEN_MAXP = 24;   // passes: 2^24 exceeds every supported length
 constexpr int GEN_MAXE = 8;    // complex values a thread carries: lines x n <= 8 x FNT
