@@ -600,9 +600,9 @@ static int tridiag_t(c3d_ctx* c, void* spec, void* ck, const Batch& b) {
     if (g.nt) launch_lds(k_tridiag_lds<T, 1, true>);
     else launch_lds(k_tridiag_lds<T, 1, false>);
   } else if (nl * b.n * 2 <= 1024LL * 64) {
-    // at most a wavefront per SIMD: the lines' serial chains bound the sweep,
-    // and single-wave workgroups of 16-row segments spread them over the most
-    // CUs (192x128x160: 0.040 ms against 0.043, 64^3: 0.017 against 0.022)
+    // at most a wavefront per SIMD, or lines too long for LDS: the serial chains
+    // bound the sweep, and single-wave workgroups of 16-row segments spread them
+    // over the most CUs (192x128x160: 0.040 ms against 0.043)
     if (g.nt) launch(k_tridiag_ck2<T, CSEG, true>, 64, 2);
     else launch(k_tridiag_ck2<T, CSEG, false>, 64, 2);
   } else {
