@@ -598,9 +598,9 @@ int launch_les_y3(c3d_ctx* c, void* const u[3], void* const rhs[3], const void* 
                   int add_dpmdxns);
 // pressure += (1 - pmBetaT d/dy nut d/dy) phi; phi's wall ghosts must be set
 int launch_prupd_les(c3d_ctx* c, void* pr, const void* phi);
-// FluidVelUpdate, PressureUpdate_PIMP_LES and every wall ghost in one pass (phi's
-// own Neumann ghosts applied on the fly)
-int launch_proj_les(c3d_ctx* c, const void* phi, void* ux, void* uy, void* uz, void* pr);
+// FluidVelUpdate, PressureUpdate_PIMP_LES and every wall ghost in one pass, phi's
+// own among them
+int launch_proj_les(c3d_ctx* c, void* phi, void* ux, void* uy, void* uz, void* pr);
 
 // ---- launchers (k_stats.hip) ----
 int launch_stat(c3d_ctx* c, const void* ux, const void* uy, const void* uz, const void* pr);

@@ -221,6 +221,29 @@ def test_les_multistep_parity(O, name, nsteps):
     g.close()
 
 
+@pytest.mark.parametrize("nt", ["0", "1"])
+def test_les_substep_leaves_phi_ghosts(monkeypatch, nt):
+    """after a fused substep RealHalo holds phi with SetBC_and_UpdateHalo_pr's wall ghosts,
+    as after the routines"""
+    from channel3d_amd import Channel, lib as L
+    monkeypatch.setenv("C3D_NT", nt)
+    case = dict(cases.SMALL, nxc=72, nyc=13, nzc=20, les_type=2, filter_type=1)
+    with Channel(case) as g:
+        rng = np.random.default_rng(0)
+        for f in (L.UX, L.UY, L.UZ):
+            a = np.zeros(g.shape(L.HALO), order="F")
+            a[1:73, 1:14, 1:21] = rng.uniform(-0.2, 1.0, (72, 13, 20))
+            g.upload(f, a)
+        g.project()
+        g.Clc_SGS_Vis()
+        for ns in (1, 2, 3):
+            g.substep(ns)
+            phi = g.download(L.HALOARR)
+            assert np.abs(phi[:, 1]).max() > 0 and np.abs(phi[:, 13]).max() > 0
+            assert np.array_equal(phi[:, 0], phi[:, 1])
+            assert np.array_equal(phi[:, 14], phi[:, 13])
+
+
 def test_set_les_rejects(O):
     from channel3d_amd import Channel, lib as L
     g = Channel(cases.SMALL)
