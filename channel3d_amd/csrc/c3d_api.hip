@@ -482,23 +482,6 @@ int ensure_mixed_tables(c3d_ctx* c) {
   twiddles<float>(nk, nk, a);
   twiddles<float>(2 * nk, nk + 1, b);
   twiddles<float>(nz, nz, z);
-  const size_t n = a.size() + b.size() + z.size();
-  void* tw = nullptr;
-  if ((rc = dalloc(c, &tw, sizeof(float) * n))) return rc;
-  float* d = (float*)tw;
-  C3D_HIP(hipMemcpy(d, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice));
-  C3D_HIP(hipMemcpy(d + a.size(), b.data(), sizeof(float) * b.size(), hipMemcpyHostToDevice));
-  C3D_HIP(hipMemcpy(d + a.size() + b.size(), z.data(), sizeof(float) * z.size(),
-                    hipMemcpyHostToDevice));
-  c->tw32_x = d;
-  c->tw32_xr = d + a.size();
-  c->tw32_z = d + a.size() + b.size();
-  void* w = nullptr;
-  // mean-mode solve (3 ny), gauge value, then the gauge partial sums
-  const size_t nw = 3 * ((size_t)g.ny + 1) + (size_t)((g.nx + 63) / 64) * g.nz;
-  if ((rc = dalloc(c, &w, nw * sizeof(double)))) return rc;
-  C3D_HIP(hipMemset(w, 0, nw * sizeof(double)));
-  c->d_mean64 = (double*)w;
   // pivots and factors of the (0,0) line, by the elimination's operations
   std::vector<double> fac(2 * (size_t)g.ny, 0.0);
   const auto &am = c->met[C3D_M_AM2PR], &ac = c->met[C3D_M_AC2PR], &ap = c->met[C3D_M_AP2PR];
@@ -510,10 +493,29 @@ int ensure_mixed_tables(c3d_ctx* c) {
     fac[g.ny + j] = arr;
     cprev = ap[j + 1];
   }
-  void* mf = nullptr;
-  if ((rc = dalloc(c, &mf, fac.size() * sizeof(double)))) return rc;
-  c->d_meanfac = (double*)mf;
-  C3D_HIP(hipMemcpy(mf, fac.data(), fac.size() * sizeof(double), hipMemcpyHostToDevice));
+  void* w = nullptr;
+  // mean-mode solve (3 ny), gauge value, then the gauge partial sums
+  const size_t nw = 3 * ((size_t)g.ny + 1) + (size_t)((g.nx + 63) / 64) * g.nz;
+  if ((rc = dalloc(c, &w, nw * sizeof(double)))) return rc;
+  C3D_HIP(hipMemset(w, 0, nw * sizeof(double)));
+  c->d_mean64 = (double*)w;
+  // the line's tables and the twiddles in one block, put there by one copy
+  const size_t nf = fac.size() * sizeof(double);
+  std::vector<unsigned char> blk(nf + sizeof(float) * (a.size() + b.size() + z.size()));
+  std::memcpy(blk.data(), fac.data(), nf);
+  size_t off = nf;
+  for (const std::vector<float>* v : {&a, &b, &z}) {
+    std::memcpy(blk.data() + off, v->data(), sizeof(float) * v->size());
+    off += sizeof(float) * v->size();
+  }
+  void* tw = nullptr;
+  if ((rc = dalloc(c, &tw, blk.size()))) return rc;
+  C3D_HIP(hipMemcpy(tw, blk.data(), blk.size(), hipMemcpyHostToDevice));
+  c->d_meanfac = (double*)tw;
+  float* d = (float*)((unsigned char*)tw + nf);
+  c->tw32_x = d;
+  c->tw32_xr = d + a.size();
+  c->tw32_z = d + a.size() + b.size();
   c->d_tw32 = tw;
   return C3D_OK;
 }
@@ -597,10 +599,10 @@ extern "C" int c3d_destroy(c3d_ctx* c) {
     if (c->state[i]) hipFree(c->state[i]);
   for (void* p : c->user_fields) hipFree(p);
   void* bufs[] = {c->tmpA, c->spec, c->sarr, c->d_partials, c->d_sc, c->d_tw, c->d_met, c->d_tabs,
-                  c->d_dyp, c->d_stat, c->d_tw32, c->d_met32, c->resid32, c->d_mean64, c->d_meanfac,
+                  c->d_dyp, c->d_stat, c->d_tw32, c->d_met32, c->resid32, c->d_mean64,
                   c->d_lesmet, c->d_spec1d, c->spec2, c->d_spec2d, c->cln_d, c->cln_f,
                   c->cln_fb, c->bspec, c->bsarr, c->bmean, c->bres, c->btmp,
-                  c->les_arr[0], c->les_arr[1]};
+                  c->les_block};
   for (void* p : bufs)
     if (p) hipFree(p);
   if (c->staging) hipHostFree(c->staging);
@@ -838,12 +840,16 @@ extern "C" int c3d_create(const c3d_params* p, const double* yp, c3d_ctx** out) 
     e = hipMemset(c->state[i], 0, b);
     if (e != hipSuccess) return fail(hip_fail(e, "hipMemset"));
   }
-  if ((rc = dalloc(c, &c->tmpA, fbytes))) return fail(rc);
-  // convolved right-hand sides of uy and uz where a substep convolves the three
-  // components in one launch (small fields; an LES context uses them as well)
-  if (c->order == 2 && adi3_fields(g, c->esize))
-    for (int d = 0; d < 2; ++d)
-      if ((rc = dalloc(c, &c->les_arr[d], fbytes))) return fail(rc);
+  // with room for the convolved right-hand sides of uy and uz where a substep
+  // convolves the three components in one launch (small fields; an LES context
+  // uses them as well).  One allocation of the three, and one copy of the FP32 tables
+  // above, keep c3d_create short: 0.57-0.61 ms for 64^3 and 0.94 for 192x96x128
+  // with each on its own, 0.51 and 0.86 so
+  const bool three = c->order == 2 && adi3_fields(g, c->esize);
+  const size_t fstep = (fbytes + 255) / 256 * 256;
+  if ((rc = dalloc(c, &c->tmpA, three ? 2 * fstep + fbytes : fbytes))) return fail(rc);
+  if (three)
+    for (int d = 0; d < 2; ++d) c->les_arr[d] = (unsigned char*)c->tmpA + (d + 1) * fstep;
   if ((rc = dalloc(c, &c->spec, (size_t)g.nspec * 2 * c->esize))) return fail(rc);
   if ((rc = dalloc(c, &c->sarr, (size_t)g.nspec * c->esize))) return fail(rc);
   {
@@ -1758,9 +1764,12 @@ extern "C" int c3d_set_les(c3d_ctx* c, int les_type, int filter_type) {
     if ((rc = dalloc(c, &c->state[C3D_NUT], fbytes))) return rc;
     C3D_HIP(hipMemset(c->state[C3D_NUT], 0, fbytes));  // nut = zero (m_Variables.f90:71-74)
   }
-  for (int d = 0; d < 2; ++d)
-    if (!c->les_arr[d] && (rc = dalloc(c, &c->les_arr[d], (size_t)c->g.nfield * c->esize)))
-      return rc;
+  if (!c->les_arr[0]) {
+    const size_t fbytes = (size_t)c->g.nfield * c->esize, fstep = (fbytes + 255) / 256 * 256;
+    if ((rc = dalloc(c, &c->les_block, fstep + fbytes))) return rc;
+    c->les_arr[0] = c->les_block;
+    c->les_arr[1] = (unsigned char*)c->les_block + fstep;
+  }
   if (!c->d_lesmet) {
     const size_t L = (size_t)c->g.ny + 3;
     if ((rc = dalloc(c, &c->d_lesmet, 4 * L * c->esize))) return rc;

@@ -444,8 +444,10 @@ struct c3d_ctx {
   double les_fcoe[9] = {};
   void* d_lesmet = nullptr;
   // uy's and uz's field-sized scratch (ux's is tmpA): checkpoints of the LES
-  // solves, convolved right-hand sides of the merged 2nd-order solves
+  // solves, convolved right-hand sides of the merged 2nd-order solves.  They lie
+  // behind tmpA in its allocation, or in les_block
   void* les_arr[2] = {nullptr, nullptr};
+  void* les_block = nullptr;
   c3d::LesMet<double> lmd{};
   c3d::LesMet<float> lmf{};
 
@@ -481,7 +483,7 @@ struct c3d_ctx {
   double prof_bytes[c3d::ST_COUNT] = {};
 
   // mixed-precision pressure solve: the (0,0) line's pivots vecm[ny] and
-  // factors arr[ny]
+  // factors arr[ny], at the head of d_tw32's block
   double* d_meanfac = nullptr;
 };
 
