@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "../../include/channel3d.h"
+#include "c3d_quot.h"
 
 namespace c3d {
 
@@ -85,38 +86,6 @@ __device__ __forceinline__ double row_prev(double v, double edge) {
 __device__ __forceinline__ double row_next(double v, double edge, int lane, int last) {
   const double r = dpp_shift(v, edge, false);
   return lane == last ? edge : r;
-}
-
-// Several quotients by one divisor.  quot_recip(v) is 1/v to about an ulp
-// (the hardware estimate and two Newton steps); quot(a, v, r) multiplies and
-// corrects with the exact remainder a - v q (Markstein's step), which rounds
-// a/v correctly; div_fixup restores the special cases (zeros, infinities,
-// NaN).  v and a/v must be in the normal range.  The first quotient costs
-// about what `/` does, each further one four instructions instead of twelve.
-__device__ __forceinline__ double quot_recip(double v) {
-  double r = __builtin_amdgcn_rcp(v);
-  r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
-}
-__device__ __forceinline__ double quot(double a, double v, double r) {
-  const double q = a * r;
-  return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-v, q, a), r, q), v, a);
-}
-__device__ __forceinline__ float quot_recip(float v) {
-  const float r = __builtin_amdgcn_rcpf(v);  // within an ulp: one step suffices
-  return __builtin_fmaf(__builtin_fmaf(-v, r, 1.0f), r, r);
-}
-__device__ __forceinline__ float quot(float a, float v, float r) {
-  const float q = a * r;
-  return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-v, q, a), r, q), v, a);
-}
-
-// quot by a divisor whose reciprocal is tabulated: r is 1/v rounded (FP64), or
-// that rounded to FP32 and refined for the FP32 divisor.
-__device__ __forceinline__ double tab_recip(double, double r) { return r; }
-__device__ __forceinline__ float tab_recip(float v, double r) {
-  const float q = (float)r;
-  return __builtin_fmaf(__builtin_fmaf(-v, q, 1.0f), q, q);
 }
 
 // Reproducible sums.  Each double term is truncated to a multiple of 2^-80
