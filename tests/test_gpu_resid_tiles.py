@@ -58,6 +58,32 @@ def test_pressure_refinement(grid):
             assert e2 <= rate ** 2 * e0 + 1e-12
 
 
+@pytest.mark.parametrize("grid", LONG + [(16, 3, 8), (64, 33, 16)],
+                         ids=lambda v: "x".join(map(str, v)))
+def test_mean_mode(grid):
+    """The (0, 0) mode alone: a source that depends on y only, small integers, so that
+    the FP32 transforms (lengths of powers of two) are exact.  Its line is solved in
+    FP64 and rounded to FP32 once: 2^-24 of the largest value, where an FP32
+    elimination would lose eps ny^2; a sweep squares that.  Besides, FP64 rounding of
+    the line, whose condition number is about ny^2."""
+    from channel3d_amd import lib as L
+    nx, ny, nz = grid
+    with _channel(*grid) as g:
+        src, a, b = (g.alloc_batch(lay, 2) for lay in (L.INTERIOR,) + (L.HALO,) * 2)
+        rng = np.random.default_rng(ny)
+        for q in range(2):
+            f = rng.integers(-1000, 1000, ny).astype(float)
+            g.upload(src[q], np.broadcast_to(f[None, :, None], grid), L.INTERIOR)
+        g.ppe_batch(src, a, -1)
+        rounding = np.finfo(float).eps * ny ** 2
+        for sweeps, once in ((0, 2.0 ** -24), (1, 2.0 ** -48), (2, 0.0)):
+            g.ppe_batch(src, b, sweeps)
+            for q in range(2):
+                x, y = (g.download(h[q], L.HALO)[1:-2, 1:ny + 1, 1:-2] for h in (a, b))
+                assert np.abs(x).max() > 0
+                assert np.abs(x - y).max() <= (once + rounding) * np.abs(x).max()
+
+
 @pytest.mark.parametrize("grid", GRIDS, ids=lambda v: "x".join(map(str, v)))
 @pytest.mark.parametrize("comp", [0, 1])
 def test_velocity_refinement(grid, comp):
