@@ -5,8 +5,10 @@ remainders.  A cell whose residual is wrong keeps the FP32 solve's error, so
 the refined solution must approach the FP64 solve of the same source (which
 the oracle tests cover) everywhere.  Bounds: a sweep multiplies the error by at
 most the FP32 solve's relative error, FP32's eps times the condition number of
-the operator: about ny^2 for the Neumann line of the pressure's mean mode, below
-20 for the velocity operator; what remains is FP64 rounding (1e-12)."""
+the operator: for the pressure's worst line, the y operator's largest entry
+(about ny^2) over the smallest non-zero wavenumber term (1 in these boxes; the
+mean mode's line is solved in FP64 and has a test of its own); below 20 for the
+velocity operator.  What remains is FP64 rounding (1e-12)."""
 import math
 
 import numpy as np
