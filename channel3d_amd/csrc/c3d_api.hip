@@ -354,9 +354,10 @@ static void thomas_factors(const std::vector<double>& a, const std::vector<doubl
   }
 }
 
-// per substep: x taps (nx), z taps (nz), then ten y vectors of ny+2: the
+// per substep: x taps (nx), z taps (nz), then twelve y vectors of ny+2: the
 // cell operator's a, vecm, arr, the node operator's a, vecm, arr, the cell
-// operator's b and c, the node operator's b and c
+// operator's b and c, the node operator's b and c, 1/vecm of the cell and of the
+// node operator
 static size_t adi_table_len(const Geom& g) {
   return (size_t)g.nx + (size_t)g.nz + 12 * ((size_t)g.ny + 2);
 }
@@ -840,7 +841,7 @@ extern "C" int c3d_create(const c3d_params* p, const double* yp, c3d_ctx** out) 
     e = hipMemset(c->state[i], 0, b);
     if (e != hipSuccess) return fail(hip_fail(e, "hipMemset"));
   }
-  // with room for the convolved right-hand sides of uy and uz where a substep
+  // tmpA, with room for the convolved right-hand sides of uy and uz where a substep
   // convolves the three components in one launch (small fields; an LES context
   // uses them as well).  One allocation of the three, and one copy of the FP32 tables
   // above, keep c3d_create short: 0.57-0.61 ms for 64^3 and 0.94 for 192x96x128

@@ -225,7 +225,7 @@ __device__ inline double bulk_shift(const Bulk& b, DevScalars* sc, bool keep) {
   return d;
 }
 
-// wall values of the velocity, m_BC_and_Halo.f90; order 4: noslip_p = channel
+// wall values of the velocity, m_BC_and_Halo.f90 (2nd order)
 struct WallBC {
   int bcym, bcyp;
   double uxm, uym, uzm, uxp, uyp, uzp;  // wall values
@@ -340,8 +340,9 @@ struct c3d_ctx {
   void* d_tabs = nullptr;
   // y solver (YS_*): checkpointed sweeps, or the sweeps storing the forward pass
   int ymode = 0;
-  // lanes per wavenumber pair of the checkpointed PPE sweep: 2 (or 0), 1 forced
-  // for tests of both forms
+  // PPE sweep: 0 by the line and row counts (LDS, or two lanes per wavenumber pair
+  // with checkpoints); 1 or 2 forces the checkpointed form with that many lanes,
+  // for tests of the forms against each other
   int tri_lanes = 0;
   int y_threads = 0;  // lines per workgroup of the checkpointed y sweep (0: by grid size)
   int z_tile = 0;     // kx lines per workgroup of the z transform (0: 8)
@@ -592,7 +593,8 @@ int run_ppe(c3d_ctx* c, void* prsrc, void* phi);
 // the pressure source (with the -nu/2 div pressure correction when pr is
 // given) fused into the x forward pass of the FP64-solve pressure equation;
 // the source lands in the spectral array only, max |div| in its slots.
-// SetBC_and_UpdateHaloForPrSrc is part of it.  Then run_ppe_from_spectrum finishes the solve into phi.
+// SetBC_and_UpdateHaloForPrSrc is part of it where the grid's fields fit in the
+// caches (not Geom::nt).  Then run_ppe_from_spectrum finishes the solve into phi.
 int launch_prsrc_fft_x(c3d_ctx* c, const void* ux, const void* uy, const void* uz, void* pr);
 int run_ppe_from_spectrum(c3d_ctx* c, void* phi);
 // FP32 transforms of the mixed-precision solve

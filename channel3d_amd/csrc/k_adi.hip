@@ -78,7 +78,10 @@ __global__ __launch_bounds__(ABX* ABY) void k_conv_z(Geom g, const double* __res
 // LDS (with the x halo) and convolved along x, the results enter a register
 // window of 2*MZ+1 planes, and one z-convolved plane is written per step.
 // Every input element is read from HBM once per chunk (plus the 2*MZ-plane
-// lead-in), every output element written once.
+// lead-in), every output element written once.  Bound: instructions (an LDS read, a
+// table word and a multiply-add per tap and cell in a loop of run-time length),
+// 3.6 ps a cell in FP64 (4.3 TB/s) and 3.2 ps in FP32 at half the bytes, where the
+// vector units are active 63-79 % of the time.
 constexpr int MAXMX = 32;
 
 // TIN: type of the right-hand side read (an FP32 solve of an FP64 right-hand

@@ -528,7 +528,7 @@ __global__ __launch_bounds__(FNT) void k_fft_z(Geom g, typename CT<T>::t* __rest
 // took 25, 31, 34 and 25 us; now 11, 14, 17 and 14 (4 us of HBM time each).
 // ===========================================================================
 constexpr int GEN_MAXP = 24;   // passes: 2^24 exceeds every supported length
-constexpr int GEN_MAXE = 8;    // complex values a thread carries: lines x n <= 8 x FNT
+constexpr int GEN_MAXE = 8;    // lines x n <= 8 x FNT (a pass rounds up: 9 values a thread for radix 3, 10 for 5)
 constexpr int GEN_NMAX = 4095; // one line of (N+1) FP64 complex fits 64 KiB
 
 // x / d for x and d up to 2^16: with m = ceil(2^32 / d) the product exceeds
@@ -743,7 +743,7 @@ __global__ __launch_bounds__(FNT) void k_fftg_x_inv(Geom g, FftPlan pl,
   __shared__ long long rb[16];
   spec += bsp * blockIdx.y;
   out += bout * blockIdx.y;
-  const int N = pl.n, lines = pl.lines, ldn = N + 1;
+  const int N = pl.n, lines = pl.lines;
   const int row0 = blockIdx.x * lines;
   const int nrows = g.ny * g.nz;
   row_offsets(g, row0, lines, rb);
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(FNT) void k_fftg_z(Geom g, FftPlan pl,
   extern __shared__ __align__(16) unsigned char gen_raw[];
   T2* sm = (T2*)gen_raw;
   spec += bsp * blockIdx.z;
-  const int N = pl.n, lines = pl.lines, ldn = N + 1;
+  const int lines = pl.lines;
   const int kx0 = blockIdx.x * lines;
   const int nl = min(lines, g.nk + 1 - kx0);
   const long long sk = (long long)g.P * g.ny;

@@ -17,10 +17,6 @@
 
 namespace c3d {
 
-// these kernels run mostly on grids that fit in the caches: ordinary
-// accesses for the once-touched words
-constexpr bool NTS = false;
-
 namespace {
 
 constexpr int LBX = 64, LBY = 4, LKCH = 8;
@@ -106,11 +102,11 @@ __device__ __forceinline__ void nut_ghosts(const Geom& g, const LesCoef<T>& q, T
 // (LZ = 2), whose residual on the face k+1 reaches k+2; that residual is the next
 // cell's at k, and the one quantity kept.  The squared residuals the reference
 // stores in Ktemp are formed by each cell for its other faces (same operands,
-// same operations).  Bound: HBM, 4 words per cell.
+// same operations).  Bound: FP64 arithmetic, some 280 vector instructions a cell
+// (vector units active 67 % of the time), beside 4 words per cell of HBM.
 // With every operand fetched on its own (MTS: over 90 loads a cell, both
 // residuals of each component from memory) MTS took 0.724 ms at 384x192x288,
-// WALE 0.026 ms at 96x96x72; now 0.284 (2.4 TB/s; FP64 latency of the square
-// roots and divisions at three wavefronts per SIMD is what remains) and 0.018 ms.
+// WALE 0.026 ms at 96x96x72; now 0.284 (2.4 TB/s) and 0.018 ms.
 // ---------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ T filt_res(const T* F, const T* a, const T* b, const T* c) {
@@ -382,7 +378,7 @@ __global__ __launch_bounds__(LBX* LBY, 2) void k_rhs_les(Geom g, Metrics<T> m, L
         for (int f = 0; f < 5; ++f) sb[buf][f][tid + NT * s] = st[f][s];
       }
   };
-  const int jc = j0 + ty, jrow = min(jc, ny), jp = jrow + 1;
+  const int jc = j0 + ty, jrow = min(jc, ny);
   const int e = (ty + 1) * LW + tx + 1;
   const bool live = i0 + tx < nx && jc <= ny;
   const T rdx = q.rdx, rdz = q.rdz;

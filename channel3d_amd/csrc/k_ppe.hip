@@ -717,7 +717,7 @@ __device__ void mean_mode_fp64(const Geom& g, const Metrics<double>& m,
 
 // Workgroup 0 of a field solves the (0,0) mode, the others every other line
 // by the checkpointed elimination.
-template <typename T, int C, bool NTS>
+template <typename T, int C>
 __global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, PprRows(T), Metrics<double> md,
                                                        const double* __restrict__ fac,
                                                        typename CT2<T>::t* __restrict__ spec,
@@ -731,8 +731,7 @@ __global__ __launch_bounds__(256) void k_tridiag_mixed(Geom g, PprRows(T), Metri
   }
   const long long l = ((long long)(blockIdx.x - 1) * 256 + threadIdx.x) >> 1;
   if (l == 0) return;
-  k_tridiag_ck2_body<T, C, NTS>(g, am, ac, ap, wx, wz, spec, ckp + bck * blockIdx.y,
-                                line_of(g, l));
+  k_tridiag_ck2_body<T, C>(g, am, ac, ap, wx, wz, spec, ckp + bck * blockIdx.y, line_of(g, l));
 }
 
 // r = f - L phi in FP64, L the discrete operator the spectral solve inverts:
@@ -884,7 +883,7 @@ static int ppe_mixed(c3d_ctx* c, const void* prsrc, void* phi, int sweeps, void*
     prof_begin(c, ST_TRIDIAG, &ev);
     const long long nl = (long long)(g.nk + 1) * g.nz;
     const dim3 grid((unsigned)(1 + (2 * nl + 255) / 256), b.n), blk(256);
-    hipLaunchKernelGGL((k_tridiag_mixed<float, tri_rows<float>(), false>), grid, blk, 0, c->stream,
+    hipLaunchKernelGGL((k_tridiag_mixed<float, tri_rows<float>()>), grid, blk, 0, c->stream,
                        g, PPR_OF(c->mf), c->md, c->d_meanfac, (float2*)spec, (float*)ck, w,
                        b.spec32, b.ck, b.mean);
     C3D_HIP(hipGetLastError());

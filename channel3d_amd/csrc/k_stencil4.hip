@@ -16,10 +16,6 @@
 
 namespace c3d {
 
-// these kernels run mostly on grids that fit in the caches: ordinary
-// accesses for the once-touched words
-constexpr bool NTS = false;
-
 constexpr int B4X = 64, B4Y = 4, K4CH = 4;
 
 __device__ __forceinline__ int wr(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
